@@ -21,10 +21,20 @@ namespace {
 
 constexpr int kT = 256;
 
-__device__ inline uint64_t wave_sum64(uint64_t v) {
+// One atomic per block: atomics on one address take ~12 ns each in turn, so
+// one per wave of a launch over 2^22 vertices cost ~0.8 ms (SCALE 22; the
+// kernels' own memory time is below 0.02 ms).  All threads of the block call.
+__device__ inline void block_add(uint64_t v, unsigned long long* cnt) {
+  __shared__ uint64_t part[kT / kWave];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
+  if (lane_id() == 0) part[threadIdx.x / kWave] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kT / kWave; ++w) v += part[w];
+    if (v) atomicAdd(cnt, (unsigned long long)v);
+  }
 }
 
 __global__ __launch_bounds__(kT) void k_core_init(const int64_t* __restrict__ row_off,
@@ -99,33 +109,97 @@ __global__ __launch_bounds__(kT) void k_core_by_target(const uint32_t* __restric
   if (atomicSub(&deg[t], 1u) == 1u) alive[t] = 0;
 }
 
-// live out-degree in the core, per vertex
-__global__ __launch_bounds__(kT) void k_core_count(const int64_t* __restrict__ row_off,
-                                                  const uint32_t* __restrict__ col,
-                                                  const uint8_t* __restrict__ alive,
-                                                  int64_t n_c, uint64_t* __restrict__ cnt) {
+// Core edges, taken from the CSR's entries in tiles of kFilterTile, one block
+// a tile, so that a row's length never decides how long a lane works: with a
+// thread a row (the earlier form) the hub rows, 10^5 entries and more at SCALE
+// 22, were walked by single lanes, and counting and writing took 42 and 85 ms
+// there; the tiles take 0.47 and 1.18 ms, bound by the random reads of the
+// targets' flags and original IDs.
+// kCount: kept entries per tile; kWrite: the kept entries as (original ID,
+// original ID) pairs in entry order from tile_off[tile] on.  tile_row[t] is
+// the row that holds entry t * kFilterTile.
+constexpr int kFilterItems = 8;
+constexpr int kFilterTile = kT * kFilterItems;
+enum { kCount = 0, kWrite = 1 };
+
+__global__ __launch_bounds__(kT) void k_core_tile_rows(const int64_t* __restrict__ row_off,
+                                                      int64_t n_c,
+                                                      uint32_t* __restrict__ tile_row) {
   const int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (v >= n_c) return;
-  uint64_t c = 0;
-  if (alive[v])
-    for (int64_t e = row_off[v]; e < row_off[v + 1]; ++e) c += alive[col[e]];
-  cnt[v] = c;
+  const int64_t end = row_off[v + 1];
+  for (int64_t t = ceil_div(row_off[v], kFilterTile); t * kFilterTile < end; ++t)
+    tile_row[t] = (uint32_t)v;
 }
 
-// core edge list in original IDs (both directions, already deduplicated)
-__global__ __launch_bounds__(kT) void k_core_edges(const int64_t* __restrict__ row_off,
-                                                  const uint32_t* __restrict__ col,
-                                                  const uint8_t* __restrict__ alive,
-                                                  const uint32_t* __restrict__ n2o,
-                                                  const uint64_t* __restrict__ off,
-                                                  int64_t n_c, uint2* __restrict__ out) {
-  const int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (v >= n_c || !alive[v]) return;
-  uint64_t p = off[v];
-  const uint32_t ov = n2o[v];
-  for (int64_t e = row_off[v]; e < row_off[v + 1]; ++e) {
-    const uint32_t u = col[e];
-    if (alive[u]) out[p++] = make_uint2(ov, n2o[u]);
+template <int kPass>
+__global__ __launch_bounds__(kT) void k_core_filter(
+    const int64_t* __restrict__ row_off, const uint32_t* __restrict__ col,
+    const uint8_t* __restrict__ alive, const uint32_t* __restrict__ n2o,
+    const uint32_t* __restrict__ tile_row, int64_t n_c, int64_t m,
+    uint32_t* __restrict__ tile_cnt, const uint64_t* __restrict__ tile_off,
+    uint2* __restrict__ out) {
+  // start of each row of the tile, relative to the tile; every row holds an
+  // entry, so at most kFilterTile rows start inside it
+  __shared__ int rstart[kFilterTile + 1];
+  __shared__ uint32_t kept[kFilterItems][kT / kWave];
+  const int t = threadIdx.x, wave = t / kWave;
+  const int64_t base = (int64_t)blockIdx.x * kFilterTile;
+  const int64_t last = (m - base < kFilterTile ? m : base + kFilterTile) - 1;
+  const int64_t r0 = tile_row[blockIdx.x];
+  // the row of the tile's last entry: the owner of the next tile's first
+  // entry, or the row before it
+  int64_t r1 = n_c - 1;
+  if (last + 1 < m) {
+    r1 = tile_row[blockIdx.x + 1];
+    if (row_off[r1] > last) --r1;
+  }
+  const int rows = (int)(r1 - r0) + 1;
+  for (int i = t; i < rows; i += kT) {
+    const int64_t d = row_off[r0 + i] - base;
+    rstart[i] = d < 0 ? 0 : (int)d;
+  }
+  __syncthreads();
+  uint32_t src[kFilterItems], dst[kFilterItems];
+  uint64_t mask[kFilterItems];
+#pragma unroll
+  for (int k = 0; k < kFilterItems; ++k) {
+    const int li = k * kT + t;
+    const bool in = base + li <= last;
+    const uint32_t u = in ? col[base + li] : 0u;
+    int lo = 0, hi = rows;  // last row that starts at or before li
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (rstart[mid] <= li) lo = mid;
+      else hi = mid;
+    }
+    src[k] = (uint32_t)(r0 + lo);
+    dst[k] = u;
+    mask[k] = __ballot(in && alive[u] && alive[r0 + lo]);
+    if (lane_id() == 0) kept[k][wave] = (uint32_t)__popcll(mask[k]);
+  }
+  __syncthreads();
+  uint32_t run = 0;
+  if (kPass == kCount) {
+    if (t == 0) {
+      for (int k = 0; k < kFilterItems; ++k)
+        for (int w = 0; w < kT / kWave; ++w) run += kept[k][w];
+      tile_cnt[blockIdx.x] = run;
+    }
+    return;
+  }
+  uint2* o = out + tile_off[blockIdx.x];
+#pragma unroll
+  for (int k = 0; k < kFilterItems; ++k) {
+    uint32_t before = run;
+#pragma unroll
+    for (int w = 0; w < kT / kWave; ++w) {
+      const uint32_t c = kept[k][w];
+      before += w < wave ? c : 0u;
+      run += c;
+    }
+    if ((mask[k] >> lane_id()) & 1ull)
+      o[before + __popcll(mask[k] & lanemask_lt())] = make_uint2(n2o[src[k]], n2o[dst[k]]);
   }
 }
 
@@ -135,16 +209,16 @@ __global__ __launch_bounds__(kT) void k_core_forest(const uint32_t* __restrict__
                                                    int64_t n_c, uint32_t* __restrict__ tp,
                                                    unsigned long long* __restrict__ hp,
                                                    unsigned long long* cnt) {
-  const int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x;
   uint64_t c = 0;
-  if (v < n_c && par[v] != kNoParent) {
+  for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n_c;
+       v += (int64_t)gridDim.x * kT) {
+    if (par[v] == kNoParent) continue;
     const uint32_t o = n2o[v];
     tp[o] = n2o[par[v]];
     atomicOr(&hp[o >> 6], 1ull << (o & 63));
-    c = 1;
+    ++c;
   }
-  c = wave_sum64(c);
-  if (lane_id() == 0 && c) atomicAdd(cnt, (unsigned long long)c);
+  block_add(c, cnt);
 }
 
 // reach[o] = o is a core vertex the hd_root BFS visited
@@ -162,30 +236,30 @@ __global__ __launch_bounds__(kT) void k_reach_init(const uint32_t* __restrict__ 
 __global__ __launch_bounds__(kT) void k_reach_sweep(const uint32_t* __restrict__ tp,
                                                    int64_t n, uint8_t* reach,
                                                    unsigned long long* cnt) {
-  const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
   uint64_t c = 0;
-  if (o < n && !reach[o]) {
+  for (int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x; o < n;
+       o += (int64_t)gridDim.x * kT) {
+    if (reach[o]) continue;
     const uint32_t p = tp[o];
     if (p != kNoParent && __atomic_load_n(&reach[p], __ATOMIC_RELAXED)) {
       reach[o] = 1;
-      c = 1;
+      ++c;
     }
   }
-  c = wave_sum64(c);
-  if (lane_id() == 0 && c) atomicAdd(cnt, (unsigned long long)c);
+  block_add(c, cnt);
 }
 
 __global__ __launch_bounds__(kT) void k_reach_reset(uint32_t* __restrict__ tp,
                                                    const uint8_t* __restrict__ reach,
                                                    int64_t n, unsigned long long* cnt) {
-  const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
   uint64_t c = 0;
-  if (o < n && tp[o] != kNoParent && !reach[o]) {
+  for (int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x; o < n;
+       o += (int64_t)gridDim.x * kT) {
+    if (tp[o] == kNoParent || reach[o]) continue;
     tp[o] = kNoParent;
-    c = 1;
+    ++c;
   }
-  c = wave_sum64(c);
-  if (lane_id() == 0 && c) atomicAdd(cnt, (unsigned long long)c);
+  block_add(c, cnt);
 }
 
 // largest original ID that is a core vertex or has a parent
@@ -193,13 +267,21 @@ __global__ __launch_bounds__(kT) void k_max_used(const uint32_t* __restrict__ o2
                                                 int64_t n, int64_t n_c,
                                                 const uint64_t* __restrict__ hp,
                                                 unsigned long long* mx) {
-  const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (o >= n) return;
-  if ((int64_t)o2n[o] < n_c || ((hp[o >> 6] >> (o & 63)) & 1ull))
-    atomicMax(mx, (unsigned long long)o);
+  unsigned long long best = 0;
+  for (int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x; o < n;
+       o += (int64_t)gridDim.x * kT)
+    if ((int64_t)o2n[o] < n_c || ((hp[o >> 6] >> (o & 63)) & 1ull)) best = (unsigned long long)o;
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const unsigned long long x = __shfl_xor(best, s, kWave);
+    best = x > best ? x : best;
+  }
+  if (lane_id() == 0 && best) atomicMax(mx, best);
 }
 
 unsigned blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, ceil_div(n, kT)); }
+// grid of the kernels that end with an atomic (grid-stride): four blocks a CU
+unsigned few_blocks(int64_t n) { return std::min(blocks(n), 1024u); }
 
 uint64_t read_u64(const unsigned long long* d, hipStream_t s) {
   unsigned long long h = 0;
@@ -263,7 +345,7 @@ void corebfs_prune(g500_graph* g) {
   G500_CHECK_HIP(hipMemsetAsync(g->has_parent.get(), 0, ceil_div(n, 64) * sizeof(uint64_t), s));
   G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(unsigned long long), s));
   if (n_c > 0) {
-    hipLaunchKernelGGL(k_core_forest, dim3(blocks(n_c)), dim3(kT), 0, s, par.get(),
+    hipLaunchKernelGGL(k_core_forest, dim3(few_blocks(n_c)), dim3(kT), 0, s, par.get(),
                        g->new2orig.get(), n_c, g->tree_parent.get(),
                        (unsigned long long*)g->has_parent.get(), cnt.get());
     G500_CHECK_LAUNCH();
@@ -272,29 +354,41 @@ void corebfs_prune(g500_graph* g) {
   par.release();
 
   // 4. core edge list (original IDs) -> core CSR in the same vertex space
-  DevBuf<uint64_t> ccnt;
-  ccnt.alloc((size_t)nn + 1);
-  if (n_c > 0) {
-    hipLaunchKernelGGL(k_core_count, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
-                       g->col.get(), alive.get(), n_c, ccnt.get());
+  const int64_t tiles = ceil_div(g->m, kFilterTile);
+  DevBuf<uint32_t> tile_row, tile_cnt;
+  DevBuf<uint64_t> tile_off;
+  tile_row.alloc((size_t)tiles);
+  tile_cnt.alloc((size_t)tiles);
+  tile_off.alloc((size_t)tiles + 1);
+  if (tiles > 0) {
+    hipLaunchKernelGGL(k_core_tile_rows, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
+                       n_c, tile_row.get());
+    G500_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_core_filter<kCount>, dim3((unsigned)tiles), dim3(kT), 0, s,
+                       g->row_off.get(), g->col.get(), alive.get(), g->new2orig.get(),
+                       tile_row.get(), n_c, g->m, tile_cnt.get(), (const uint64_t*)nullptr,
+                       (uint2*)nullptr);
     G500_CHECK_LAUNCH();
   }
-  exclusive_scan<uint64_t>(ccnt.get(), ccnt.get(), n_c, g->scan_ws, s);
+  exclusive_scan<uint32_t>(tile_cnt.get(), tile_off.get(), tiles, g->scan_ws, s);
   uint64_t m_core = 0;
-  G500_CHECK_HIP(hipMemcpyAsync(&m_core, ccnt.get() + n_c, sizeof(uint64_t),
+  G500_CHECK_HIP(hipMemcpyAsync(&m_core, tile_off.get() + tiles, sizeof(uint64_t),
                                 hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipStreamSynchronize(s));
   DevBuf<uint2> core_edges;
   core_edges.alloc((size_t)std::max<uint64_t>(m_core, 1));
-  if (n_c > 0) {
-    hipLaunchKernelGGL(k_core_edges, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
-                       g->col.get(), alive.get(), g->new2orig.get(), ccnt.get(), n_c,
+  if (tiles > 0) {
+    hipLaunchKernelGGL(k_core_filter<kWrite>, dim3((unsigned)tiles), dim3(kT), 0, s,
+                       g->row_off.get(), g->col.get(), alive.get(), g->new2orig.get(),
+                       tile_row.get(), n_c, g->m, tile_cnt.get(), tile_off.get(),
                        core_edges.get());
     G500_CHECK_LAUNCH();
   }
   G500_CHECK_HIP(hipStreamSynchronize(s));
   alive.release();
-  ccnt.release();
+  tile_row.release();
+  tile_cnt.release();
+  tile_off.release();
   // drop the full CSR before building the core one
   g->col.release();
   g->first.release();
@@ -306,7 +400,7 @@ void corebfs_prune(g500_graph* g) {
 
   // find_max_used_vertex over has_edge = core vertex or forest vertex
   G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL(k_max_used, dim3(blocks(n)), dim3(kT), 0, s, g->orig2new.get(), n,
+  hipLaunchKernelGGL(k_max_used, dim3(few_blocks(n)), dim3(kT), 0, s, g->orig2new.get(), n,
                      g->n_c, g->has_parent.get(), cnt.get());
   G500_CHECK_LAUNCH();
   g->max_used = (int64_t)read_u64(cnt.get(), s);
@@ -337,13 +431,13 @@ void corebfs_reset_unreachable(g500_graph* g, const uint64_t* visited, hipStream
   for (int iter = 0;; ++iter) {
     if (iter > (1 << 16)) fail(G500_ERR_STATE, "forest reachability did not converge");
     G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(k_reach_sweep, dim3(blocks(n)), dim3(kT), 0, s,
+    hipLaunchKernelGGL(k_reach_sweep, dim3(few_blocks(n)), dim3(kT), 0, s,
                        g->tree_parent.get(), n, reach.get(), cnt.get());
     G500_CHECK_LAUNCH();
     if (read_u64(cnt.get(), s) == 0) break;
   }
   G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL(k_reach_reset, dim3(blocks(n)), dim3(kT), 0, s, g->tree_parent.get(),
+  hipLaunchKernelGGL(k_reach_reset, dim3(few_blocks(n)), dim3(kT), 0, s, g->tree_parent.get(),
                      reach.get(), n, cnt.get());
   G500_CHECK_LAUNCH();
   g->removed_parents = (int64_t)read_u64(cnt.get(), s);
