@@ -54,15 +54,16 @@ struct DevBuf {
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() { release(); }
   void alloc(size_t count) {
-    release();
-    if (count == 0) count = 1;
-    void* q = nullptr;
-    hipError_t e = hipMalloc(&q, count * sizeof(T));
+    const hipError_t e = reserve(count);
     if (e != hipSuccess)
       fail(G500_ERR_NOMEM, "hipMalloc(%zu bytes): %s", count * sizeof(T),
            hipGetErrorString(e));
-    p = static_cast<T*>(q);
-    n = count;
+  }
+  // false where the device has no room: for a caller that can do without
+  bool try_alloc(size_t count) {
+    if (reserve(count) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
   }
   void release() {
     if (p) (void)hipFree(p);
@@ -70,6 +71,19 @@ struct DevBuf {
     n = 0;
   }
   T* get() const { return p; }
+
+ private:
+  hipError_t reserve(size_t count) {
+    release();
+    if (count == 0) count = 1;
+    void* q = nullptr;
+    const hipError_t e = hipMalloc(&q, count * sizeof(T));
+    if (e == hipSuccess) {
+      p = static_cast<T*>(q);
+      n = count;
+    }
+    return e;
+  }
 };
 
 }  // namespace g500

@@ -11,9 +11,11 @@
 // std::sort leaves them unspecified), which makes the whole CSR a pure
 // function of the edge list.
 //
-// Pipeline: atomics for degrees -> radix sort of (inverted degree, ID) keys ->
-// relabel maps -> (new_src, new_dst) keys, loops as a max-value sentinel ->
-// radix sort -> flag/scan/scatter dedupe into row offsets + uint32 columns.
+// Pipeline: degrees counted in LDS (csrsort.hip) -> IDs radix-sorted by
+// inverted degree -> relabel maps -> rows by bucket partition and LDS sort
+// (csrsort.hip).  Lists that partition cannot handle take the general form:
+// (new_src, new_dst) keys, loops as a max-value sentinel -> radix sort ->
+// flag/scan/scatter dedupe into row offsets + uint32 columns.
 #include <algorithm>
 
 #include "internal.hpp"
@@ -24,71 +26,43 @@ namespace {
 
 constexpr int kT = 256;
 
-__device__ inline uint64_t wave_or(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, kWave);
-  return v;
-}
-__device__ inline uint64_t wave_sum(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-__device__ inline uint64_t wave_max(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint64_t w = __shfl_xor(v, o, kWave);
-    v = w > v ? w : v;
-  }
-  return v;
-}
-
-// stats[0] |= endpoint IDs of non-loop edges, stats[1] += non-loop edges
-// (symmetric input: each directed edge counts once, toward its source)
-__global__ __launch_bounds__(kT) void k_degree(const uint2* __restrict__ e,
-                                              int64_t ne, int symmetric,
-                                              uint32_t* __restrict__ deg,
-                                              unsigned long long* stats) {
-  uint64_t orv = 0, cnt = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < ne;
-       i += (int64_t)gridDim.x * kT) {
-    const uint2 x = e[i];
-    if (x.x == x.y) continue;
-    atomicAdd(&deg[x.x], 1u);
-    if (!symmetric) atomicAdd(&deg[x.y], 1u);
-    orv |= (uint64_t)(x.x | x.y);
-    ++cnt;
-  }
-  orv = wave_or(orv);
-  cnt = wave_sum(cnt);
-  if (lane_id() == 0) {
-    if (orv) atomicOr(&stats[0], (unsigned long long)orv);
-    if (cnt) atomicAdd(&stats[1], (unsigned long long)cnt);
-  }
-}
-
 // stats[2] = max degree, stats[3] = #vertices with degree > 0,
-// stats[4] = max vertex with degree > 0
+// stats[4] = max vertex with degree > 0.  Three atomics a block: on one
+// address they take ~12 ns each in turn (one set per wave of 8 192 blocks cost
+// 1.14 ms at SCALE 24, now 0.03).
 __global__ __launch_bounds__(kT) void k_deg_stats(const uint32_t* __restrict__ deg,
                                                  int64_t n,
                                                  unsigned long long* stats) {
-  uint64_t mx = 0, nz = 0, mu = 0;
+  __shared__ uint64_t part[3][kT / kWave];
+  uint64_t x[3] = {0, 0, 0};
   for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < n;
        v += (int64_t)gridDim.x * kT) {
     const uint32_t d = deg[v];
-    mx = d > mx ? d : mx;
+    x[0] = d > x[0] ? d : x[0];
     if (d) {
-      ++nz;
-      mu = (uint64_t)v;
+      ++x[1];
+      x[2] = (uint64_t)v;
     }
   }
-  mx = wave_max(mx);
-  nz = wave_sum(nz);
-  mu = wave_max(mu);
-  if (lane_id() == 0) {
-    if (mx) atomicMax(&stats[2], (unsigned long long)mx);
-    if (nz) atomicAdd(&stats[3], (unsigned long long)nz);
-    if (mu) atomicMax(&stats[4], (unsigned long long)mu);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t a = __shfl_xor(x[0], o, kWave), c = __shfl_xor(x[2], o, kWave);
+    x[0] = a > x[0] ? a : x[0];
+    x[1] += __shfl_xor(x[1], o, kWave);
+    x[2] = c > x[2] ? c : x[2];
+  }
+  if (lane_id() == 0)
+    for (int j = 0; j < 3; ++j) part[j][threadIdx.x / kWave] = x[j];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kT / kWave; ++w) {
+      x[0] = part[0][w] > x[0] ? part[0][w] : x[0];
+      x[1] += part[1][w];
+      x[2] = part[2][w] > x[2] ? part[2][w] : x[2];
+    }
+    if (x[0]) atomicMax(&stats[2], (unsigned long long)x[0]);
+    if (x[1]) atomicAdd(&stats[3], (unsigned long long)x[1]);
+    if (x[2]) atomicMax(&stats[4], (unsigned long long)x[2]);
   }
 }
 
@@ -101,17 +75,17 @@ __global__ __launch_bounds__(kT) void k_vertex_keys(const uint32_t* __restrict__
 }
 
 __global__ __launch_bounds__(kT) void k_relabel(const uint64_t* __restrict__ keys,
-                                               int64_t n, uint64_t mask,
-                                               const uint32_t* __restrict__ deg,
+                                               int64_t n, int lg, uint64_t maxdeg,
                                                uint32_t* __restrict__ n2o,
                                                uint32_t* __restrict__ o2n,
                                                uint32_t* __restrict__ deg_new) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (i >= n) return;
-  const uint32_t o = (uint32_t)(keys[i] & mask);
+  const uint64_t k = keys[i];
+  const uint32_t o = (uint32_t)(k & ((1ull << lg) - 1));
   n2o[i] = o;
   o2n[o] = (uint32_t)i;
-  deg_new[i] = deg[o];
+  deg_new[i] = (uint32_t)(maxdeg - (k >> lg));
 }
 
 // Two keys per input edge ((a,b) and (b,a)), or one when the input is
@@ -209,33 +183,75 @@ __global__ void k_set_i64(int64_t* p, int64_t v) { *p = v; }
 
 // Copy of each row's first entry with its original ID, stored densely so that
 // the bottom-up sweep reads both coalesced (the reference keeps the same
-// "isolated first edge", mpi/graph_constructor.hpp:1387-1557).
+// "isolated first edge", mpi/graph_constructor.hpp:1387-1557), and bit v of
+// `multi`: row v has more than one entry (a bottom-up vertex whose first
+// neighbour is unvisited has nothing else to scan otherwise).
 __global__ __launch_bounds__(kT) void k_first_nbr(const int64_t* __restrict__ row_off,
                                                  const uint32_t* __restrict__ col,
                                                  const uint32_t* __restrict__ n2o,
-                                                 int64_t n_c, uint2* __restrict__ first) {
+                                                 int64_t n_c, uint2* __restrict__ first,
+                                                 uint64_t* __restrict__ multi) {
   const int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x;
+  bool more = false;
   if (v < n_c) {
-    const uint32_t u = col[row_off[v]];
+    const int64_t beg = row_off[v];
+    const uint32_t u = col[beg];
     first[v] = make_uint2(u, n2o[u]);
+    more = row_off[v + 1] - beg > 1;
   }
-}
-
-// Bit v: row v has more than one entry (a bottom-up vertex whose first
-// neighbour is unvisited has nothing else to scan otherwise).
-__global__ __launch_bounds__(kT) void k_multi_bits(const int64_t* __restrict__ row_off,
-                                                  int64_t n_c, uint64_t* __restrict__ multi) {
-  const int64_t w = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (w * 64 >= n_c) return;
-  uint64_t bits = 0;
-  const int64_t v0 = w * 64;
-  const int cnt = (int)(n_c - v0 < 64 ? n_c - v0 : 64);
-  for (int b = 0; b < cnt; ++b)
-    if (row_off[v0 + b + 1] - row_off[v0 + b] > 1) bits |= 1ull << b;
-  multi[w] = bits;
+  // 64 consecutive vertices from a multiple of 64: one word
+  const uint64_t word = __ballot(more);
+  if (lane_id() == 0 && v < n_c) multi[v >> 6] = word;
 }
 
 int bitlen(uint64_t x) { return x ? 64 - __builtin_clzll(x) : 0; }
+
+// The general form: any list, the symmetric (new_src, new_dst) keys radix
+// sorted and then deduplicated (80 ms at SCALE 24, where the buckets take 24).
+void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
+  hipStream_t s = g->stream;
+  const int lg = g->log_n;
+  const int64_t n = g->n;
+  const int64_t nk = symmetric ? ne : 2 * ne;
+  DevBuf<uint64_t> ek, ek_alt;
+  ek.alloc((size_t)nk);
+  ek_alt.alloc((size_t)nk);
+  const uint64_t sentinel = ((uint64_t)(n - 1) << lg) | (uint64_t)(n - 1);
+  if (ne > 0) {
+    hipLaunchKernelGGL(k_sym_keys, dim3((unsigned)ceil_div(ne, kT)), dim3(kT), 0,
+                       s, edges, ne, (int)symmetric, g->orig2new.get(), lg, sentinel,
+                       ek.get());
+    G500_CHECK_LAUNCH();
+  }
+  uint64_t* sorted = radix_sort_u64(ek.get(), ek_alt.get(), nk, 0, 2 * lg,
+                                    g->radix_ws, s);
+  const int64_t ms = g->m_sym;  // sentinels sort to the end
+  const int64_t tiles = std::max<int64_t>(1, ceil_div(ms, kDedupTile));
+  DevBuf<uint32_t> tcnt;
+  DevBuf<uint64_t> toff;
+  tcnt.alloc((size_t)tiles);
+  toff.alloc((size_t)tiles + 1);
+  hipLaunchKernelGGL(k_dedup_count, dim3((unsigned)tiles), dim3(kT), 0, s,
+                     sorted, ms, tcnt.get());
+  G500_CHECK_LAUNCH();
+  exclusive_scan<uint32_t>(tcnt.get(), toff.get(), tiles, g->scan_ws, s);
+  uint64_t m_total = 0;
+  G500_CHECK_HIP(hipMemcpyAsync(&m_total, toff.get() + tiles, sizeof(uint64_t),
+                                hipMemcpyDeviceToHost, s));
+  G500_CHECK_HIP(hipStreamSynchronize(s));
+  g->m = (int64_t)m_total;
+  // padding: bottom-up scans read aligned 16-byte groups, which may run a
+  // few entries past the last row
+  g->col.alloc((size_t)g->m + kColPad);
+  g->row_off.alloc((size_t)g->n_c + 1);
+  hipLaunchKernelGGL(k_dedup_write, dim3((unsigned)tiles), dim3(kT), 0, s,
+                     sorted, ms, lg, toff.get(), g->col.get(), g->row_off.get());
+  G500_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_set_i64, dim3(1), dim3(1), 0, s, g->row_off.get() + g->n_c,
+                     g->m);
+  G500_CHECK_LAUNCH();
+  G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
+}
 
 }  // namespace
 
@@ -250,14 +266,11 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
   DevBuf<uint32_t> deg;
   deg.alloc((size_t)nv);
   G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, nv * sizeof(uint32_t), s));
-  if (ne > 0) {
-    const int64_t blocks = std::min<int64_t>(ceil_div(ne, kT), 8192);
-    hipLaunchKernelGGL(k_degree, dim3((unsigned)blocks), dim3(kT), 0, s,
-                       edges, ne, (int)symmetric, deg.get(), stats.get());
-    G500_CHECK_LAUNCH();
-  }
+  if (ne > 0)
+    count_degrees(edges, ne, symmetric ? DegreeMode::kSourceNoLoops : DegreeMode::kBothEnds, nv,
+                  deg.get(), stats.get(), s);
   {
-    const int64_t blocks = std::min<int64_t>(ceil_div(nv, kT), 8192);
+    const int64_t blocks = std::min<int64_t>(ceil_div(nv, kT * 8), 1024);
     hipLaunchKernelGGL(k_deg_stats, dim3((unsigned)blocks), dim3(kT), 0, s,
                        deg.get(), nv, stats.get());
     G500_CHECK_LAUNCH();
@@ -289,66 +302,27 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
     hipLaunchKernelGGL(k_vertex_keys, dim3((unsigned)blocks), dim3(kT), 0, s,
                        deg.get(), n, lg, (uint64_t)maxdeg, vk.get());
     G500_CHECK_LAUNCH();
-    uint64_t* sorted = radix_sort_u64(vk.get(), vk_alt.get(), n,
+    // the IDs start in ascending order and the sort is stable: the degree bits
+    // alone decide
+    uint64_t* sorted = radix_sort_u64(vk.get(), vk_alt.get(), n, lg,
                                       lg + std::max(1, bitlen(maxdeg)),
                                       g->radix_ws, s);
     hipLaunchKernelGGL(k_relabel, dim3((unsigned)blocks), dim3(kT), 0, s, sorted,
-                       n, (uint64_t)(n - 1), deg.get(), g->new2orig.get(),
+                       n, lg, (uint64_t)maxdeg, g->new2orig.get(),
                        g->orig2new.get(), g->deg_new.get());
     G500_CHECK_LAUNCH();
     G500_CHECK_HIP(hipStreamSynchronize(s));
   }
   deg.release();
 
-  // ---- symmetric (new_src, new_dst) keys, sorted, then deduplicated
+  if (!build_rows(g, edges, ne, symmetric)) sort_rows(g, edges, ne, symmetric);
   {
-    const int64_t nk = symmetric ? ne : 2 * ne;
-    DevBuf<uint64_t> ek, ek_alt;
-    ek.alloc((size_t)nk);
-    ek_alt.alloc((size_t)nk);
-    const uint64_t sentinel = ((uint64_t)(n - 1) << lg) | (uint64_t)(n - 1);
-    if (ne > 0) {
-      hipLaunchKernelGGL(k_sym_keys, dim3((unsigned)ceil_div(ne, kT)), dim3(kT), 0,
-                         s, edges, ne, (int)symmetric, g->orig2new.get(), lg, sentinel,
-                         ek.get());
-      G500_CHECK_LAUNCH();
-    }
-    uint64_t* sorted = radix_sort_u64(ek.get(), ek_alt.get(), nk, 2 * lg,
-                                      g->radix_ws, s);
-    const int64_t ms = g->m_sym;  // sentinels sort to the end
-    const int64_t tiles = std::max<int64_t>(1, ceil_div(ms, kDedupTile));
-    DevBuf<uint32_t> tcnt;
-    DevBuf<uint64_t> toff;
-    tcnt.alloc((size_t)tiles);
-    toff.alloc((size_t)tiles + 1);
-    hipLaunchKernelGGL(k_dedup_count, dim3((unsigned)tiles), dim3(kT), 0, s,
-                       sorted, ms, tcnt.get());
-    G500_CHECK_LAUNCH();
-    exclusive_scan<uint32_t>(tcnt.get(), toff.get(), tiles, g->scan_ws, s);
-    uint64_t m_total = 0;
-    G500_CHECK_HIP(hipMemcpyAsync(&m_total, toff.get() + tiles, sizeof(uint64_t),
-                                  hipMemcpyDeviceToHost, s));
-    G500_CHECK_HIP(hipStreamSynchronize(s));
-    g->m = (int64_t)m_total;
-    // padding: bottom-up scans read aligned 16-byte groups, which may run a
-    // few entries past the last row
-    g->col.alloc((size_t)g->m + kColPad);
-    g->row_off.alloc((size_t)g->n_c + 1);
-    hipLaunchKernelGGL(k_dedup_write, dim3((unsigned)tiles), dim3(kT), 0, s,
-                       sorted, ms, lg, toff.get(), g->col.get(), g->row_off.get());
-    G500_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_set_i64, dim3(1), dim3(1), 0, s, g->row_off.get() + g->n_c,
-                       g->m);
-    G500_CHECK_LAUNCH();
     g->first.alloc((size_t)std::max<int64_t>(g->n_c, 1));
     g->multi.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), 64));
     if (g->n_c > 0) {
       hipLaunchKernelGGL(k_first_nbr, dim3((unsigned)ceil_div(g->n_c, kT)), dim3(kT), 0, s,
                          g->row_off.get(), g->col.get(), g->new2orig.get(), g->n_c,
-                         g->first.get());
-      G500_CHECK_LAUNCH();
-      hipLaunchKernelGGL(k_multi_bits, dim3((unsigned)ceil_div(ceil_div(g->n_c, 64), kT)),
-                         dim3(kT), 0, s, g->row_off.get(), g->n_c, g->multi.get());
+                         g->first.get(), g->multi.get());
       G500_CHECK_LAUNCH();
     }
     G500_CHECK_HIP(hipStreamSynchronize(s));

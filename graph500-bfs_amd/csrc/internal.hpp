@@ -76,6 +76,21 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
 void construct_graph(g500_graph* g, int corebfs);
 void ensure_host_orig2new(g500_graph* g);
 
+// csrsort.hip
+enum class DegreeMode {
+  kBothEnds,       // both endpoints of every edge that is no loop
+  kSourceNoLoops,  // the source of every edge that is no loop
+  kSourceEnd       // the source of every edge
+};
+// deg[v] += edges at v for IDs below nv; stats[0] |= the IDs of the edges
+// counted, stats[1] += their number
+void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, uint32_t* deg,
+                   unsigned long long* stats, hipStream_t s);
+// Sorted rows without repeated entries (g->m, col, row_off) from the edges,
+// g's maps and degrees.  False, with nothing kept, where this form cannot sort
+// them (an unexpected spread of a long row's targets, or too little memory).
+bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric);
+
 // corebfs.hip
 constexpr uint32_t kNoParent = 0xFFFFFFFFu;
 // entries allocated past the end of col (aligned 16-byte loads of a row's

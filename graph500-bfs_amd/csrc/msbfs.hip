@@ -58,13 +58,14 @@ __device__ inline uint64_t block_sum(uint64_t v, uint64_t* lds) {
 
 // Input edges by source vertex, by new ID: the traversed-edge count of a root
 // is the sum over the vertices it reaches (the validator counts an input edge
-// when its source is reached).
-__global__ __launch_bounds__(kT) void k_ms_cnt0(const uint2* __restrict__ e, int64_t ne,
-                                               const uint32_t* __restrict__ o2n,
+// when its source is reached).  The counts by original ID come from
+// count_degrees; here they move to their new IDs (an atomic per edge on the
+// new ID, the earlier form, took 112 ms at SCALE 26).
+__global__ __launch_bounds__(kT) void k_ms_cnt0(const uint32_t* __restrict__ deg_orig,
+                                               int64_t n, const uint32_t* __restrict__ o2n,
                                                uint32_t* __restrict__ cnt0) {
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < ne;
-       i += (int64_t)gridDim.x * kT)
-    atomicAdd(&cnt0[o2n[e[i].x]], 1u);
+  const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (o < n) cnt0[o2n[o]] = deg_orig[o];
 }
 
 // First new ID whose degree is below each threshold (deg_new is descending).
@@ -1855,6 +1856,22 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
   G500_CHECK_HIP(hipStreamCreate(&b->stream));
   G500_CHECK_HIP(hipEventCreate(&b->ev_begin));
   G500_CHECK_HIP(hipEventCreate(&b->ev_end));
+  // first, so that its scratch is gone before the engine's own arrays come
+  b->cnt0.alloc((size_t)g->n);
+  {
+    const int64_t nv = (int64_t)1 << g->id_bits;  // covers every input ID
+    DevBuf<uint32_t> deg;
+    DevBuf<unsigned long long> stats;
+    deg.alloc((size_t)nv);
+    stats.alloc(2);
+    G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, (size_t)nv * sizeof(uint32_t), b->stream));
+    count_degrees(g->edges.get(), g->nedges, DegreeMode::kSourceEnd, nv, deg.get(), stats.get(),
+                  b->stream);
+    hipLaunchKernelGGL(k_ms_cnt0, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, b->stream,
+                       deg.get(), g->n, g->orig2new.get(), b->cnt0.get());
+    G500_CHECK_LAUNCH();
+    G500_CHECK_HIP(hipStreamSynchronize(b->stream));
+  }
   const int64_t nc = std::max<int64_t>(1, g->n_c);
   b->seen.alloc((size_t)nc * b->kmax);
   b->fptr.alloc(kMaxLevels + 1);  // F_0..F_255
@@ -1873,21 +1890,12 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
   b->fb[1].alloc((size_t)bitmap_words(b));
   b->fe.alloc(kMaxLevels + 2);
   b->act.alloc((size_t)(kMaxLevels + 2) * 4);
-  b->cnt0.alloc((size_t)g->n);
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_roots, (G500_MSBFS_MAX_ROOTS + 1) * sizeof(int64_t),
                                hipHostMallocDefault));
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_cnt, (kMaxLevels + 2) * sizeof(unsigned long long),
                                hipHostMallocDefault));
   for (int l = 0; l < kInitialLevels; ++l) add_level_buffer(b);
 
-  G500_CHECK_HIP(hipMemsetAsync(b->cnt0.get(), 0, (size_t)g->n * sizeof(uint32_t), b->stream));
-  if (g->nedges > 0) {
-    const unsigned grid = (unsigned)std::max<int64_t>(
-        1, std::min<int64_t>(ceil_div(g->nedges, kT), (int64_t)num_cus(g->device) * 16));
-    hipLaunchKernelGGL(k_ms_cnt0, dim3(grid), dim3(kT), 0, b->stream, g->edges.get(),
-                       g->nedges, g->orig2new.get(), b->cnt0.get());
-    G500_CHECK_LAUNCH();
-  }
   if (g->m > 0) {
     // tiles of 2048 edges read entries 2t and 2t+2: room for both past the end
     b->stream_tile_v0.alloc((size_t)ceil_div(g->m, kStreamUnit) + 3);

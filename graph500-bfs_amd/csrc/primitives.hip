@@ -252,15 +252,15 @@ void RadixWorkspace::reserve(int64_t n) {
   cap = n;
 }
 
-uint64_t* radix_sort_u64(uint64_t* keys, uint64_t* alt, int64_t n, int bits,
+uint64_t* radix_sort_u64(uint64_t* keys, uint64_t* alt, int64_t n, int begin, int bits,
                          RadixWorkspace& ws, hipStream_t s) {
-  if (n <= 1 || bits <= 0) return keys;
+  if (n <= 1 || bits <= begin) return keys;
   ws.reserve(n);
   const int64_t tiles = ceil_div(n, kRadixTile);
   if (tiles > 0x7FFFFFFF) fail(G500_ERR_ARG, "radix sort: too many keys");
   uint64_t* src = keys;
   uint64_t* dst = alt;
-  for (int shift = 0; shift < bits; shift += 8) {
+  for (int shift = begin; shift < bits; shift += 8) {
     hipLaunchKernelGGL(k_rs_upsweep, dim3((unsigned)tiles), dim3(kRadixThreads),
                        0, s, src, n, shift, ws.counts.get(), tiles);
     G500_CHECK_LAUNCH();

@@ -30,9 +30,9 @@ struct RadixWorkspace {
   void reserve(int64_t n);
 };
 
-// Sorts keys[0..n) ascending on bits [0, bits).  `alt` must hold n keys.
-// Returns the buffer that holds the result (keys or alt).
-uint64_t* radix_sort_u64(uint64_t* keys, uint64_t* alt, int64_t n, int bits,
+// Sorts keys[0..n) ascending on bits [begin, bits), stable.  `alt` must hold
+// n keys.  Returns the buffer that holds the result (keys or alt).
+uint64_t* radix_sort_u64(uint64_t* keys, uint64_t* alt, int64_t n, int begin, int bits,
                          RadixWorkspace& ws, hipStream_t s);
 
 constexpr int kRadixItems = 32;              // keys per thread per tile
