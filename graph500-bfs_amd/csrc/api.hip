@@ -127,7 +127,7 @@ g500_graph* new_graph_with_capacity(int device, int64_t capacity) {
   if (capacity < 0) g500::fail(G500_ERR_ARG, "negative edge capacity");
   g500_graph* g = new_graph(device);
   try {
-    g->edges.alloc((size_t)capacity);
+    g->edges.alloc_raw((size_t)capacity);
     g->capacity = capacity;
   } catch (...) {
     delete g;
@@ -487,6 +487,7 @@ int g500_device_memory(int device, int64_t* free_bytes, int64_t* total_bytes) {
   return guard([&] {
     if (!free_bytes || !total_bytes) g500::fail(G500_ERR_ARG, "null output pointer");
     use_device(device);
+    g500::device_trim();
     size_t f = 0, t = 0;
     G500_CHECK_HIP(hipMemGetInfo(&f, &t));
     *free_bytes = (int64_t)f;

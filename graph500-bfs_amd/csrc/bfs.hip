@@ -2116,10 +2116,8 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
     }
   }
   // the steps still queued (guesses past the last level) return at once
-  b->vis.p = cur.vis;
-  b->vis_alt.p = cur.vis_alt;
-  b->q.p = cur.q;
-  b->nq.p = cur.nq;
+  if (b->vis.get() != cur.vis) b->vis.swap(b->vis_alt);
+  if (b->q.get() != cur.q) b->q.swap(b->nq);
   // the gather: per vertex with edges its original ID, new ID, entry read and
   // written; with CoreBFS every original ID (new ID and entry written) and
   // every vertex with edges' entry
@@ -2232,7 +2230,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
 void bfs_levels(g500_bfs* b, uint16_t* out) {
   g500_graph* g = b->g;
   DevBuf<uint16_t> lv;
-  lv.alloc((size_t)g->n);
+  lv.alloc_raw((size_t)g->n);
   hipLaunchKernelGGL(k_levels, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, b->stream,
                      b->pred.get(), g->n, lv.get());
   G500_CHECK_LAUNCH();

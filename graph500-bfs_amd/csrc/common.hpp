@@ -3,10 +3,12 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <stdexcept>
 #include <string>
+#include <utility>
 
 #include "../../include/g500bfs.h"
 
@@ -44,6 +46,16 @@ __device__ inline uint64_t lanemask_lt() {
   return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
+// Device memory (devmem.hip): bytes on the current device, from a block kept
+// from an earlier release where one fits (*used: it then holds old data).
+// *got and *device go back with device_release.  Null where there is no room.
+// scratch: freed again soon, so its size may be rounded up.
+void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* device);
+// Waits for the device's queued work, as hipFree does.
+void device_release(void* p, size_t bytes, int device);
+// Gives all kept blocks back to the device.
+void device_trim();
+
 // Device allocation owned by a host object.
 template <typename T>
 struct DevBuf {
@@ -53,36 +65,54 @@ struct DevBuf {
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() { release(); }
+  // a block that held other data is cleared, as the driver clears new ones
   void alloc(size_t count) {
-    const hipError_t e = reserve(count);
-    if (e != hipSuccess)
-      fail(G500_ERR_NOMEM, "hipMalloc(%zu bytes): %s", count * sizeof(T),
-           hipGetErrorString(e));
+    bool used;
+    reserve(count, false, &used);
+    if (used) G500_CHECK_HIP(hipMemset(p, 0, n * sizeof(T)));
   }
-  // false where the device has no room: for a caller that can do without
-  bool try_alloc(size_t count) {
-    if (reserve(count) == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
+  // for arrays that are written before they are read
+  void alloc_raw(size_t count) {
+    bool used;
+    reserve(count, false, &used);
+  }
+  // scratch that is written before it is read; false where the device has no
+  // room, for a caller that can do without
+  bool try_scratch(size_t count) {
+    bool used;
+    return take(count, true, &used);
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) device_release(p, bytes_, device_);
     p = nullptr;
     n = 0;
+  }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+    std::swap(bytes_, o.bytes_);
+    std::swap(device_, o.device_);
   }
   T* get() const { return p; }
 
  private:
-  hipError_t reserve(size_t count) {
+  size_t bytes_ = 0;
+  int device_ = 0;
+
+  bool take(size_t count, bool scratch, bool* used) {
     release();
     if (count == 0) count = 1;
-    void* q = nullptr;
-    const hipError_t e = hipMalloc(&q, count * sizeof(T));
-    if (e == hipSuccess) {
-      p = static_cast<T*>(q);
-      n = count;
+    p = static_cast<T*>(device_alloc(count * sizeof(T), scratch, used, &bytes_, &device_));
+    if (!p) {
+      (void)hipGetLastError();
+      return false;
     }
-    return e;
+    n = count;
+    return true;
+  }
+  void reserve(size_t count, bool scratch, bool* used) {
+    if (!take(count, scratch, used))
+      fail(G500_ERR_NOMEM, "hipMalloc(%zu bytes): out of memory", count * sizeof(T));
   }
 };
 

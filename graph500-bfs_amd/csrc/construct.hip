@@ -214,8 +214,8 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   const int64_t n = g->n;
   const int64_t nk = symmetric ? ne : 2 * ne;
   DevBuf<uint64_t> ek, ek_alt;
-  ek.alloc((size_t)nk);
-  ek_alt.alloc((size_t)nk);
+  ek.alloc_raw((size_t)nk);
+  ek_alt.alloc_raw((size_t)nk);
   const uint64_t sentinel = ((uint64_t)(n - 1) << lg) | (uint64_t)(n - 1);
   if (ne > 0) {
     hipLaunchKernelGGL(k_sym_keys, dim3((unsigned)ceil_div(ne, kT)), dim3(kT), 0,
@@ -229,8 +229,8 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   const int64_t tiles = std::max<int64_t>(1, ceil_div(ms, kDedupTile));
   DevBuf<uint32_t> tcnt;
   DevBuf<uint64_t> toff;
-  tcnt.alloc((size_t)tiles);
-  toff.alloc((size_t)tiles + 1);
+  tcnt.alloc_raw((size_t)tiles);
+  toff.alloc_raw((size_t)tiles + 1);
   hipLaunchKernelGGL(k_dedup_count, dim3((unsigned)tiles), dim3(kT), 0, s,
                      sorted, ms, tcnt.get());
   G500_CHECK_LAUNCH();
@@ -264,7 +264,7 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
   stats.alloc(8);
   G500_CHECK_HIP(hipMemsetAsync(stats.get(), 0, 8 * sizeof(unsigned long long), s));
   DevBuf<uint32_t> deg;
-  deg.alloc((size_t)nv);
+  deg.alloc_raw((size_t)nv);
   G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, nv * sizeof(uint32_t), s));
   if (ne > 0)
     count_degrees(edges, ne, symmetric ? DegreeMode::kSourceNoLoops : DegreeMode::kBothEnds, nv,
@@ -291,13 +291,13 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
   g->m_sym = symmetric ? nonloop : 2 * nonloop;
 
   // ---- relabel by (degree desc, id asc)
-  g->new2orig.alloc((size_t)n);
-  g->orig2new.alloc((size_t)n);
-  g->deg_new.alloc((size_t)n);
+  g->new2orig.alloc_raw((size_t)n);
+  g->orig2new.alloc_raw((size_t)n);
+  g->deg_new.alloc_raw((size_t)n);
   {
     DevBuf<uint64_t> vk, vk_alt;
-    vk.alloc((size_t)n);
-    vk_alt.alloc((size_t)n);
+    vk.alloc_raw((size_t)n);
+    vk_alt.alloc_raw((size_t)n);
     const int64_t blocks = ceil_div(n, kT);
     hipLaunchKernelGGL(k_vertex_keys, dim3((unsigned)blocks), dim3(kT), 0, s,
                        deg.get(), n, lg, (uint64_t)maxdeg, vk.get());
@@ -317,8 +317,8 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
 
   if (!build_rows(g, edges, ne, symmetric)) sort_rows(g, edges, ne, symmetric);
   {
-    g->first.alloc((size_t)std::max<int64_t>(g->n_c, 1));
-    g->multi.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), 64));
+    g->first.alloc_raw((size_t)std::max<int64_t>(g->n_c, 1));
+    g->multi.alloc_raw((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), 64));
     if (g->n_c > 0) {
       hipLaunchKernelGGL(k_first_nbr, dim3((unsigned)ceil_div(g->n_c, kT)), dim3(kT), 0, s,
                          g->row_off.get(), g->col.get(), g->new2orig.get(), g->n_c,

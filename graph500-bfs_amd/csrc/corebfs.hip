@@ -304,11 +304,11 @@ void corebfs_prune(g500_graph* g) {
   DevBuf<uint8_t> alive;
   DevBuf<unsigned long long> cnt;
   const int64_t nn = std::max<int64_t>(n_c, 1);
-  deg.alloc((size_t)nn);
-  par.alloc((size_t)nn);
-  leaves.alloc((size_t)nn);
-  twig.alloc((size_t)nn);
-  alive.alloc((size_t)nn);
+  deg.alloc_raw((size_t)nn);
+  par.alloc_raw((size_t)nn);
+  leaves.alloc_raw((size_t)nn);
+  twig.alloc_raw((size_t)nn);
+  alive.alloc_raw((size_t)nn);
   cnt.alloc(4);
   if (n_c > 0) {
     hipLaunchKernelGGL(k_core_init, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
@@ -339,8 +339,8 @@ void corebfs_prune(g500_graph* g) {
   twig.release();
 
   // 3. forest parents by original ID
-  g->tree_parent.alloc((size_t)n);
-  g->has_parent.alloc((size_t)ceil_div(n, 64));
+  g->tree_parent.alloc_raw((size_t)n);
+  g->has_parent.alloc_raw((size_t)ceil_div(n, 64));
   G500_CHECK_HIP(hipMemsetAsync(g->tree_parent.get(), 0xFF, n * sizeof(uint32_t), s));
   G500_CHECK_HIP(hipMemsetAsync(g->has_parent.get(), 0, ceil_div(n, 64) * sizeof(uint64_t), s));
   G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(unsigned long long), s));
@@ -357,9 +357,9 @@ void corebfs_prune(g500_graph* g) {
   const int64_t tiles = ceil_div(g->m, kFilterTile);
   DevBuf<uint32_t> tile_row, tile_cnt;
   DevBuf<uint64_t> tile_off;
-  tile_row.alloc((size_t)tiles);
-  tile_cnt.alloc((size_t)tiles);
-  tile_off.alloc((size_t)tiles + 1);
+  tile_row.alloc_raw((size_t)tiles);
+  tile_cnt.alloc_raw((size_t)tiles);
+  tile_off.alloc_raw((size_t)tiles + 1);
   if (tiles > 0) {
     hipLaunchKernelGGL(k_core_tile_rows, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
                        n_c, tile_row.get());
@@ -376,7 +376,7 @@ void corebfs_prune(g500_graph* g) {
                                 hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipStreamSynchronize(s));
   DevBuf<uint2> core_edges;
-  core_edges.alloc((size_t)std::max<uint64_t>(m_core, 1));
+  core_edges.alloc_raw((size_t)std::max<uint64_t>(m_core, 1));
   if (tiles > 0) {
     hipLaunchKernelGGL(k_core_filter<kWrite>, dim3((unsigned)tiles), dim3(kT), 0, s,
                        g->row_off.get(), g->col.get(), alive.get(), g->new2orig.get(),
@@ -423,7 +423,7 @@ void corebfs_reset_unreachable(g500_graph* g, const uint64_t* visited, hipStream
   const int64_t n = g->n;
   DevBuf<uint8_t> reach;
   DevBuf<unsigned long long> cnt;
-  reach.alloc((size_t)n);
+  reach.alloc_raw((size_t)n);
   cnt.alloc(1);
   hipLaunchKernelGGL(k_reach_init, dim3(blocks(n)), dim3(kT), 0, s, g->orig2new.get(),
                      visited, n, g->n_c, reach.get());

@@ -339,7 +339,7 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   // LDS; a sparse list over a large ID space keeps the atomics
   DevBuf<uint16_t> ep;
   const bool dense = ranges <= kMaxRanges && ne * kPer >= nv;
-  if (!dense || !ep.try_alloc((size_t)(ne * kPer))) {
+  if (!dense || !ep.try_scratch((size_t)(ne * kPer))) {
     hipLaunchKernelGGL(k_deg_atomic<kMode>,
                        dim3((unsigned)std::min<int64_t>(ceil_div(ne, 256), 4096)), dim3(256), 0, s,
                        edges, ne, deg, stats);
@@ -348,8 +348,8 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   }
   DevBuf<unsigned long long> total;  // per range, then (off) its first slot and a cursor
   DevBuf<uint64_t> off;
-  total.alloc((size_t)ranges);
-  off.alloc((size_t)ranges + 1);
+  total.alloc_raw((size_t)ranges);
+  off.alloc_raw((size_t)ranges + 1);
   ScanWorkspace ws;
   G500_CHECK_HIP(hipMemsetAsync(total.get(), 0, ranges * sizeof(unsigned long long), s));
   hipLaunchKernelGGL(k_deg_ranges<kMode>,
@@ -925,6 +925,20 @@ void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, 
   }
 }
 
+// g->col and g->row_off for m entries; false where the device has no room.
+// The last entries of col are padding: bottom-up scans read aligned 16-byte
+// groups, which may run a few entries past the last row.
+static bool take_rows(g500_graph* g, int64_t m) {
+  try {
+    g->col.alloc_raw((size_t)m + kColPad);
+    g->row_off.alloc_raw((size_t)g->n_c + 1);
+  } catch (const Error&) {
+    return false;
+  }
+  G500_CHECK_HIP(hipMemsetAsync(g->col.get() + m, 0, kColPad * sizeof(uint32_t), g->stream));
+  return true;
+}
+
 bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   hipStream_t s = g->stream;
   const int64_t keys = g->m_sym, n_c = g->n_c;
@@ -945,14 +959,14 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   DevBuf<uint32_t> cnt, ucnt, big, flag, uniq;
   DevBuf<unsigned long long> rows, cursor, gcursor;
   // without room for all this the radix sort still fits
-  if ((two && (!part.try_alloc((size_t)(groups * group_cap)) ||
-               !gcursor.try_alloc((size_t)groups))) ||
-      !sorted.try_alloc((size_t)keys) || (!two && !uniq.try_alloc((size_t)keys)) ||
-      !roff.try_alloc((size_t)n_c + 1) || !rows.try_alloc((size_t)n_c) ||
-      !spl.try_alloc((size_t)buckets) || !off.try_alloc((size_t)buckets + 1) ||
-      !ubase.try_alloc((size_t)buckets + 1) || !cnt.try_alloc((size_t)buckets) ||
-      !cursor.try_alloc((size_t)buckets) || !ucnt.try_alloc((size_t)buckets) ||
-      !big.try_alloc((size_t)buckets + 1) || !flag.try_alloc(1))
+  if ((two && (!part.try_scratch((size_t)(groups * group_cap)) ||
+               !gcursor.try_scratch((size_t)groups))) ||
+      !sorted.try_scratch((size_t)keys) || (!two && !uniq.try_scratch((size_t)keys)) ||
+      !roff.try_scratch((size_t)n_c + 1) || !rows.try_scratch((size_t)n_c) ||
+      !spl.try_scratch((size_t)buckets) || !off.try_scratch((size_t)buckets + 1) ||
+      !ubase.try_scratch((size_t)buckets + 1) || !cnt.try_scratch((size_t)buckets) ||
+      !cursor.try_scratch((size_t)buckets) || !ucnt.try_scratch((size_t)buckets) ||
+      !big.try_scratch((size_t)buckets + 1) || !flag.try_scratch(1))
     return false;
   exclusive_scan<uint32_t>(g->deg_new.get(), roff.get(), n_c, g->scan_ws, s);
   hipLaunchKernelGGL(k_splitters, dim3((unsigned)ceil_div(buckets, 256)), dim3(256), 0, s,
@@ -1010,7 +1024,7 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   G500_CHECK_HIP(hipMemcpyAsync(&m, ubase.get() + buckets, sizeof(m), hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipMemcpyAsync(&over, flag.get(), sizeof(over), hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipStreamSynchronize(s));
-  if (over || !g->col.try_alloc((size_t)m + kColPad) || !g->row_off.try_alloc((size_t)n_c + 1))
+  if (over || !take_rows(g, (int64_t)m))
     return false;
   g->m = (int64_t)m;
   hipLaunchKernelGGL(k_collect, dim3((unsigned)buckets), dim3(256), 0, s, un, off.get(),

@@ -1,0 +1,158 @@
+// devmem.hip -- device memory that is kept for the next allocation.
+//
+// hipMalloc and hipFree of large blocks are quick only until the driver has to
+// clear what was freed before: from then on an allocation costs ~30 ms per GB.
+// A graph built, searched and freed over and over (13 GB of blocks at SCALE 24)
+// took 170 to 470 ms each time that way, its kernels 40.  So blocks from 1 MiB
+// on are kept when they are released and handed out again, up to an eighth of
+// the device's memory; the oldest are given back first, all of them when an
+// allocation fails, when free memory is asked for (g500_device_memory) and,
+// at the next call, when no one took them for ten seconds.
+//
+// A block is kept only after the device has finished all work queued so far
+// (as hipFree waits for it), so whichever thread or stream takes it next has
+// it alone.
+#include <chrono>
+#include <mutex>
+#include <vector>
+
+#include "common.hpp"
+
+namespace g500 {
+
+namespace {
+
+constexpr size_t kKeepMin = size_t(1) << 20;
+constexpr size_t kGranule = size_t(2) << 20;
+constexpr int kIdleSeconds = 10;
+
+struct Block {
+  void* p;
+  size_t bytes;
+  int device;
+  std::chrono::steady_clock::time_point since;
+};
+
+// never destroyed: handles may be released by destructors that run after
+// those of this file
+struct Kept {
+  std::mutex mu;
+  std::vector<Block> blocks;  // oldest first
+};
+Kept& kept() {
+  static Kept* k = new Kept;
+  return *k;
+}
+
+size_t keep_limit(int device) {
+  static std::mutex mu;
+  static std::vector<size_t> limit;
+  std::lock_guard<std::mutex> lock(mu);
+  if ((int)limit.size() <= device) limit.resize((size_t)device + 1, 0);
+  if (limit[(size_t)device] == 0) {
+    size_t total = 0;
+    hipDeviceProp_t prop;
+    if (hipGetDeviceProperties(&prop, device) == hipSuccess) total = prop.totalGlobalMem;
+    limit[(size_t)device] = total / 8 + 1;
+  }
+  return limit[(size_t)device];
+}
+
+void free_blocks(const std::vector<Block>& out) {
+  for (const Block& b : out) (void)hipFree(b.p);
+}
+
+}  // namespace
+
+void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* device) {
+  *used = false;
+  *got = bytes;
+  *device = 0;
+  (void)hipGetDevice(device);
+  void* p = nullptr;
+  if (bytes < kKeepMin) return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+  size_t want = (bytes + kGranule - 1) / kGranule * kGranule;
+  if (scratch) {
+    // sizes that differ a little (another seed's graph) share a block
+    const size_t step = std::max(kGranule, (size_t(1) << (63 - __builtin_clzll(want))) / 16);
+    want = (want + step - 1) / step * step;
+  }
+  const size_t most = want + (scratch ? want / 8 : want / 64);
+  std::vector<Block> old;
+  {
+    Kept& k = kept();
+    std::lock_guard<std::mutex> lock(k.mu);
+    size_t best = k.blocks.size();
+    for (size_t i = 0; i < k.blocks.size(); ++i) {
+      const Block& b = k.blocks[i];
+      if (b.device == *device && b.bytes >= want && b.bytes <= most &&
+          (best == k.blocks.size() || b.bytes < k.blocks[best].bytes))
+        best = i;
+    }
+    if (best < k.blocks.size()) {
+      p = k.blocks[best].p;
+      *got = k.blocks[best].bytes;
+      *used = true;
+      k.blocks.erase(k.blocks.begin() + (ptrdiff_t)best);
+    }
+    const auto limit = std::chrono::steady_clock::now() - std::chrono::seconds(kIdleSeconds);
+    while (!k.blocks.empty() && k.blocks.front().since < limit) {
+      old.push_back(k.blocks.front());
+      k.blocks.erase(k.blocks.begin());
+    }
+  }
+  free_blocks(old);
+  if (p) return p;
+  *got = want;
+  if (hipMalloc(&p, want) == hipSuccess) return p;
+  (void)hipGetLastError();
+  device_trim();
+  if (hipMalloc(&p, want) == hipSuccess) return p;
+  (void)hipGetLastError();
+  *got = bytes;
+  return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+}
+
+void device_release(void* p, size_t bytes, int device) {
+  int current = 0;
+  (void)hipGetDevice(&current);
+  const size_t limit = keep_limit(device);
+  // the wait fails only beside a capture that forbids it or after a fault:
+  // the block then goes back at once
+  if (bytes < kKeepMin || bytes > limit || current != device ||
+      hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipFree(p);
+    return;
+  }
+  std::vector<Block> old;
+  {
+    Kept& k = kept();
+    std::lock_guard<std::mutex> lock(k.mu);
+    k.blocks.push_back({p, bytes, device, std::chrono::steady_clock::now()});
+    size_t total = 0;
+    for (const Block& b : k.blocks) total += b.device == device ? b.bytes : 0;
+    for (size_t i = 0; i < k.blocks.size() && total > limit;) {
+      if (k.blocks[i].device != device) {
+        ++i;
+        continue;
+      }
+      total -= k.blocks[i].bytes;
+      old.push_back(k.blocks[i]);
+      k.blocks.erase(k.blocks.begin() + (ptrdiff_t)i);
+    }
+  }
+  free_blocks(old);
+}
+
+void device_trim() {
+  std::vector<Block> old;
+  {
+    Kept& k = kept();
+    std::lock_guard<std::mutex> lock(k.mu);
+    old.swap(k.blocks);
+  }
+  free_blocks(old);
+}
+
+}  // namespace g500

@@ -188,7 +188,7 @@ void generate_edges(g500_graph* g, int scale, int edgefactor, uint64_t seed1,
   a.val1 = sv[1];
   a.nedges = ne;
   a.scale = scale;
-  g->edges.alloc((size_t)ne);
+  g->edges.alloc_raw((size_t)ne);
   g->nedges = ne;
   g->id_bits = scale;
   const int64_t threads = ceil_div(ne, kEdgesPerThread);

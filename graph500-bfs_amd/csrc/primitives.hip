@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kRadixThreads) void k_rs_downsweep(
 void ScanWorkspace::reserve(int64_t n) {
   const int64_t need = scan_ws_need(n) + 1;
   if (need <= cap) return;
-  buf.alloc((size_t)need);
+  buf.alloc_raw((size_t)need);
   cap = need;
 }
 
@@ -246,8 +246,8 @@ template void exclusive_scan<uint64_t>(const uint64_t*, uint64_t*, int64_t,
 void RadixWorkspace::reserve(int64_t n) {
   if (n <= cap) return;
   const int64_t tiles = ceil_div(n, kRadixTile);
-  counts.alloc((size_t)(256 * tiles));
-  offsets.alloc((size_t)(256 * tiles + 1));
+  counts.alloc_raw((size_t)(256 * tiles));
+  offsets.alloc_raw((size_t)(256 * tiles + 1));
   scan.reserve(256 * tiles);
   cap = n;
 }
