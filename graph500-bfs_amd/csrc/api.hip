@@ -87,8 +87,8 @@ void need_result(g500_msbfs* b) {
 }
 bool has_edge_host(g500_graph* g, int64_t v) {
   if (v < 0 || v >= g->n) return false;
-  g500::ensure_host_orig2new(g);
-  if ((int64_t)g->h_orig2new[(size_t)v] < g->n_c) return true;
+  g500::ensure_edge_bits(g);
+  if (g500::has_csr_edge(g, v)) return true;
   return g500::has_parent_host(g, v);
 }
 

@@ -250,10 +250,13 @@ struct LoopInit {
 // its reservations there -- and the first step).
 __global__ __launch_bounds__(kT) void k_bfs_init(uint64_t* __restrict__ vis,
                                                 int64_t words, int64_t n_c,
-                                                int64_t root_new, int64_t* pred_new,
+                                                int64_t root, const uint32_t* __restrict__ o2n,
+                                                int64_t* pred_new,
                                                 int64_t entry, uint32_t* q, LevelSync* ls,
                                                 LoopInit li,
                                                 const int64_t* __restrict__ row_off) {
+  // root: an original ID with an edge, or -1
+  const int64_t root_new = root >= 0 ? (int64_t)o2n[root] : -1;
   for (int64_t w = (int64_t)blockIdx.x * kT + threadIdx.x; w < words;
        w += (int64_t)gridDim.x * kT) {
     const int64_t lo = w * 64;
@@ -1468,7 +1471,7 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
     b->n_core = g->n_c;
     b->pred_fill_needed = true;
   }
-  ensure_host_orig2new(g);
+  ensure_edge_bits(g);
   if (const char* ea = getenv("G500_EXEC_ALPHA")) b->exec_alpha = atof(ea);
   if (const char* sp = getenv("G500_SPECULATE")) b->spec_depth = std::max(0, atoi(sp));
   if (const char* gw = getenv("G500_GUESS")) b->guess_wrong = std::strcmp(gw, "wrong") == 0;
@@ -1949,8 +1952,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
       }
     }
   }
-  const int64_t root_new = g->h_orig2new.empty() ? -1 : (int64_t)g->h_orig2new[bfs_root];
-  const bool root_in = root_new >= 0 && root_new < n_c;
+  const bool root_in = has_csr_edge(g, bfs_root);
 
   b->trace.clear();
   b->stats = g500_run_stats{};
@@ -1979,6 +1981,9 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
     G500_CHECK_HIP(hipMemsetAsync(b->wacc.get(), 0, b->wacc.n * sizeof(uint64_t), s));
     if (root_in) {
       int64_t ro[2];
+      uint32_t root_new = 0;
+      G500_CHECK_HIP(hipMemcpy(&root_new, g->orig2new.get() + bfs_root, sizeof(root_new),
+                               hipMemcpyDeviceToHost));
       G500_CHECK_HIP(hipMemcpyAsync(ro, g->row_off.get() + root_new, sizeof(ro),
                                     hipMemcpyDeviceToHost, s));
       G500_CHECK_HIP(hipStreamSynchronize(s));
@@ -2002,8 +2007,8 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   LoopInit li{first, root_in ? 1 : 0, 0, hl.alpha_thr, hl.beta_thr, hl.exec_thr};
   G500_CHECK_HIP(hipEventRecord(b->ev_begin, s));
   hipLaunchKernelGGL(k_bfs_init, dim3(grid_for(words, kT)), dim3(kT), 0, s,
-                     b->vis.get(), words, n_c, root_in ? root_new : (int64_t)-1,
-                     b->pred_new.get(),
+                     b->vis.get(), words, n_c, root_in ? bfs_root : (int64_t)-1,
+                     g->orig2new.get(), b->pred_new.get(),
                      (int64_t)(((uint64_t)root_level << 48) | ((uint64_t)b->epoch << 32) |
                                (uint64_t)bfs_root),
                      b->q.get(),

@@ -204,6 +204,16 @@ __global__ __launch_bounds__(kT) void k_first_nbr(const int64_t* __restrict__ ro
   if (lane_id() == 0 && v < n_c) multi[v >> 6] = word;
 }
 
+// Bit o: original ID o has a CSR edge.  The host keeps these n bits to answer
+// has_edge and to place a run's root; the map itself (32 times as much, the
+// earlier form) took 15 of an engine's first 57 ms to copy at SCALE 24.
+__global__ __launch_bounds__(kT) void k_edge_bits(const uint32_t* __restrict__ o2n, int64_t n,
+                                                 int64_t n_c, uint64_t* __restrict__ bits) {
+  const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
+  const uint64_t word = __ballot(o < n && (int64_t)o2n[o] < n_c);
+  if (lane_id() == 0 && o < n) bits[o >> 6] = word;
+}
+
 int bitlen(uint64_t x) { return x ? 64 - __builtin_clzll(x) : 0; }
 
 // The general form: any list, the symmetric (new_src, new_dst) keys radix
@@ -327,7 +337,7 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
     }
     G500_CHECK_HIP(hipStreamSynchronize(s));
   }
-  g->h_orig2new.clear();
+  g->h_edge_bits.clear();
 }
 
 void construct_graph(g500_graph* g, int corebfs) {
@@ -336,11 +346,19 @@ void construct_graph(g500_graph* g, int corebfs) {
   g->constructed = true;
 }
 
-void ensure_host_orig2new(g500_graph* g) {
-  if (!g->h_orig2new.empty() || g->n == 0) return;
-  g->h_orig2new.resize((size_t)g->n);
-  G500_CHECK_HIP(hipMemcpy(g->h_orig2new.data(), g->orig2new.get(),
-                           g->n * sizeof(uint32_t), hipMemcpyDeviceToHost));
+void ensure_edge_bits(g500_graph* g) {
+  if (!g->h_edge_bits.empty() || g->n == 0) return;
+  const int64_t words = ceil_div(g->n, 64);
+  DevBuf<uint64_t> bits;
+  bits.alloc_raw((size_t)words);
+  hipLaunchKernelGGL(k_edge_bits, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, g->stream,
+                     g->orig2new.get(), g->n, g->n_c, bits.get());
+  G500_CHECK_LAUNCH();
+  std::vector<uint64_t> h((size_t)words);
+  G500_CHECK_HIP(hipMemcpyAsync(h.data(), bits.get(), words * sizeof(uint64_t),
+                                hipMemcpyDeviceToHost, g->stream));
+  G500_CHECK_HIP(hipStreamSynchronize(g->stream));
+  g->h_edge_bits.swap(h);
 }
 
 }  // namespace g500
@@ -350,5 +368,6 @@ int64_t g500_graph::device_bytes() const {
                    col.n * sizeof(uint32_t) + first.n * sizeof(uint2) +
                    multi.n * sizeof(uint64_t) +
                    (deg_new.n + new2orig.n + orig2new.n) * sizeof(uint32_t) +
-                   tree_parent.n * sizeof(uint32_t) + has_parent.n * sizeof(uint64_t));
+                   tree_parent.n * sizeof(uint32_t) + has_parent.n * sizeof(uint64_t) +
+                   ordered.n * sizeof(uint64_t) + edge_chunks.n * sizeof(g500::EdgeChunk));
 }

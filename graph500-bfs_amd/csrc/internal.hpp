@@ -3,10 +3,46 @@
 #pragma once
 
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
 #include "primitives.hpp"
+
+namespace g500 {
+// The input edges ordered for the validator (order_edges): by the target's
+// window of 2^kEdgeWindowBits IDs, then the source's slice of
+// 2^kEdgeSliceBits, then the target's part of its window.  64 bits each, from
+// the top: window, slice, part (part_bits), the source's place in its slice,
+// the target's in its part.  Chunks hold edges of one window and slice.
+constexpr int kEdgeWindowBits = 21;
+constexpr int kEdgeSliceBits = 16;
+constexpr int kEdgePartBits = 11;  // at most
+constexpr int64_t kEdgeChunk = 1 << 17;
+constexpr int64_t kOrderedEdgesMin = 1 << 20;
+constexpr int kOrderedIdBits = 28;
+struct EdgeChunk {
+  uint64_t first;
+  uint32_t count, window, slice, unused;
+};
+__host__ __device__ inline uint64_t edge_key(uint32_t s, uint32_t t, int slices_log,
+                                             int part_bits) {
+  const int low = kEdgeWindowBits - part_bits;
+  const uint64_t tile =
+      (((uint64_t)(t >> kEdgeWindowBits) << slices_log | s >> kEdgeSliceBits) << part_bits) |
+      ((t >> low) & ((1u << part_bits) - 1));
+  return tile << (kEdgeSliceBits + low) |
+         (uint64_t)(s & ((1u << kEdgeSliceBits) - 1)) << low | (t & ((1u << low) - 1));
+}
+// the source's place in its slice and the target's in its window
+__host__ __device__ inline void edge_places(uint64_t key, int part_bits, uint32_t* s,
+                                            uint32_t* t) {
+  const int low = kEdgeWindowBits - part_bits;
+  *s = (uint32_t)(key >> low) & ((1u << kEdgeSliceBits) - 1);
+  *t = (((uint32_t)(key >> (kEdgeSliceBits + low)) & ((1u << part_bits) - 1)) << low) |
+       ((uint32_t)key & ((1u << low) - 1));
+}
+}  // namespace g500
 
 struct g500_graph {
   int device = 0;
@@ -38,8 +74,9 @@ struct g500_graph {
   g500::DevBuf<uint32_t> new2orig;  // n
   g500::DevBuf<uint32_t> orig2new;  // n
 
-  // host copy of orig2new (lazily made for has_edge / root selection)
-  std::vector<uint32_t> h_orig2new;
+  // bit v: original ID v has a CSR edge (host copy, lazily made for has_edge,
+  // root selection and each run's root)
+  std::vector<uint64_t> h_edge_bits;
 
   // CoreBFS (corebfs != 0): forest parents by original ID (kNoParent = none
   // or reset as unreachable) and the bitmap of vertices that were given a
@@ -51,6 +88,15 @@ struct g500_graph {
   bool core_reset_done = false;           // reset_unreachable applied
   int64_t core_vertices = 0, tree_vertices = 0, removed_parents = 0;
   int64_t hd_root = -1;                   // highest-degree core vertex
+
+  // the input edges once more, in the validator's order (made by the first
+  // validation of a graph large enough, empty otherwise)
+  std::mutex order_mu;  // engines of one graph may validate at the same time
+  bool order_tried = false;
+  g500::DevBuf<uint64_t> ordered;
+  g500::DevBuf<g500::EdgeChunk> edge_chunks;
+  int64_t n_edge_chunks = 0;
+  int edge_part_bits = 0;
 
   g500::ScanWorkspace scan_ws;
   g500::RadixWorkspace radix_ws;
@@ -74,7 +120,10 @@ void generate_edges(g500_graph* g, int scale, int edgefactor, uint64_t seed1,
 void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
                int force_log_n);
 void construct_graph(g500_graph* g, int corebfs);
-void ensure_host_orig2new(g500_graph* g);
+void ensure_edge_bits(g500_graph* g);
+inline bool has_csr_edge(const g500_graph* g, int64_t v) {
+  return (g->h_edge_bits[(size_t)(v >> 6)] >> (v & 63)) & 1ull;
+}
 
 // csrsort.hip
 enum class DegreeMode {
@@ -90,6 +139,10 @@ void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, 
 // g's maps and degrees.  False, with nothing kept, where this form cannot sort
 // them (an unexpected spread of a long row's targets, or too little memory).
 bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric);
+
+// g->ordered and its chunks; false where the edges are few, their IDs too wide
+// or memory is short
+bool order_edges(g500_graph* g, hipStream_t s);
 
 // corebfs.hip
 constexpr uint32_t kNoParent = 0xFFFFFFFFu;
