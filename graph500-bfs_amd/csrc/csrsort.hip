@@ -412,9 +412,19 @@ __global__ __launch_bounds__(256) void k_splitters(const uint64_t* __restrict__ 
 }
 
 // The bucket of a key: the last lower bound (LDS, spl[0] below every key) at
-// or before it.
-__device__ inline int part_of(const uint64_t* spl, int parts, uint64_t key) {
-  int lo = 0, hi = parts;
+// or before it, or where the bounds are the multiples of 2^shift (shift > 0)
+// from first << shift on, the key's upper bits.
+struct Parts {
+  const uint64_t* spl;
+  int parts;
+  int shift;
+  uint64_t first;
+};
+
+__device__ inline int part_of(const Parts& p, uint64_t key) {
+  if (p.shift > 0) return (int)((key >> p.shift) - p.first);
+  const uint64_t* spl = p.spl;
+  int lo = 0, hi = p.parts;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (spl[mid] <= key) lo = mid;
@@ -430,16 +440,15 @@ struct PartLds {
 
 // Keys per bucket of a tile's keys (kPartItems a thread; bit k of `use`: item
 // k holds one).
-__device__ inline void part_count(const uint64_t* spl, uint32_t* hist, int parts,
-                                  const uint64_t (&key)[kPartItems], uint32_t use,
-                                  uint32_t* __restrict__ cnt) {
-  for (int i = threadIdx.x; i < parts; i += kSortT) hist[i] = 0;
+__device__ inline void part_count(const Parts& p, uint32_t* hist, const uint64_t (&key)[kPartItems],
+                                  uint32_t use, uint32_t* __restrict__ cnt) {
+  for (int i = threadIdx.x; i < p.parts; i += kSortT) hist[i] = 0;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < kPartItems; ++k)
-    if ((use >> k) & 1u) atomicAdd(&hist[part_of(spl, parts, key[k])], 1u);
+    if ((use >> k) & 1u) atomicAdd(&hist[part_of(p, key[k])], 1u);
   __syncthreads();
-  for (int i = threadIdx.x; i < parts; i += kSortT)
+  for (int i = threadIdx.x; i < p.parts; i += kSortT)
     if (hist[i]) atomicAdd(&cnt[i], hist[i]);
 }
 
@@ -449,18 +458,18 @@ __device__ inline void part_count(const uint64_t* spl, uint32_t* hist, int parts
 // only use places below (b + 1) * cap; what does not fit raises *overflow.
 // pack_shift: a staged key carries its bucket above this bit (64: no room, the
 // bucket is searched for again).
-__device__ inline void part_move(PartLds& l, const uint64_t* spl, uint32_t* hist, int64_t* place,
-                                 int parts, const uint64_t (&key)[kPartItems], uint32_t use,
+__device__ inline void part_move(PartLds& l, const Parts& p, uint32_t* hist, int64_t* place,
+                                 const uint64_t (&key)[kPartItems], uint32_t use,
                                  int pack_shift, unsigned long long* __restrict__ cursor,
                                  int64_t cap, uint64_t* __restrict__ out, uint32_t* overflow) {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, parts = p.parts;
   for (int i = t; i < parts; i += kSortT) hist[i] = 0;
   __syncthreads();
   uint32_t at[kPartItems];  // bucket << 13 | rank in it
 #pragma unroll
   for (int k = 0; k < kPartItems; ++k)
     if ((use >> k) & 1u) {
-      const uint32_t b = (uint32_t)part_of(spl, parts, key[k]);
+      const uint32_t b = (uint32_t)part_of(p, key[k]);
       at[k] = (b << 13) | atomicAdd(&hist[b], 1u);
     }
   __syncthreads();
@@ -502,10 +511,10 @@ __device__ inline void part_move(PartLds& l, const uint64_t* spl, uint32_t* hist
       b = (int)(x >> pack_shift);
       x &= (1ull << pack_shift) - 1;
     } else {
-      b = part_of(spl, parts, x);
+      b = part_of(p, x);
     }
-    const int64_t p = place[b] + j;
-    if (cap == 0 || p < (int64_t)(b + 1) * cap) out[p] = x;
+    const int64_t q = place[b] + j;
+    if (cap == 0 || q < (int64_t)(b + 1) * cap) out[q] = x;
   }
 }
 
@@ -513,20 +522,27 @@ __device__ inline void part_move(PartLds& l, const uint64_t* spl, uint32_t* hist
 // `parts` buckets.
 constexpr size_t part_lds(int64_t parts) { return (size_t)parts * 20; }
 
-// From the edges: the keys of a tile -- both directions, or the one the list
-// holds -- counted by or moved into the buckets of every step-th bound.
-template <bool kSym, bool kMove>
+// What a key is made of: both directions of an edge by new IDs, the one the
+// list holds, or the edge itself (loops too) by original IDs as edge_key puts it
+// (lg: log2 of the slices; step: the part bits).
+enum { kKeyBoth = 0, kKeyOne = 1, kKeyEdge = 2 };
+
+// From the edges: the keys of a tile counted by or moved into the buckets of
+// every step-th bound (spl), or of the keys' bits from `shift` on.
+template <int kKind, bool kMove>
 __global__ __launch_bounds__(kSortT) void k_part_edges(
     const uint2* __restrict__ e, int64_t ne, const uint32_t* __restrict__ o2n, int lg,
-    const uint64_t* __restrict__ spl, int64_t step, int parts, int pack_shift,
+    const uint64_t* __restrict__ spl, int64_t step, int parts, int shift, int pack_shift,
     uint32_t* __restrict__ cnt, unsigned long long* __restrict__ cursor, int64_t cap,
     uint64_t* __restrict__ out, uint32_t* overflow) {
   extern __shared__ uint64_t dyn[];
   uint64_t* s = dyn;
   int64_t* place = (int64_t*)(dyn + parts);
   uint32_t* hist = (uint32_t*)(dyn + 2 * parts);
-  for (int i = threadIdx.x; i < parts; i += kSortT) s[i] = spl[(int64_t)i * step];
-  constexpr int kEdges = kSym ? kPartItems : kPartItems / 2;
+  if (kKind != kKeyEdge)
+    for (int i = threadIdx.x; i < parts; i += kSortT) s[i] = spl[(int64_t)i * step];
+  const Parts p{s, parts, kKind == kKeyEdge ? shift : 0, 0};
+  constexpr int kEdges = kKind == kKeyBoth ? kPartItems / 2 : kPartItems;
   const int64_t base = (int64_t)blockIdx.x * (kEdges * kSortT);
   uint64_t key[kPartItems];
   uint32_t use = 0;
@@ -538,12 +554,17 @@ __global__ __launch_bounds__(kSortT) void k_part_edges(
   }
 #pragma unroll
   for (int k = 0; k < kEdges; ++k) {
+    if constexpr (kKind == kKeyEdge) {
+      key[k] = edge_key(x[k].x, x[k].y, lg, (int)step);
+      use |= (uint32_t)(base + k * kSortT + threadIdx.x < ne) << k;
+      continue;
+    }
     const bool ok = x[k].x != x[k].y;
     const uint64_t a = ok ? o2n[x[k].x] : 0u, b = ok ? o2n[x[k].y] : 0u;
-    if (kSym) {
+    if constexpr (kKind == kKeyOne) {
       key[k] = (a << lg) | b;
       use |= (uint32_t)ok << k;
-    } else {
+    } else if constexpr (kKind == kKeyBoth) {
       key[2 * k] = (a << lg) | b;
       key[2 * k + 1] = (b << lg) | a;
       use |= (ok ? 3u : 0u) << (2 * k);
@@ -551,30 +572,39 @@ __global__ __launch_bounds__(kSortT) void k_part_edges(
   }
   if constexpr (kMove) {
     __shared__ PartLds l;
-    part_move(l, s, hist, place, parts, key, use, pack_shift, cursor, cap, out, overflow);
+    part_move(l, p, hist, place, key, use, pack_shift, cursor, cap, out, overflow);
   } else {
-    part_count(s, hist, parts, key, use, cnt);
+    part_count(p, hist, key, use, cnt);
   }
 }
 
-// From group blockIdx.y (keys from g * in_cap up to in_end[g]): its keys
-// counted by or moved into its buckets.
+// From group blockIdx.y: its keys counted by or moved into its buckets.  The
+// group's keys begin at g * in_cap, or with in_cap 0 where the previous
+// group's end, and end at in_end[g].
 template <bool kMove>
 __global__ __launch_bounds__(kSortT) void k_part_keys(
     const uint64_t* __restrict__ in, const unsigned long long* __restrict__ in_end,
-    int64_t in_cap, const uint64_t* __restrict__ spl, int64_t buckets, int step, int pack_shift,
-    uint32_t* __restrict__ cnt, unsigned long long* __restrict__ cursor,
+    int64_t in_cap, const uint64_t* __restrict__ spl, int64_t buckets, int step, int shift,
+    int pack_shift, uint32_t* __restrict__ cnt, unsigned long long* __restrict__ cursor,
     uint64_t* __restrict__ out) {
   extern __shared__ uint64_t dyn[];
   const int64_t g = blockIdx.y;
-  const int64_t end = (int64_t)in_end[g] < (g + 1) * in_cap ? (int64_t)in_end[g] : (g + 1) * in_cap;
-  const int64_t base = g * in_cap + (int64_t)blockIdx.x * kPartTile;
+  int64_t beg, end = (int64_t)in_end[g];
+  if (in_cap > 0) {
+    beg = g * in_cap;
+    end = end < beg + in_cap ? end : beg + in_cap;
+  } else {
+    beg = g > 0 ? (int64_t)in_end[g - 1] : 0;
+  }
+  const int64_t base = beg + (int64_t)blockIdx.x * kPartTile;
   if (base >= end) return;
   const int parts = (int)(buckets - g * step < step ? buckets - g * step : step);
   uint64_t* s = dyn;
   int64_t* place = (int64_t*)(dyn + step);
   uint32_t* hist = (uint32_t*)(dyn + 2 * step);
-  for (int i = threadIdx.x; i < parts; i += kSortT) s[i] = spl[g * step + i];
+  if (shift == 0)
+    for (int i = threadIdx.x; i < parts; i += kSortT) s[i] = spl[g * step + i];
+  const Parts p{s, parts, shift, (uint64_t)(g * step)};
   uint64_t key[kPartItems];
   uint32_t use = 0;
 #pragma unroll
@@ -585,9 +615,9 @@ __global__ __launch_bounds__(kSortT) void k_part_keys(
   }
   if constexpr (kMove) {
     __shared__ PartLds l;
-    part_move(l, s, hist, place, parts, key, use, pack_shift, cursor + g * step, 0, out, nullptr);
+    part_move(l, p, hist, place, key, use, pack_shift, cursor + g * step, 0, out, nullptr);
   } else {
-    part_count(s, hist, parts, key, use, cnt + g * step);
+    part_count(p, hist, key, use, cnt + g * step);
   }
 }
 
@@ -980,18 +1010,18 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   const unsigned tiles = (unsigned)ceil_div(ne, symmetric ? kPartTile : kPartTile / 2);
   auto from_edges = [&](auto kernel, unsigned long long* cur, int64_t cap, uint64_t* out) {
     hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kSortT), part_lds(groups), s, edges, ne,
-                       g->orig2new.get(), lg, spl.get(), step, (int)groups, pack, cnt.get(), cur,
+                       g->orig2new.get(), lg, spl.get(), step, (int)groups, 0, pack, cnt.get(), cur,
                        cap, out, flag.get());
     G500_CHECK_LAUNCH();
   };
   auto from_groups = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(group_cap, kPartTile), (unsigned)groups),
                        dim3(kSortT), part_lds(step), s, part.get(), gcursor.get(), group_cap,
-                       spl.get(), buckets, (int)step, pack, cnt.get(), cursor.get(),
+                       spl.get(), buckets, (int)step, 0, pack, cnt.get(), cursor.get(),
                        sorted.get());
     G500_CHECK_LAUNCH();
   };
-  auto move_edges = symmetric ? k_part_edges<true, true> : k_part_edges<false, true>;
+  auto move_edges = symmetric ? k_part_edges<kKeyOne, true> : k_part_edges<kKeyBoth, true>;
   if (two) {
     hipLaunchKernelGGL(k_group_places, dim3((unsigned)ceil_div(groups, 256)), dim3(256), 0, s,
                        gcursor.get(), (int)groups, group_cap);
@@ -999,7 +1029,7 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
     from_edges(move_edges, gcursor.get(), group_cap, part.get());
     from_groups(k_part_keys<false>);
   } else {
-    from_edges(symmetric ? k_part_edges<true, false> : k_part_edges<false, false>, nullptr, 0,
+    from_edges(symmetric ? k_part_edges<kKeyOne, false> : k_part_edges<kKeyBoth, false>, nullptr, 0,
                nullptr);
   }
   exclusive_scan<uint32_t>(cnt.get(), off.get(), buckets, g->scan_ws, s);
@@ -1034,6 +1064,101 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
                      rows.get(), ubase.get(), n_c, g->m, g->row_off.get());
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
+  return true;
+}
+
+bool order_edges(g500_graph* g, hipStream_t s) {
+  const int64_t ne = g->nedges;
+  if (ne < kOrderedEdgesMin || g->id_bits > kOrderedIdBits) return false;
+  size_t free_b = 0, total_b = 0;
+  G500_CHECK_HIP(hipMemGetInfo(&free_b, &total_b));
+  if ((uint64_t)ne * sizeof(uint64_t) > total_b / 16) return false;
+  const int wlog = std::max(0, g->id_bits - kEdgeWindowBits);
+  const int slog = std::max(0, g->id_bits - kEdgeSliceBits);
+  // as many parts of a window as two passes can tell apart
+  int pass_log = 0;
+  while ((1 << (pass_log + 1)) <= kMaxParts) ++pass_log;
+  const int part_bits = std::min(kEdgePartBits, 2 * pass_log - wlog - slog);
+  if (part_bits < 0) return false;
+  const int tile_shift = kEdgeSliceBits + kEdgeWindowBits - part_bits;
+  const int64_t tiles = (int64_t)1 << (wlog + slog + part_bits);
+  int step_log = 0;
+  if (tiles > kMaxParts)
+    while (((int64_t)1 << (2 * step_log)) < tiles) ++step_log;
+  const int64_t step = (int64_t)1 << step_log, groups = ceil_div(tiles, step);
+  DevBuf<uint64_t> part, keys, off;
+  DevBuf<uint32_t> cnt;
+  DevBuf<unsigned long long> cursor;
+  if ((step > 1 && !part.try_scratch((size_t)ne)) || !keys.try_scratch((size_t)ne) ||
+      !off.try_scratch((size_t)tiles + 1) || !cnt.try_scratch((size_t)tiles) ||
+      !cursor.try_scratch((size_t)tiles))
+    return false;
+  const unsigned blocks = (unsigned)ceil_div(ne, kPartTile);
+  // places of the buckets from their counts
+  auto places = [&](int64_t n) {
+    exclusive_scan<uint32_t>(cnt.get(), off.get(), n, g->scan_ws, s);
+    G500_CHECK_HIP(hipMemcpyAsync(cursor.get(), off.get(), n * sizeof(uint64_t),
+                                  hipMemcpyDeviceToDevice, s));
+  };
+  auto from_edges = [&](auto kernel, uint64_t* out) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kSortT), part_lds(groups), s, g->edges.get(),
+                       ne, (const uint32_t*)nullptr, slog, (const uint64_t*)nullptr,
+                       (int64_t)part_bits, (int)groups, tile_shift + step_log, 64, cnt.get(), cursor.get(),
+                       (int64_t)0, out, (uint32_t*)nullptr);
+    G500_CHECK_LAUNCH();
+  };
+  G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, groups * sizeof(uint32_t), s));
+  from_edges(k_part_edges<kKeyEdge, false>, nullptr);
+  places(groups);
+  from_edges(k_part_edges<kKeyEdge, true>, step > 1 ? part.get() : keys.get());
+  if (step > 1) {
+    std::vector<uint32_t> h((size_t)groups);
+    DevBuf<unsigned long long> gend;  // the cursors stand at the groups' ends now
+    gend.alloc_raw((size_t)groups);
+    G500_CHECK_HIP(hipMemcpyAsync(gend.get(), cursor.get(), groups * sizeof(uint64_t),
+                                  hipMemcpyDeviceToDevice, s));
+    G500_CHECK_HIP(hipMemcpyAsync(h.data(), cnt.get(), groups * sizeof(uint32_t),
+                                  hipMemcpyDeviceToHost, s));
+    G500_CHECK_HIP(hipStreamSynchronize(s));
+    const unsigned most = (unsigned)std::max<int64_t>(
+        1, ceil_div((int64_t)*std::max_element(h.begin(), h.end()), kPartTile));
+    auto from_groups = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(most, (unsigned)groups), dim3(kSortT), part_lds(step), s,
+                         part.get(), gend.get(), (int64_t)0, (const uint64_t*)nullptr, tiles,
+                         (int)step, tile_shift, 64, cnt.get(), cursor.get(), keys.get());
+      G500_CHECK_LAUNCH();
+    };
+    G500_CHECK_HIP(hipMemsetAsync(cnt.get(), 0, tiles * sizeof(uint32_t), s));
+    from_groups(k_part_keys<false>);
+    places(tiles);
+    from_groups(k_part_keys<true>);
+    G500_CHECK_HIP(hipStreamSynchronize(s));  // gend is freed here
+  }
+  // chunks of the edges of one window and slice
+  std::vector<uint64_t> h((size_t)tiles + 1);
+  G500_CHECK_HIP(hipMemcpyAsync(h.data(), off.get(), h.size() * sizeof(uint64_t),
+                                hipMemcpyDeviceToHost, s));
+  G500_CHECK_HIP(hipStreamSynchronize(s));
+  std::vector<EdgeChunk> chunks;
+  const size_t parts = (size_t)1 << part_bits;
+  for (uint32_t w = 0; w < 1u << wlog; ++w)
+    for (uint32_t c = 0; c < 1u << slog; ++c) {
+      const size_t i = (((size_t)w << slog) + c) * parts;
+      const uint64_t beg = h[i], end = h[i + parts];
+      // even pieces
+      const uint64_t pieces = (uint64_t)ceil_div((int64_t)(end - beg), kEdgeChunk);
+      for (uint64_t k = 0; k < pieces; ++k) {
+        const uint64_t a = beg + (end - beg) * k / pieces, e = beg + (end - beg) * (k + 1) / pieces;
+        chunks.push_back({a, (uint32_t)(e - a), w, c, 0});
+      }
+    }
+  g->edge_chunks.alloc_raw(chunks.size());
+  G500_CHECK_HIP(hipMemcpyAsync(g->edge_chunks.get(), chunks.data(),
+                                chunks.size() * sizeof(EdgeChunk), hipMemcpyHostToDevice, s));
+  G500_CHECK_HIP(hipStreamSynchronize(s));
+  g->ordered.swap(keys);
+  g->n_edge_chunks = (int64_t)chunks.size();
+  g->edge_part_bits = part_bits;
   return true;
 }
 

@@ -90,7 +90,8 @@ struct g500_bfs {
   int64_t unreach = 0;  // vertices with edges the last run left unreached
 
   // validation scratch
-  g500::DevBuf<unsigned long long> vcount;  // [G500_VERR_NUM + 2]
+  g500::DevBuf<unsigned long long> vcount;  // error and edge counts (validate.hip)
+  g500::DevBuf<uint8_t> vcode;              // depth and parent bits per vertex, by slices
   g500::DevBuf<uint8_t> pred_valid;         // n
 
   hipEvent_t ev_begin = nullptr, ev_end = nullptr;
