@@ -180,6 +180,7 @@ struct MsLevel {
   const uint64_t* act_l;   // lanes present anywhere in F_L (4 words)
   uint64_t* act_n;         // the same for F_{L+1}, ORed by the kernels that write it
   unsigned long long thr;
+  unsigned long long mark_thr;
   const int64_t* d_roots;  // [0] = batch size
   double stream_frac;
   int64_t n_c;
@@ -193,6 +194,9 @@ struct MsLevel {
   unsigned long long* lane_part;
   uint64_t* split_mask;
 };
+
+// top-down levels over at least m / kMarkShare frontier edges push without marks
+constexpr int64_t kMarkShare = 64;
 
 enum { kModeTopDown = 0, kModeStream = 1, kModePull = 2, kModeSplit = 3 };
 // rows of per-lane degree sums for a split level: block b of a top-down
@@ -215,6 +219,15 @@ enum { kDenseStream = 1, kDenseHybrid = 2 };
 
 __device__ inline bool ms_active(const MsLevel& a) { return a.cnt[a.L] != 0; }
 __device__ inline bool ms_top_down(const MsLevel& a, int l) { return a.fe[l] < a.thr; }
+// A top-down level's pushes mark their targets in the next bitmap only where
+// the frontier is light; beyond mark_thr edges the count pass finds the
+// non-empty words by reading all of F_{L+1} instead.  On a heavy level the
+// marks cost far more than the lanes themselves: rows are sorted, so the
+// lanes of a wave hit the same bitmap word at once, and atomics on one address
+// are taken one at a time (the heavy rows' pushes of one level: 1.17 -> 0.08 ms
+// at SCALE 20 with 64 roots, 2.07 -> 1.47 at SCALE 26 with 128).  The light
+// levels keep the marks: reading all of F_{L+1} costs 0.05-0.1 ms.
+__device__ inline bool ms_marks(const MsLevel& a) { return a.fe[a.L] < a.mark_thr; }
 // top-down while the frontier is light; else a streaming pull while few
 // (root, vertex) pairs are reached yet, then a per-vertex pull -- split at
 // the first bottom-up level after top-down ones (light roots push)
@@ -309,13 +322,15 @@ __device__ inline void push_targets(const uint32_t* col, int64_t e0, int64_t ste
 // afterwards from F_{L+1} by k_ms_td_count.  The bitmap word is read beside
 // seen so a vertex already in the next frontier costs no second atomic.
 template <int K>
-__device__ inline void ms_push_n(const MsLevel& a, const uint32_t (&w)[kPushIlp],
+__device__ inline void ms_push_n(const MsLevel& a, bool mark, const uint32_t (&w)[kPushIlp],
                                  const bool (&ok)[kPushIlp], const uint64_t (&f)[K]) {
   uint64_t sw[kPushIlp][K], bw[kPushIlp];
 #pragma unroll
-  for (int u = 0; u < kPushIlp; ++u) {
-    load_lanes<K>(a.seen + (int64_t)w[u] * K, sw[u]);
-    bw[u] = __hip_atomic_load(&a.fbn[w[u] >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int u = 0; u < kPushIlp; ++u) load_lanes<K>(a.seen + (int64_t)w[u] * K, sw[u]);
+  if (mark) {
+#pragma unroll
+    for (int u = 0; u < kPushIlp; ++u)
+      bw[u] = __hip_atomic_load(&a.fbn[w[u] >> 6], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 #pragma unroll
   for (int u = 0; u < kPushIlp; ++u) {
@@ -329,7 +344,7 @@ __device__ inline void ms_push_n(const MsLevel& a, const uint32_t (&w)[kPushIlp]
         any = true;
       }
     }
-    if (any && !(bw[u] & bit))
+    if (mark && any && !(bw[u] & bit))
       atomicOr((unsigned long long*)&a.fbn[w[u] >> 6], (unsigned long long)bit);
   }
 }
@@ -377,7 +392,7 @@ __global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, int64_t vb, int64_t v
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModeTopDown && mode != kModeSplit) return;
-  const bool split = mode == kModeSplit;
+  const bool split = mode == kModeSplit, mark = ms_marks(a);
   uint64_t pm[K];
   if (!push_lanes<K>(a, split, pm)) return;
   const int lig = threadIdx.x % G;
@@ -402,7 +417,7 @@ __global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, int64_t vb, int64_t v
       if (split)
         hyb_push_n<K>(a, w, ok, f);
       else
-        ms_push_n<K>(a, w, ok, f);
+        ms_push_n<K>(a, mark, w, ok, f);
     }
   }
 }
@@ -416,7 +431,7 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModeTopDown && mode != kModeSplit) return;
-  const bool split = mode == kModeSplit;
+  const bool split = mode == kModeSplit, mark = ms_marks(a);
   uint64_t pm[K];
   if (!push_lanes<K>(a, split, pm)) return;
   const int lane = lane_id();
@@ -443,7 +458,7 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
       if (split)
         hyb_push_n<K>(a, w, ok, f);
       else
-        ms_push_n<K>(a, w, ok, f);
+        ms_push_n<K>(a, mark, w, ok, f);
     }
   }
 }
@@ -468,11 +483,25 @@ __global__ __launch_bounds__(kT) void k_ms_td_count(MsLevel a) {
   uint64_t disc = 0, edges = 0, lanes[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) lanes[k] = 0;
-  for (int64_t v = (int64_t)blockIdx.x * kT + threadIdx.x; v < a.n_c;
-       v += (int64_t)gridDim.x * kT) {
-    if (!in_bitmap(a.fbn, v)) continue;
+  const bool marked = ms_marks(a);
+  // wave-uniform: 64 consecutive vertices from a multiple of 64, one bitmap word
+  for (int64_t v0 = (int64_t)blockIdx.x * kT + (threadIdx.x & ~(kWave - 1)); v0 < a.n_c;
+       v0 += (int64_t)gridDim.x * kT) {
+    const int64_t v = v0 + lane_id();
+    const uint64_t word = marked ? a.fbn[v0 >> 6] : ~0ull;
+    if (word == 0) continue;
     uint64_t x[K];
-    load_lanes<K>(a.fn + v * K, x);
+    bool any = false;
+    if (v < a.n_c && ((word >> lane_id()) & 1ull)) {
+      load_lanes<K>(a.fn + v * K, x);
+#pragma unroll
+      for (int k = 0; k < K; ++k) any = any || x[k] != 0;
+    }
+    if (!marked) {
+      const uint64_t found = __ballot(any);
+      if (lane_id() == 0) a.fbn[v0 >> 6] = found;
+    }
+    if (!any) continue;
     const unsigned long long d = a.deg[v];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -1472,6 +1501,7 @@ MsLevel level_args(const g500_msbfs* b, int L) {
   a.act_l = b->act.get() + (int64_t)L * 4;
   a.act_n = b->act.get() + (int64_t)(L + 1) * 4;
   a.thr = b->td_threshold;
+  a.mark_thr = (unsigned long long)(g->m / kMarkShare);
   a.d_roots = b->roots.get();
   a.stream_frac = b->tuning.stream_frac;
   a.dense_algo = b->tuning.dense_algo;
