@@ -598,8 +598,8 @@ __global__ __launch_bounds__(kT) void k_td_expand(
   if (t == 0) epart[blockIdx.x] = s;
 }
 
-// Bottom-up levels.  A wave owns a chunk of 64 bitmap words (4096 vertices)
-// and, for it, a segment of 4096 entries in the unvisited lists: after a
+// Bottom-up levels.  A wave owns a chunk of cw bitmap words (64 cw vertices)
+// and, for it, a segment of as many entries in the unvisited lists: after a
 // bottom-up level the segment's first unv_cnt[chunk] entries are the chunk's
 // still-unvisited vertices.  The first bottom-up level after top-down ones
 // sweeps the bitmap (k_bu_sweep); later ones walk the lists (k_bu_list),
@@ -616,7 +616,15 @@ __global__ __launch_bounds__(kT) void k_td_expand(
 // and 2979-3005).  The parent is the first visited neighbour in row order.
 constexpr int kBuIlp = 8;   // vertices in flight per lane
 constexpr int kBuBatch = kWave * kBuIlp;
-constexpr int kChunkVerts = kWave * 64;
+// Words per chunk: 64 where that leaves every resident wave several chunks,
+// else down to 8 (one batch of vertices per lane): with 64 everywhere the 2^18
+// vertices of SCALE 18 kept 42 waves busy on 256 CUs, and SCALE 24 half the
+// resident ones.  A run at SCALE 18 / 22 / 24 / 26: 0.24 / 0.40 / 0.535 / 1.07
+// ms before, 0.18 / 0.31 / 0.475 / 1.05 now; one or two chunks per wave cost
+// 1-3 % at SCALE 24 and 26, eight 3 % at SCALE 26 (shorter deferred lists).
+constexpr int kMaxChunkWords = kWave;
+constexpr int kMinChunkWords = kBuIlp;
+constexpr int kChunksPerWave = 4;
 // The visited bits of the lowest new IDs (the highest degrees) sit in LDS:
 // most first neighbours are such hubs, so most probes never leave the CU.
 constexpr int kHubWords = 4096;
@@ -732,7 +740,7 @@ constexpr int kBuStep = 8;  // row entries a lane probes per step (two uint4 loa
 
 __global__ __launch_bounds__(kBuT) void k_bu_sweep(
     const uint64_t* __restrict__ vis_old, uint64_t* __restrict__ vis_new,
-    int64_t words, const int64_t* __restrict__ row_off,
+    int64_t words, int cw, const int64_t* __restrict__ row_off,
     const uint32_t* __restrict__ col, const uint2* __restrict__ first,
     const uint64_t* __restrict__ multi, const uint32_t* __restrict__ n2o,
     int64_t* __restrict__ pred_new, uint32_t* __restrict__ unv,
@@ -745,16 +753,18 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
   __shared__ uint64_t hub[kHubWords];
   const VisProbe visited = stage_hubs(hub, vis_old, words);
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const int64_t nchunks = ceil_div(words, kWave);
+  const int64_t nchunks = ceil_div(words, cw);
+  const uint32_t cverts = (uint32_t)cw * 64u;
   const bool count = wacc != nullptr;  // counting runs tally the row-scan bytes
   uint64_t nfound = 0, scan_b = 0;
   for (int64_t c = (int64_t)blockIdx.x * kBuWaves + wave; c < nchunks;
        c += (int64_t)gridDim.x * kBuWaves) {
-    const int64_t w = c * kWave + lane;
-    const uint64_t myword = w < words ? vis_old[w] : ~0ull;
-    const uint64_t mymulti = w < words ? multi[w] : 0ull;
-    uint32_t* useg = unv + c * kChunkVerts;
-    const uint32_t vbase = (uint32_t)(c * kChunkVerts);
+    const int64_t w = c * cw + lane;
+    const bool own = lane < cw && w < words;  // lane l: word l of the chunk
+    const uint64_t myword = own ? vis_old[w] : ~0ull;
+    const uint64_t mymulti = own ? multi[w] : 0ull;
+    uint32_t* useg = unv + c * cverts;
+    const uint32_t vbase = (uint32_t)(c * cverts);
     uint64_t newbits = 0;  // lane l: bits found in word l of the chunk
     // final misses fill the segment from the front, deferred row scans from
     // the back; together they never exceed the chunk's unvisited vertices
@@ -771,7 +781,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
       okn[j] = !((readlane64(myword, j) >> lane) & 1ull);
       fn[j] = okn[j] ? get_pair(first + vbase + (uint32_t)(j * 64 + lane)) : make_uint2(0u, 0u);
     }
-    for (int j0 = 0; j0 < kWave; j0 += kBuIlp) {
+    for (int j0 = 0; j0 < cw; j0 += kBuIlp) {
       uint32_t v[kBuIlp];
       uint2 f[kBuIlp];
       bool ok[kBuIlp], hit[kBuIlp], fin[kBuIlp], defer[kBuIlp];
@@ -781,7 +791,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
         f[j] = fn[j];
         v[j] = vbase + (uint32_t)((j0 + j) * 64 + lane);
       }
-      if (j0 + kBuIlp < kWave) {
+      if (j0 + kBuIlp < cw) {
 #pragma unroll
         for (int j = 0; j < kBuIlp; ++j) {
           okn[j] = !((readlane64(myword, j0 + kBuIlp + j) >> lane) & 1ull);
@@ -811,7 +821,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
           if (fin[j] || defer[j]) {
             const uint32_t pos =
                 fin[j] ? wp + addf + (uint32_t)__popcll(mf & below)
-                       : kChunkVerts - dn - 1 - (addd + (uint32_t)__popcll(md & below));
+                       : cverts - dn - 1 - (addd + (uint32_t)__popcll(md & below));
             __builtin_nontemporal_store(v[j], useg + pos);
           }
           addf += (uint32_t)__popcll(mf);
@@ -830,7 +840,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
     fw[wave][lane] = 0;
     wave_sync();
     {
-      const uint32_t dbase = kChunkVerts - dn;
+      const uint32_t dbase = cverts - dn;
       uint32_t taken = 0;  // wave-uniform
       bool have = false;
       uint32_t dv = 0;
@@ -904,7 +914,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
     }
     wave_sync();
     newbits |= fw[wave][lane];
-    if (w < words) vis_new[w] = myword | newbits;
+    if (own) vis_new[w] = myword | newbits;
     nfound += (uint64_t)__popcll(newbits);
     if (lane == 0) unv_cnt[c] = wp;
     // the entries of the vertices found, and the chunk's unvisited list
@@ -925,6 +935,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_sweep(
 // unvisited list.
 __global__ __launch_bounds__(kBuT) void k_bu_long(
     const uint64_t* __restrict__ vis_old, unsigned long long* vis_new, int64_t words,
+    int cw,
     const int64_t* __restrict__ row_off, const uint32_t* __restrict__ col,
     const uint32_t* __restrict__ n2o, int64_t* __restrict__ pred_new,
     uint32_t* __restrict__ unv, uint32_t* unv_cnt,
@@ -978,9 +989,9 @@ __global__ __launch_bounds__(kBuT) void k_bu_long(
         atomicOr(vis_new + (v >> 6), 1ull << (v & 63));
         ++nfound;
       } else {
-        const uint32_t c = v / (uint32_t)kChunkVerts;
+        const uint32_t cverts = (uint32_t)cw * 64u, c = v / cverts;
         const uint32_t pos = atomicAdd(unv_cnt + c, 1u);
-        unv[(int64_t)c * kChunkVerts + pos] = v;
+        unv[(int64_t)c * cverts + pos] = v;
       }
     }
   }
@@ -998,7 +1009,7 @@ __global__ __launch_bounds__(kBuT) void k_bu_long(
 // latency-bound.
 __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void k_bu_list(
     const uint64_t* __restrict__ vis_old, uint64_t* __restrict__ vis_new,
-    int64_t words, const int64_t* __restrict__ row_off,
+    int64_t words, int cw, const int64_t* __restrict__ row_off,
     const uint32_t* __restrict__ col, const uint2* __restrict__ first,
     const uint64_t* __restrict__ multi, const uint32_t* __restrict__ n2o,
     int64_t* __restrict__ pred_new, uint32_t* __restrict__ unv,
@@ -1010,16 +1021,18 @@ __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void 
   __shared__ uint64_t hub[kHubWords];
   const VisProbe visited = stage_hubs(hub, vis_old, words);
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const int64_t nchunks = ceil_div(words, kWave);
+  const int64_t nchunks = ceil_div(words, cw);
+  const uint32_t cverts = (uint32_t)cw * 64u;
   const bool count = wacc != nullptr;
   uint64_t nfound = 0, scan_b = 0;
   for (int64_t c = (int64_t)blockIdx.x * kBuWaves + wave; c < nchunks;
        c += (int64_t)gridDim.x * kBuWaves) {
-    const int64_t w = c * kWave + lane;
-    const uint64_t myword = w < words ? vis_old[w] : ~0ull;
+    const int64_t w = c * cw + lane;
+    const bool own = lane < cw && w < words;
+    const uint64_t myword = own ? vis_old[w] : ~0ull;
     const uint32_t n = unv_cnt[c];
-    uint32_t* useg = unv + c * kChunkVerts;
-    const uint32_t vbase = (uint32_t)(c * kChunkVerts);
+    uint32_t* useg = unv + c * cverts;
+    const uint32_t vbase = (uint32_t)(c * cverts);
     fw[wave][lane] = 0;
     wave_sync();
     // compaction in place: misses of a batch land below the next batch, so
@@ -1078,7 +1091,7 @@ __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void 
     }
     wave_sync();
     const uint64_t fbits = fw[wave][lane];
-    if (w < words) vis_new[w] = myword | fbits;
+    if (own) vis_new[w] = myword | fbits;
     nfound += (uint64_t)__popcll(fbits);
     if (lane == 0) unv_cnt[c] = wp;
     if (count) scan_b += 8u * (uint64_t)__popcll(fbits) + (lane == 0 ? 4u * (uint64_t)wp : 0u);
@@ -1408,9 +1421,6 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   b->boff.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile));
   b->prep_ticket.alloc(1);
   G500_CHECK_HIP(hipMemset(b->prep_ticket.get(), 0, sizeof(unsigned int)));
-  const int64_t chunks = ceil_div(b->words, kWave);
-  b->unv.alloc((size_t)(chunks * kChunkVerts));
-  b->unv_cnt.alloc((size_t)chunks);
   // bottom-up grids: what stays resident (each block stages the hub bits
   // once), never more blocks than chunk groups
   int cus = 0, per_cu[3] = {0, 0, 0};
@@ -1421,6 +1431,15 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
       &per_cu[1], reinterpret_cast<const void*>(&k_bu_list), kBuT, 0));
   G500_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &per_cu[2], reinterpret_cast<const void*>(&k_bu_long), kBuT, 0));
+  // chunks for the waves the sweep keeps resident, kChunksPerWave each
+  b->chunk_words = kMaxChunkWords;
+  while (b->chunk_words > kMinChunkWords &&
+         ceil_div(b->words, b->chunk_words) <
+             (int64_t)cus * std::max(per_cu[0], 1) * kBuWaves * kChunksPerWave)
+    b->chunk_words /= 2;
+  const int64_t chunks = ceil_div(b->words, b->chunk_words);
+  b->unv.alloc((size_t)(chunks * b->chunk_words * 64));
+  b->unv_cnt.alloc((size_t)chunks);
   for (int i = 0; i < 3; ++i)
     b->bu_grid[i] = (unsigned)std::max<int64_t>(
         1, std::min<int64_t>((int64_t)std::max(cus, 1) * std::max(per_cu[i], 1),
@@ -1620,13 +1639,13 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
     *nsweep_ev += 2;
     G500_CHECK_HIP(hipEventRecord(pool_event(b->sweep_events, st.sweep_ev), s));
     hipLaunchKernelGGL(k_bu_sweep, dim3(b->bu_grid[0]), dim3(kBuT), 0, s, in.vis, in.vis_alt,
-                       b->words, g->row_off.get(), g->col.get(), g->first.get(),
+                       b->words, b->chunk_words, g->row_off.get(), g->col.get(), g->first.get(),
                        g->multi.get(), g->new2orig.get(), b->pred_new.get(), b->unv.get(),
                        b->unv_cnt.get(), in.nq, ls, code, b->lpart.get(), level_bits, wsweep);
     G500_CHECK_LAUNCH();
     G500_CHECK_HIP(hipEventRecord(pool_event(b->sweep_events, st.sweep_ev + 1), s));
     hipLaunchKernelGGL(k_bu_long, dim3(b->bu_grid[2]), dim3(kBuT), 0, s, in.vis,
-                       (unsigned long long*)in.vis_alt, b->words, g->row_off.get(),
+                       (unsigned long long*)in.vis_alt, b->words, b->chunk_words, g->row_off.get(),
                        g->col.get(), g->new2orig.get(), b->pred_new.get(), b->unv.get(),
                        b->unv_cnt.get(), in.nq, ls, code, b->lpart.get() + b->bu_grid[0],
                        level_bits, wlong);
@@ -1685,7 +1704,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       break;
     case kModeBUList:
       hipLaunchKernelGGL(k_bu_list, dim3(b->bu_grid[1]), dim3(kBuT), 0, s, in.vis, in.vis_alt,
-                         b->words, g->row_off.get(), g->col.get(), g->first.get(),
+                         b->words, b->chunk_words, g->row_off.get(), g->col.get(), g->first.get(),
                          g->multi.get(), g->new2orig.get(), b->pred_new.get(), b->unv.get(),
                          b->unv_cnt.get(), ls, code, b->lpart.get(), level_bits, wlist);
       G500_CHECK_LAUNCH();

@@ -72,8 +72,9 @@ struct g500_bfs {
   g500::DevBuf<uint32_t> tile_owner; // frontier index owning each top-down tile's first edge
   g500::DevBuf<uint64_t> bsum, boff;  // per prep block: degree total, its offset
   g500::DevBuf<unsigned int> prep_ticket;  // blocks done in the prep's first launch
-  // unvisited vertices after a bottom-up level: 4096 entries per chunk of 64
-  // bitmap words, unv_cnt[chunk] of them in use
+  // unvisited vertices after a bottom-up level: an entry per vertex of each
+  // chunk of chunk_words bitmap words, unv_cnt[chunk] of them in use
+  int chunk_words = 64;
   g500::DevBuf<uint32_t> unv, unv_cnt;
   unsigned bu_grid[3] = {1, 1, 1};  // resident blocks of the sweep / list / long-row kernels
   g500::DevBuf<LevelSync> lsync;   // level-loop state on the device
