@@ -28,11 +28,17 @@ struct Mat5 {
   uint32_t a[25];  // row-major
 };
 
-// x < 2^62 -> x mod (2^31 - 1), using 2^31 == 1 (mod m).
+// x < 2^62 -> x mod (2^31 - 1), using 2^31 == 1 (mod m).  The first fold fits
+// 32 bits, so the second is plain 32-bit arithmetic.
 __host__ __device__ inline uint32_t mrg_reduce(uint64_t x) {
-  uint64_t r = (x & kMrgP) + (x >> 31);
+  uint32_t r = ((uint32_t)x & kMrgP) + (uint32_t)(x >> 31);
   r = (r & kMrgP) + (r >> 31);
-  return (uint32_t)(r >= kMrgP ? r - kMrgP : r);
+  const uint32_t s = r - kMrgP;  // wraps to a large value where r < kMrgP
+  return r < s ? r : s;
+}
+// the same for any x (two folds bring it below 2^62)
+__host__ __device__ inline uint32_t mrg_reduce_any(uint64_t x) {
+  return mrg_reduce((x & kMrgP) + (x >> 31));
 }
 
 __host__ __device__ inline uint32_t mrg_next(MrgState& s) {
@@ -51,11 +57,12 @@ __host__ __device__ inline void mat5_apply(const Mat5& m, MrgState& s) {
   uint32_t o[5];
 #pragma unroll
   for (int i = 0; i < 5; ++i) {
+    // four products of 31-bit factors fit 64 bits
     uint64_t acc = 0;
 #pragma unroll
-    for (int k = 0; k < 5; ++k)
-      acc += mrg_reduce((uint64_t)m.a[i * 5 + k] * s.z[k]);
-    o[i] = mrg_reduce(acc);
+    for (int k = 0; k < 4; ++k) acc += (uint64_t)m.a[i * 5 + k] * s.z[k];
+    acc = (acc & kMrgP) + (acc >> 31);
+    o[i] = mrg_reduce_any(acc + (uint64_t)m.a[i * 5 + 4] * s.z[4]);
   }
 #pragma unroll
   for (int i = 0; i < 5; ++i) s.z[i] = o[i];
