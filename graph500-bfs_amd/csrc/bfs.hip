@@ -1396,6 +1396,269 @@ __global__ __launch_bounds__(kT) void k_levels(const int64_t* __restrict__ pred,
   if (i < n) out[i] = (uint16_t)((uint64_t)pred[i] >> 48);
 }
 
+// ---- a whole run in one block
+//
+// On a graph this small a run is a chain of ~20 launches that each keep a few
+// waves busy for a few microseconds.  One block of 16 waves with the bitmaps,
+// queues, parents and levels in LDS runs all its levels with barriers between
+// them and writes pred by original ID at the end.  It takes the same
+// directions (decide_next) and leaves the host a record per step; a run of
+// more than kSmallSteps steps leaves none and the level loop runs instead.
+// A run at SCALE 10 / 12 / 13 / 14: 150 / 186 / 201 / 201 us as a level loop, 38 / 46 /
+// 58 / 72 here (SCALE 15: 157 in the loop, past the LDS of one block).
+constexpr int kSmallT = 1024;
+constexpr int kSmallVerts = 16384;
+constexpr int64_t kSmallEdges = 1 << 19;
+constexpr int kSmallSteps = 63;
+constexpr int kSmallIlp = 4;
+constexpr uint32_t kSmallRow = 16;  // longer row rests are scanned by a wave
+
+struct SmallGraph {
+  const uint32_t* o2n;
+  const int64_t* row_off;
+  const uint32_t* col;
+  const uint2* first;
+  const uint32_t* n2o;
+  const uint32_t* deg_new;
+  int n_c;
+};
+
+__global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t root, LoopInit li,
+                                                      HostReport* __restrict__ rep,
+                                                      int64_t* __restrict__ pred) {
+  __shared__ uint32_t vis[kSmallVerts / 32], found[kSmallVerts / 32];
+  __shared__ uint16_t par[kSmallVerts], qa[kSmallVerts], qb[kSmallVerts];
+  __shared__ uint8_t lev[kSmallVerts];
+  __shared__ uint32_t es[kSmallT + 1], rs[kSmallT], wsum[kSmallT / kWave], fill;
+  __shared__ uint64_t red[2][kSmallT / kWave];
+  __shared__ LevelSync ls;
+  const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+  constexpr int kWords = kSmallVerts / 32;
+  uint16_t *q = qa, *nq = qb;
+  for (int i = t; i < kWords; i += kSmallT) {
+    const int valid = g.n_c - i * 32;
+    vis[i] = valid >= 32 ? 0u : valid <= 0 ? ~0u : ~0u << valid;
+  }
+  for (int i = t; i < kSmallVerts; i += kSmallT) lev[i] = 0xFF;
+  __syncthreads();
+  if (t == 0) {
+    const uint32_t r = g.o2n[root];
+    vis[r >> 5] |= 1u << (r & 31);
+    lev[r] = 0;
+    par[r] = (uint16_t)r;
+    q[0] = (uint16_t)r;
+    ls.step = li.first;
+    ls.growing = 1u;
+    ls.qlen = 1;
+    ls.qedges = g.row_off[r + 1] - g.row_off[r];
+    ls.prev_nq = 0;
+    ls.alpha_thr = li.alpha_thr;
+    ls.beta_thr = li.beta_thr;
+    ls.exec_thr = li.exec_thr;
+  }
+  __syncthreads();
+  // two block sums, valid in thread 0
+  auto sums = [&](uint64_t a, uint64_t b, uint64_t* sa, uint64_t* sb) {
+    a = wave_sum_u64(a);
+    b = wave_sum_u64(b);
+    if (lane == 0) {
+      red[0][wave] = a;
+      red[1][wave] = b;
+    }
+    __syncthreads();
+    *sa = *sb = 0;
+    if (t == 0)
+      for (int w = 0; w < kSmallT / kWave; ++w) {
+        *sa += red[0][w];
+        *sb += red[1][w];
+      }
+  };
+  // exclusive prefix sum over the block
+  auto scan = [&](uint32_t v, uint32_t* total) {
+    uint32_t x = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o, kWave);
+      if (lane >= o) x += y;
+    }
+    if (lane == kWave - 1) wsum[wave] = x;
+    __syncthreads();
+    uint32_t off = 0, all = 0;
+    for (int w = 0; w < kSmallT / kWave; ++w) {
+      off += w < wave ? wsum[w] : 0u;
+      all += wsum[w];
+    }
+    __syncthreads();
+    *total = all;
+    return x - v + off;
+  };
+  // the vertices of found, ascending, into dst; returns this thread's degree sum
+  auto to_queue = [&](uint16_t* dst, uint32_t* total) {
+    uint32_t bits = t < kWords ? found[t] : 0u;
+    uint32_t pos = scan((uint32_t)__popc(bits), total);
+    uint64_t edges = 0;
+    for (; bits; bits &= bits - 1) {
+      const uint32_t v = (uint32_t)t * 32 + (uint32_t)__ffs((int)bits) - 1;
+      dst[pos++] = (uint16_t)v;
+      edges += g.deg_new[v];
+    }
+    return edges;
+  };
+  int step = 0;
+  for (;; ++step) {
+    const uint32_t code = ls.step;
+    const uint32_t mode = step_mode(code);
+    const int level = step_level(code);
+    if (mode == kModeDone || step == kSmallSteps) break;
+    uint64_t count = 0, edges = 0;  // this thread's share
+    if (mode == kModeTD || mode == kModeTDS) {
+      const int qlen = (int)ls.qlen;
+      if (t == 0) fill = 0;
+      for (int w0 = 0; w0 < qlen; w0 += kSmallT) {
+        const int nwin = min(qlen - w0, kSmallT);
+        const uint32_t v = t < nwin ? q[w0 + t] : 0u;
+        const int64_t beg = t < nwin ? g.row_off[v] : 0;
+        const uint32_t len = t < nwin ? (uint32_t)(g.row_off[v + 1] - beg) : 0u;
+        uint32_t all;
+        es[t] = scan(len, &all);
+        rs[t] = (uint32_t)beg;
+        __syncthreads();
+        for (uint32_t e0 = (uint32_t)t; e0 < all; e0 += kSmallT * kSmallIlp) {
+          uint32_t own[kSmallIlp], u[kSmallIlp];
+#pragma unroll
+          for (int j = 0; j < kSmallIlp; ++j) {
+            const uint32_t e = e0 + (uint32_t)j * kSmallT;
+            int lo = 0, hi = nwin;
+            while (hi - lo > 1) {
+              const int mid = (lo + hi) >> 1;
+              if (es[mid] <= e) lo = mid;
+              else hi = mid;
+            }
+            own[j] = (uint32_t)lo;
+            u[j] = e < all ? g.col[rs[lo] + (e - es[lo])] : 0xFFFFFFFFu;
+          }
+#pragma unroll
+          for (int j = 0; j < kSmallIlp; ++j) {
+            if (u[j] == 0xFFFFFFFFu) continue;
+            const uint32_t bit = 1u << (u[j] & 31);
+            if ((vis[u[j] >> 5] & bit) || (atomicOr(&vis[u[j] >> 5], bit) & bit)) continue;
+            par[u[j]] = q[w0 + own[j]];
+            lev[u[j]] = (uint8_t)level;
+            nq[atomicAdd(&fill, 1u)] = (uint16_t)u[j];
+            edges += g.deg_new[u[j]];
+            ++count;
+          }
+        }
+        __syncthreads();
+      }
+    } else if (mode != kModeConv) {
+      for (int i = t; i < kWords; i += kSmallT) found[i] = 0;
+      if (t == 0) fill = 0;
+      __syncthreads();
+      auto take = [&](uint32_t v, uint32_t parent) {
+        par[v] = (uint16_t)parent;
+        lev[v] = (uint8_t)level;
+        atomicOr(&found[v >> 5], 1u << (v & 31));
+        ++count;
+      };
+      auto visited = [&](uint32_t u) { return (vis[u >> 5] >> (u & 31)) & 1u; };
+      for (int v0 = t; v0 < g.n_c; v0 += kSmallT * kSmallIlp) {
+        uint2 f[kSmallIlp];
+        bool open[kSmallIlp];
+#pragma unroll
+        for (int j = 0; j < kSmallIlp; ++j) {
+          const int v = v0 + j * kSmallT;
+          open[j] = v < g.n_c && !visited((uint32_t)v);
+          f[j] = open[j] ? g.first[v] : make_uint2(0u, 0u);
+        }
+#pragma unroll
+        for (int j = 0; j < kSmallIlp; ++j) {
+          if (!open[j]) continue;
+          const uint32_t v = (uint32_t)(v0 + j * kSmallT);
+          if (visited(f[j].x)) {
+            take(v, f[j].x);
+            continue;
+          }
+          const int64_t end = g.row_off[v + 1];
+          int64_t k = g.row_off[v] + 1;
+          if (end - k > (int64_t)kSmallRow) {
+            nq[atomicAdd(&fill, 1u)] = (uint16_t)v;  // no level queue is in use
+            continue;
+          }
+          while (k < end) {
+            uint32_t u[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[i] = k + i < end ? g.col[k + i] : f[j].x;
+            int hit = 4;
+#pragma unroll
+            for (int i = 3; i >= 0; --i) hit = visited(u[i]) ? i : hit;
+            if (hit < 4) {
+              take(v, hit == 0 ? u[0] : hit == 1 ? u[1] : hit == 2 ? u[2] : u[3]);
+              break;
+            }
+            k += 4;
+          }
+        }
+      }
+      __syncthreads();
+      const int rows = (int)fill;
+      for (int i = wave; i < rows; i += kSmallT / kWave) {
+        const uint32_t v = nq[i];
+        const int64_t end = g.row_off[v + 1];
+        for (int64_t k = g.row_off[v] + 1; k < end; k += kWave) {
+          const uint32_t u = k + lane < end ? g.col[k + lane] : 0u;
+          const uint64_t hits = __ballot(k + lane < end && visited(u));
+          if (!hits) continue;
+          const int at = __ffsll((long long)hits) - 1;
+          if (lane == at) take(v, u);
+          break;
+        }
+      }
+      __syncthreads();
+      for (int i = t; i < kWords; i += kSmallT) vis[i] |= found[i];
+    }
+    if (mode == kModeConv || mode == kModeTDX) {
+      __syncthreads();
+      uint32_t total;
+      uint16_t* dst = mode == kModeConv ? q : nq;
+      edges = to_queue(dst, &total);
+      count = t == 0 ? total : 0;
+    }
+    uint64_t sc, se;
+    sums(count, edges, &sc, &se);
+    if (t == 0) {
+      const LevelSync cur = ls;
+      uint32_t next;
+      if (mode == kModeConv) {
+        ls.qlen = (long long)sc;
+        ls.qedges = (long long)se;
+        next = step_code(level, td_step_mode((long long)sc, (long long)se, cur.exec_thr));
+        ls.step = next;
+      } else {
+        next = decide_next(cur, &ls, code, (long long)sc, (long long)se);
+      }
+      HostReport* r = rep + 1 + step;
+      r->w[0] = sc;
+      r->w[1] = se;
+      r->w[2] = next;
+      r->w[3] = code;
+    }
+    __syncthreads();
+    if (mode == kModeTD || mode == kModeTDS || mode == kModeTDX) {
+      uint16_t* x = q;
+      q = nq;
+      nq = x;
+    }
+  }
+  const bool done = step_mode(ls.step) == kModeDone;
+  if (t == 0) rep[0].w[0] = done ? (unsigned long long)step : ~0ull;
+  if (!done) return;
+  for (int v = t; v < g.n_c; v += kSmallT)
+    pred[g.n2o[v]] = lev[v] == 0xFF
+                         ? (int64_t)-1
+                         : (int64_t)(((uint64_t)lev[v] << 48) | (uint64_t)g.n2o[par[v]]);
+}
+
 unsigned grid_for(int64_t work_items, int64_t per_block) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ceil_div(work_items, per_block)));
 }
@@ -1449,9 +1712,11 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   b->wacc.alloc((size_t)b->bu_grid[0] + b->bu_grid[2] + b->bu_grid[1]);
   b->lsync.alloc(1);
   G500_CHECK_HIP(hipMemset(b->lsync.get(), 0, sizeof(LevelSync)));
-  G500_CHECK_HIP(hipHostMalloc((void**)&b->h_report, kReportSlots * sizeof(HostReport),
+  // the level loop's ring, then the one-block run's header and steps
+  constexpr size_t kReports = kReportSlots + 1 + kSmallSteps;
+  G500_CHECK_HIP(hipHostMalloc((void**)&b->h_report, kReports * sizeof(HostReport),
                                hipHostMallocMapped | hipHostMallocCoherent));
-  std::memset((void*)b->h_report, 0, kReportSlots * sizeof(HostReport));
+  std::memset((void*)b->h_report, 0, kReports * sizeof(HostReport));
   G500_CHECK_HIP(hipHostGetDevicePointer((void**)&b->d_report, b->h_report, 0));
   // ev_begin only times the run; ev_end also tells the host the run is done
   G500_CHECK_HIP(hipEventCreateWithFlags(&b->ev_begin, hipEventDisableSystemFence));
@@ -1934,6 +2199,87 @@ void speculate(g500_bfs* b, std::deque<Step>& pend, const HostLoop& hl, size_t d
 
 }  // namespace
 
+namespace {
+
+// Writes pred entries from the host, behind the stream's kernels.
+void write_path(g500_bfs* b, const std::vector<std::pair<uint32_t, int64_t>>& path) {
+  for (size_t i = 0; i < path.size(); i += kMaxPathArgs) {
+    PathArgs pa;
+    pa.count = (int)std::min<size_t>(kMaxPathArgs, path.size() - i);
+    for (int j = 0; j < pa.count; ++j) {
+      pa.v[j] = path[i + j].first;
+      pa.e[j] = path[i + j].second;
+    }
+    hipLaunchKernelGGL(k_write_path, dim3(1), dim3(kMaxPathArgs), 0, b->stream, pa,
+                       b->pred.get());
+    G500_CHECK_LAUNCH();
+  }
+}
+
+// The run in one block (k_bfs_small) where the graph fits it; false, with
+// nothing of the result written, where it does not or the run takes too many
+// steps.  Runs that time or count their levels, and engines told to guess
+// otherwise than by default, take the level loop.
+bool run_small(g500_bfs* b, int64_t root, const LoopInit& li, HostLoop& hl, int64_t* at) {
+  g500_graph* g = b->g;
+  if (b->n_core == 0 || g->n_c > kSmallVerts || g->m > kSmallEdges || li.qlen != 1 || b->timing ||
+      b->counting || b->guess_wrong || b->spec_depth != 1)
+    return false;
+  hipStream_t s = b->stream;
+  const SmallGraph sg{g->orig2new.get(), g->row_off.get(), g->col.get(), g->first.get(),
+                      g->new2orig.get(), g->deg_new.get(), (int)g->n_c};
+  G500_CHECK_HIP(hipEventRecord(b->ev_begin, s));
+  hipLaunchKernelGGL(k_bfs_small, dim3(1), dim3(kSmallT), 0, s, sg, root, li,
+                     b->d_report + kReportSlots, b->pred.get());
+  G500_CHECK_LAUNCH();
+  if (b->iso_root >= 0) {  // the last run's root without edges
+    write_path(b, {{(uint32_t)b->iso_root, -1}});
+    b->iso_root = -1;
+  }
+  G500_CHECK_HIP(hipEventRecord(b->ev_end, s));
+  G500_CHECK_HIP(hipEventSynchronize(b->ev_end));
+  const HostReport* rep = b->h_report + kReportSlots;
+  const unsigned long long steps = rep[0].w[0];
+  if (steps > (unsigned long long)kSmallSteps) return false;
+  uint32_t next = li.first;
+  for (unsigned long long i = 0; i < steps; ++i) {
+    const HostReport& r = rep[1 + i];
+    const uint32_t code = (uint32_t)r.w[3], mode = step_mode(code);
+    const int64_t nq_size = (int64_t)r.w[0], nq_edges = (int64_t)r.w[1];
+    if (code != next) fail(G500_ERR_STATE, "step %u ran where %u was next", code, next);
+    if (mode == kModeConv) {
+      next = step_code(step_level(code), td_step_mode(nq_size, nq_edges, hl.exec_thr));
+    } else {
+      const bool td = mode_is_td(mode);
+      at[G500_AT_LEVEL] = step_level(code);
+      g500_level_trace tr{};
+      tr.level = step_level(code);
+      tr.top_down = td ? 1 : 0;
+      tr.nq_size = nq_size;
+      tr.nq_edges = td ? nq_edges : 0;
+      tr.exec_bottom_up = (mode == kModeTD || mode == kModeTDS) ? 0 : 1;
+      b->trace.push_back(tr);
+      next = hl.after_level(code, nq_size, td ? nq_edges : 0, at);
+    }
+    if ((uint32_t)r.w[2] != next)
+      fail(G500_ERR_STATE, "level %d: the device chose step %u:%u, the reference rule %u:%u",
+           step_level(code), step_level((uint32_t)r.w[2]), step_mode((uint32_t)r.w[2]),
+           step_level(next), step_mode(next));
+  }
+  float ms = 0;
+  G500_CHECK_HIP(hipEventElapsedTime(&ms, b->ev_begin, b->ev_end));
+  b->stats.gpu_ms = ms;
+  b->stats.nlevels = (int)b->trace.size();
+  b->unreach = std::max<int64_t>(0, g->n_c - hl.visited);
+  for (const auto& tr : b->trace)
+    if (tr.top_down) b->stats.td_edges += tr.nq_edges;
+  b->have_result = true;
+  b->last_root = root;
+  return true;
+}
+
+}  // namespace
+
 void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
              double beta, int64_t* at) {
   g500_graph* g = b->g;
@@ -2024,6 +2370,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   hl.unreach = b->unreach;
   const uint32_t first = step_code(root_level + 1, kModeTDS);
   LoopInit li{first, root_in ? 1 : 0, 0, hl.alpha_thr, hl.beta_thr, hl.exec_thr};
+  if (run_small(b, root, li, hl, at)) return;
   G500_CHECK_HIP(hipEventRecord(b->ev_begin, s));
   hipLaunchKernelGGL(k_bfs_init, dim3(grid_for(words, kT)), dim3(kT), 0, s,
                      b->vis.get(), words, n_c, root_in ? bfs_root : (int64_t)-1,
@@ -2174,16 +2521,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
       b->iso_root = root;
     }
   }
-  for (size_t i = 0; i < path.size(); i += kMaxPathArgs) {
-    PathArgs pa;
-    pa.count = (int)std::min<size_t>(kMaxPathArgs, path.size() - i);
-    for (int j = 0; j < pa.count; ++j) {
-      pa.v[j] = path[i + j].first;
-      pa.e[j] = path[i + j].second;
-    }
-    hipLaunchKernelGGL(k_write_path, dim3(1), dim3(kMaxPathArgs), 0, s, pa, b->pred.get());
-    G500_CHECK_LAUNCH();
-  }
+  write_path(b, path);
   G500_CHECK_HIP(hipEventRecord(b->ev_end, s));
   G500_CHECK_HIP(hipEventSynchronize(b->ev_end));
   float ms = 0;
@@ -2253,14 +2591,17 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
 
 void bfs_levels(g500_bfs* b, uint16_t* out) {
   g500_graph* g = b->g;
-  DevBuf<uint16_t> lv;
-  lv.alloc_raw((size_t)g->n);
+  // kept: allocating and freeing a few KB took longer than everything else
+  // here (large ones come from the kept blocks either way)
+  DevBuf<uint16_t>& lv = b->lv;
+  if (!lv.get()) lv.alloc_raw((size_t)g->n);
   hipLaunchKernelGGL(k_levels, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, b->stream,
                      b->pred.get(), g->n, lv.get());
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipMemcpyAsync(out, lv.get(), g->n * sizeof(uint16_t),
                                 hipMemcpyDeviceToHost, b->stream));
   G500_CHECK_HIP(hipStreamSynchronize(b->stream));
+  if (g->n > kSmallVerts * 4) lv.release();
 }
 
 }  // namespace g500

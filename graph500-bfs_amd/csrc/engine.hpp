@@ -90,6 +90,8 @@ struct g500_bfs {
   bool guess_wrong = false;
   int64_t unreach = 0;  // vertices with edges the last run left unreached
 
+  g500::DevBuf<uint16_t> lv;  // levels by original ID (small graphs keep it)
+
   // validation scratch
   g500::DevBuf<unsigned long long> vcount;  // error and edge counts (validate.hip)
   g500::DevBuf<uint8_t> vcode;              // depth and parent bits per vertex, by slices
