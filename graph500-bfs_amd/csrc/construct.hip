@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kT) void k_edge_bits(const uint32_t* __restrict__ o
 int bitlen(uint64_t x) { return x ? 64 - __builtin_clzll(x) : 0; }
 
 // The general form: any list, the symmetric (new_src, new_dst) keys radix
-// sorted and then deduplicated (80 ms at SCALE 24, where the buckets take 24).
+// sorted and then deduplicated (80 ms at SCALE 24, where the buckets take 22).
 void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   hipStream_t s = g->stream;
   const int lg = g->log_n;

@@ -20,9 +20,9 @@
 // repeated edges, say) buckets come out larger than LDS: up to kBigCap keys
 // one block sorts them range by range, beyond that (or with a group of buckets
 // past its room) the caller sorts with the radix sort.  At SCALE 24 the
-// 2^29 keys take 24 ms (radix sort and deduplication: 80): 9.4 for the first
-// pass, bound by its random reads of the new IDs, 1.8 + 3.2 for counting and
-// moving in the second, 8.3 for the LDS sort, bound by its ballots, 0.9 for the
+// 2^29 keys take 22 ms (radix sort and deduplication: 80): 10.5 for the first
+// pass, bound by its random reads of the new IDs, 1.3 + 2.7 for counting and
+// moving in the second, 6.8 for the LDS sort, bound by its ballots, 0.9 for the
 // last copy.
 #include <algorithm>
 
@@ -379,9 +379,12 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
 // --------------------------------------------------------------------- rows
 constexpr int kSortT = 512;
 constexpr int kSortWaves = kSortT / kWave;
-constexpr int kBucketCap = 8192;   // keys the LDS sort holds
-constexpr int kBucketMean = 4096;  // keys a bucket is laid out for
-constexpr int kSplitDegree = 1024; // rows up to this length stay in one bucket
+// Keys the LDS sort holds (40 KB: four blocks on a CU; with 8192 keys and two
+// blocks construction took 4-8 % longer at SCALE 18 to 24), keys a bucket is
+// laid out for, and the length up to which a row stays in one bucket.
+constexpr int kBucketCap = 4096;
+constexpr int kBucketMean = 3072;
+constexpr int kSplitDegree = 512;
 constexpr int kPartItems = 16;
 constexpr int kPartTile = kSortT * kPartItems;  // keys partitioned at a time
 constexpr int kMaxParts = 2048;                 // buckets of one partition pass
@@ -976,10 +979,10 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   if (keys <= 0 || n_c <= 0) return false;
   const int64_t buckets = ceil_div(keys, kBucketMean);
   // one pass up to kMaxParts buckets; above that groups of `step` buckets
-  // first, about as many groups as buckets in each
+  // first, one to four times as many groups as buckets in each
   int64_t step = 1;
   if (buckets > kMaxParts)
-    while (step * step < buckets) step *= 2;
+    while (4 * step * step <= buckets) step *= 2;
   const int64_t groups = ceil_div(buckets, step);
   if (groups > kMaxParts || step > kMaxParts || lg > 31) return false;
   const bool two = step > 1;

@@ -72,10 +72,12 @@ def _skewed(vertices, edges, seed):
     return rng.permutation(vertices)[v % vertices]
 
 
-# keys are laid out 4096 a bucket (2048 edges), one partition pass up to 2048
-# buckets (2^23 keys), two beyond; tiles of 8192 keys
+# keys are laid out 3072 a bucket (1536 edges) and sorted up to 4096 a time,
+# one partition pass up to 2048 buckets (3145728 edges), two beyond; tiles of
+# 8192 keys
 @pytest.mark.parametrize("vertices,edges", [
-    (2, 1), (5, 3), (100, 2047), (100, 2048), (100, 2049), (3000, 4096), (3000, 4097),
+    (2, 1), (5, 3), (100, 1535), (100, 1536), (100, 1537), (100, 2047), (100, 2048), (100, 2049),
+    (3000, 4096), (3000, 4097), (200003, 3145727), (200003, 3145731),
     (70001, 300007),          # two ID ranges of 2^16
     (1048577, 1100001),       # IDs past 2^20: endpoints partitioned before they are counted
     (300007, 4194305),        # one key pair more than one pass holds
@@ -83,8 +85,6 @@ def _skewed(vertices, edges, seed):
 @pytest.mark.parametrize("symmetric", [False, True])
 def test_rows_of_skewed_lists(G, vertices, edges, symmetric):
     print(f"\n[build] {vertices} vertices {edges} edges symmetric={symmetric}", flush=True)
-    if symmetric and edges > 3000000:
-        pytest.skip("the sizes below cover it")
     v0, v1 = _skewed(vertices, edges, edges)
     _same_csr(G, v0, v1, symmetric_input=symmetric)
 
