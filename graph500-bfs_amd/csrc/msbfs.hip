@@ -114,6 +114,7 @@ __global__ __launch_bounds__(kT) void k_ms_init(const int64_t* __restrict__ d_ro
   for (int64_t j = i0; j < ncnt; j += stride) {
     cnt[j] = 0;
     fe[j] = 0;
+    fe[ncnt + j] = 0;
   }
   for (int64_t j = i0; j < (int64_t)ncnt * 4; j += stride) act[j] = 0;
   for (int64_t j = i0; j < G500_MSBFS_MAX_ROOTS; j += stride) te[j] = 0;
@@ -177,10 +178,13 @@ struct MsLevel {
   uint64_t* fbn;        // bitmap of F_{L+1}
   unsigned long long* cnt;
   unsigned long long* fe;
+  unsigned long long* feh;  // degree sums of the frontier's heavy vertices
   const uint64_t* act_l;   // lanes present anywhere in F_L (4 words)
   uint64_t* act_n;         // the same for F_{L+1}, ORed by the kernels that write it
   unsigned long long thr;
   unsigned long long mark_thr;
+  unsigned long long hub_thr;
+  int64_t hubs;            // vertices below this are the heavy ones
   const int64_t* d_roots;  // [0] = batch size
   double stream_frac;
   int64_t n_c;
@@ -197,6 +201,17 @@ struct MsLevel {
 
 // top-down levels over at least m / kMarkShare frontier edges push without marks
 constexpr int64_t kMarkShare = 64;
+// Top-down levels up to kHubLevels may pull from the hubs (ms_hub_pull): when
+// the frontier's share of the hubs' edges times the lane words passes
+// kHubShare.  Pulling reads all those edges whatever the frontier, a push costs
+// an atomic per edge and lane word.  Level by push and by pull, in ms: share
+// times words 2.0 (SCALE 24, 200 roots) 2.49 / 0.62, 0.36 (SCALE 26, 128) 1.47 /
+// 2.90; whole batches break even at about 0.4.
+constexpr int kHubLevels = 2;
+constexpr double kHubShare = 0.45;
+// From this many lane words on, a split level pulls from the hubs too: with
+// two to four words batches got 1-5 % faster, with one 4 % slower (SCALE 25, 26).
+constexpr int kSplitHubWords = 2;
 
 enum { kModeTopDown = 0, kModeStream = 1, kModePull = 2, kModeSplit = 3 };
 // rows of per-lane degree sums for a split level: block b of a top-down
@@ -228,6 +243,13 @@ __device__ inline bool ms_top_down(const MsLevel& a, int l) { return a.fe[l] < a
 // at SCALE 20 with 64 roots, 2.07 -> 1.47 at SCALE 26 with 128).  The light
 // levels keep the marks: reading all of F_{L+1} costs 0.05-0.1 ms.
 __device__ inline bool ms_marks(const MsLevel& a) { return a.fe[a.L] < a.mark_thr; }
+// A heavy top-down level whose frontier holds most of the hubs is not pushed
+// along the hubs' rows: every vertex pulls its hub neighbours instead, the
+// first entries of its row (IDs are degree-descending): no atomics, and the
+// hubs' lane words stay cached.
+__device__ inline bool ms_hub_pull(const MsLevel& a) {
+  return a.feh[a.L] >= a.hub_thr && !ms_marks(a) && ms_top_down(a, a.L);
+}
 // top-down while the frontier is light; else a streaming pull while few
 // (root, vertex) pairs are reached yet, then a per-vertex pull -- split at
 // the first bottom-up level after top-down ones (light roots push)
@@ -431,6 +453,8 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModeTopDown && mode != kModeSplit) return;
+  // a split level's pulls take the hubs' lanes, k_ms_hub_pull a heavy level's
+  if (mode == kModeSplit ? K >= kSplitHubWords : ms_hub_pull(a)) return;
   const bool split = mode == kModeSplit, mark = ms_marks(a);
   uint64_t pm[K];
   if (!push_lanes<K>(a, split, pm)) return;
@@ -480,7 +504,7 @@ __global__ __launch_bounds__(kT) void k_ms_td_count(MsLevel a) {
     if (threadIdx.x < K) lall[threadIdx.x] = 0;
     __syncthreads();
   }
-  uint64_t disc = 0, edges = 0, lanes[K];
+  uint64_t disc = 0, edges = 0, hub_edges = 0, lanes[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) lanes[k] = 0;
   const bool marked = ms_marks(a);
@@ -510,6 +534,7 @@ __global__ __launch_bounds__(kT) void k_ms_td_count(MsLevel a) {
       if (split) lane_add(lfe + 64 * k, lall + k, x[k], d);
     }
     edges += d;
+    if (v < a.hubs) hub_edges += d;
   }
   if (split) {
     __syncthreads();
@@ -521,6 +546,117 @@ __global__ __launch_bounds__(kT) void k_ms_td_count(MsLevel a) {
   }
   ms_note_lanes<K>(a, lanes);
   ms_flush(a, red, disc, edges);
+  __syncthreads();
+  hub_edges = block_sum(hub_edges, red);
+  if (threadIdx.x == 0 && hub_edges) atomicAdd(&a.feh[a.L + 1], (unsigned long long)hub_edges);
+}
+
+// Hub pull of a heavy top-down level: vertex v ORs the lane words of its
+// neighbours among the first a.hubs vertices, masked with seen, into the
+// cleared F_{L+1}[v] (the pushes of the other frontier vertices follow).
+// G lanes per vertex over new IDs [vb, ve); the words of the hubs stay in the
+// L2, and a word outside the frontier is zero.
+template <int K, int G, int U>
+__global__ __launch_bounds__(kT) void k_ms_hub_pull(MsLevel a, int64_t vb, int64_t ve) {
+  if (!ms_active(a) || !ms_hub_pull(a)) return;
+  const int lig = threadIdx.x % G;
+  const int64_t gid = ((int64_t)blockIdx.x * kT + threadIdx.x) / G;
+  const int64_t ngroups = (int64_t)gridDim.x * (kT / G);
+  const uint32_t hubs = (uint32_t)a.hubs;
+  for (int64_t v = vb + gid; v < ve; v += ngroups) {
+    const int64_t beg = a.row_off[v], end = a.row_off[v + 1];
+    uint64_t acc[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = 0;
+    for (int64_t base = beg; base < end; base += (int64_t)G * U) {
+      uint32_t u[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const int64_t e = base + (int64_t)j * G + lig;
+        u[j] = e < end ? ld_col(a.col + e) : 0xFFFFFFFFu;
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j)
+        if (u[j] < hubs) {
+          uint64_t x[K];
+          load_lanes<K>(a.fl + (int64_t)u[j] * K, x);
+#pragma unroll
+          for (int k = 0; k < K; ++k) acc[k] |= x[k];
+        }
+      // rows ascend: the last entry read ends the prefix
+      int past = u[U - 1] >= hubs ? 1 : 0;
+      if constexpr (G > 1) past = __shfl(past, (lane_id() / G) * G + G - 1, kWave);
+      if (past) break;
+    }
+    if constexpr (G > 1) {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) acc[k] |= __shfl_xor(acc[k], o, kWave);
+    }
+    if (lig == 0) {
+      bool any = false;
+#pragma unroll
+      for (int k = 0; k < K; ++k) any = any || acc[k] != 0;
+      if (any) {
+        uint64_t s[K];
+        load_lanes<K>(a.seen + v * K, s);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          if (acc[k] & ~s[k]) a.fn[v * K + k] = acc[k] & ~s[k];
+      }
+    }
+  }
+}
+
+// The heavy rows' hub pull, one wave per work item of `chunk` edges.
+template <int K>
+__global__ __launch_bounds__(kT) void k_ms_hub_pull_heavy(MsLevel a,
+                                                         const uint64_t* __restrict__ item_start,
+                                                         const uint32_t* __restrict__ item_vertex,
+                                                         int64_t n_items, int chunk) {
+  if (!ms_active(a) || !ms_hub_pull(a)) return;
+  const int lane = lane_id();
+  const int64_t wid = ((int64_t)blockIdx.x * kT + threadIdx.x) / kWave;
+  const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
+  const uint32_t hubs = (uint32_t)a.hubs;
+  constexpr int U = 4;
+  for (int64_t it = wid; it < n_items; it += nw) {
+    const int64_t v = item_vertex[it];
+    const int64_t beg = a.row_off[v] + (int64_t)(it - item_start[v]) * chunk;
+    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)chunk);
+    uint64_t acc[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] = 0;
+    for (int64_t base = beg; base < end; base += (int64_t)kWave * U) {
+      uint32_t u[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const int64_t e = base + (int64_t)j * kWave + lane;
+        u[j] = e < end ? ld_col(a.col + e) : 0xFFFFFFFFu;
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j)
+        if (u[j] < hubs) {
+          uint64_t x[K];
+          load_lanes<K>(a.fl + (int64_t)u[j] * K, x);
+#pragma unroll
+          for (int k = 0; k < K; ++k) acc[k] |= x[k];
+        }
+      if (__any(u[U - 1] >= hubs)) break;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) acc[k] |= __shfl_xor(acc[k], o, kWave);
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint64_t x = acc[k] & ~a.seen[v * K + k];
+        if (x) atomicOr((unsigned long long*)&a.fn[v * K + k], (unsigned long long)x);
+      }
+    }
+  }
 }
 
 // Streaming pull: the edge array is cut into tiles of kTile edges, one block
@@ -930,8 +1066,12 @@ __global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve)
   const int mode = ms_mode(a, a.L);
   if (mode != kModePull && mode != kModeSplit) return;
   // split level: the pushing lanes count as covered too, and the lanes the
-  // pushes (queued first) put into F_{L+1} join the lanes pulled
+  // pushes (queued first) put into F_{L+1} join the lanes pulled.  The hubs do
+  // not push: a vertex with a pushing lane missing pulls all its hub
+  // neighbours, the first entries of its row, before it may stop.
   const bool split = mode == kModeSplit;
+  const bool hubs_pulled = split && K >= kSplitHubWords;
+  const uint32_t hubs = hubs_pulled ? (uint32_t)a.hubs : 0u;
   const int lig = threadIdx.x % G;
   const int64_t gid0 = ((int64_t)blockIdx.x * kT + threadIdx.x) / G;
   const int64_t ngroups = (int64_t)gridDim.x * (kT / G);
@@ -964,13 +1104,14 @@ __global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve)
       load_lanes<K>(a.seen + v * K, s0);
       load_lanes<K>(a.fl + v * K, f);
       if (split) load_lanes<K>(a.fn + v * K, acc);
-      bool full = true;
+      bool full = true, hub = false;
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         s[k] = s0[k] | f[k];
         full = full && ((s[k] | inact[k]) == ~0ull);
+        hub = hub || (hubs_pulled && (a.split_mask[k] & ~s[k]) != 0);
       }
-      if (!full) {
+      if (!full || hub) {
         const int64_t beg = a.row_off[v], end = a.row_off[v + 1];
         for (int64_t base = beg; base < end; base += (int64_t)G * U) {
           uint32_t u[U];
@@ -997,7 +1138,13 @@ __global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve)
           bool cov = true;
 #pragma unroll
           for (int k = 0; k < K; ++k) cov = cov && ((acc[k] | s[k] | inact[k]) == ~0ull);
-          if (cov) break;
+          // rows ascend: the last entry of the round ends the hub prefix
+          int past = 1;
+          if (hub) {
+            past = u[U - 1] >= hubs ? 1 : 0;
+            if constexpr (G > 1) past = __shfl(past, (lane_id() / G) * G + G - 1, kWave);
+          }
+          if (cov && past) break;
         }
       }
 #pragma unroll
@@ -1064,13 +1211,15 @@ __global__ __launch_bounds__(kT) void k_ms_bu_heavy(MsLevel a,
     load_lanes<K>(a.seen + v * K, s);
     load_lanes<K>(a.fl + v * K, f);
     load_lanes<K>(gacc + v * K, g0);
-    bool full = true;
+    bool full = true, hub = false;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       s[k] |= f[k];
       full = full && ((s[k] | g0[k] | inact[k]) == ~0ull);
+      hub = hub || (K >= kSplitHubWords && mode == kModeSplit &&
+                    (a.split_mask[k] & ~(s[k] | g0[k])) != 0);
     }
-    if (full) continue;
+    if (full && !hub) continue;
     const int64_t beg = a.row_off[v] + (int64_t)(it - item_start[v]) * chunk;
     const int64_t end = min(a.row_off[v + 1], beg + (int64_t)chunk);
     uint64_t acc[K];
@@ -1099,7 +1248,7 @@ __global__ __launch_bounds__(kT) void k_ms_bu_heavy(MsLevel a,
       bool cov = true;
 #pragma unroll
       for (int k = 0; k < K; ++k) cov = cov && ((acc[k] | s[k] | g0[k] | inact[k]) == ~0ull);
-      if (cov) break;
+      if (cov && (!hub || __any(u[U - 1] >= (uint32_t)a.hubs))) break;
     }
     if (lane == 0) {
 #pragma unroll
@@ -1498,10 +1647,13 @@ MsLevel level_args(const g500_msbfs* b, int L) {
   a.fbn = b->fb[(L + 1) & 1].get();
   a.cnt = b->cnt.get();
   a.fe = b->fe.get();
+  a.feh = b->fe.get() + (kMaxLevels + 2);
   a.act_l = b->act.get() + (int64_t)L * 4;
   a.act_n = b->act.get() + (int64_t)(L + 1) * 4;
   a.thr = b->td_threshold;
   a.mark_thr = (unsigned long long)(g->m / kMarkShare);
+  a.hubs = b->bin_heavy;
+  a.hub_thr = ~0ull;  // set per lane-word count by level_kernels
   a.d_roots = b->roots.get();
   a.stream_frac = b->tuning.stream_frac;
   a.dense_algo = b->tuning.dense_algo;
@@ -1551,6 +1703,16 @@ void launch_hyb_push(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t 
   G500_CHECK_LAUNCH();
 }
 
+template <int K, int G>
+void launch_hub_pull(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t ve,
+                     hipStream_t s) {
+  if (ve <= vb) return;
+  constexpr int U = G == 1 ? 4 : 2;
+  hipLaunchKernelGGL((k_ms_hub_pull<K, G, U>), dim3(sweep_grid(b, ve - vb, G)), dim3(kT), 0, s, a,
+                     vb, ve);
+  G500_CHECK_LAUNCH();
+}
+
 template <int K>
 void level_kernels(const g500_msbfs* b, int L, hipStream_t s) {
   MsLevel a = level_args(b, L);
@@ -1561,6 +1723,9 @@ void level_kernels(const g500_msbfs* b, int L, hipStream_t s) {
   // for 64 and 128 roots, 50-100 for 256)
   if (K > 2) a.split_thr = (unsigned long long)((double)a.split_thr * 2.0 / K);
   const int64_t h = b->bin_heavy, m = b->bin_medium, n_c = b->g->n_c;
+  if (L <= kHubLevels)
+    a.hub_thr = std::max<unsigned long long>(
+        1, (unsigned long long)(kHubShare * (double)b->heavy_edges / K));
   const int chunk = b->tuning.heavy_chunk;
   const int64_t bw = bitmap_words(b);
   const unsigned pgrid = (unsigned)std::max<int64_t>(
@@ -1578,6 +1743,14 @@ void level_kernels(const g500_msbfs* b, int L, hipStream_t s) {
   const unsigned hgrid = (unsigned)std::max<int64_t>(
       1, std::min<int64_t>(ceil_div(b->n_items, kWavesPerBlock),
                            (int64_t)num_cus(b->g->device) * b->tuning.blocks_per_cu));
+  // hub pulls follow a top-down level (whose count pass takes the degree sums)
+  if (b->n_items > 0 && L > 0 && L <= kHubLevels) {
+    hipLaunchKernelGGL((k_ms_hub_pull_heavy<K>), dim3(hgrid), dim3(kT), 0, s, a,
+                       b->item_start.get(), b->item_vertex.get(), b->n_items, chunk);
+    G500_CHECK_LAUNCH();
+    launch_hub_pull<K, 16>(b, a, h, m, s);
+    launch_hub_pull<K, 1>(b, a, m, n_c, s);
+  }
   if (b->n_items > 0) {
     hipLaunchKernelGGL((k_ms_push_heavy<K>), dim3(hgrid), dim3(kT), 0, s, a,
                        b->item_start.get(), b->item_vertex.get(), b->n_items, chunk);
@@ -1797,6 +1970,8 @@ void update_bins(g500_msbfs* b) {
   b->bin_heavy = hm[0];
   b->bin_medium = std::max(hm[0], hm[1]);
   const int64_t h = b->bin_heavy;
+  G500_CHECK_HIP(hipMemcpy(&b->heavy_edges, g->row_off.get() + h, sizeof(int64_t),
+                           hipMemcpyDeviceToHost));
   b->item_start.alloc((size_t)h + 1);
   b->acc.alloc((size_t)std::max<int64_t>(1, h) * b->kmax);
   G500_CHECK_HIP(hipMemsetAsync(b->acc.get(), 0, b->acc.n * sizeof(uint64_t), s));
@@ -1918,7 +2093,7 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
   }
   b->fb[0].alloc((size_t)bitmap_words(b));
   b->fb[1].alloc((size_t)bitmap_words(b));
-  b->fe.alloc(kMaxLevels + 2);
+  b->fe.alloc(2 * (kMaxLevels + 2));  // of all the frontier, of its heavy vertices
   b->act.alloc((size_t)(kMaxLevels + 2) * 4);
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_roots, (G500_MSBFS_MAX_ROOTS + 1) * sizeof(int64_t),
                                hipHostMallocDefault));

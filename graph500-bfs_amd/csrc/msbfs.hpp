@@ -47,6 +47,7 @@ struct g500_msbfs {
 
   g500_msbfs_tuning tuning{};
   int64_t bin_heavy = 0, bin_medium = 0;    // new-ID bin ends for the tuning
+  int64_t heavy_edges = 0;  // CSR entries of the heavy bin's rows
   unsigned long long td_threshold = 0;      // top-down while frontier edges < this
   g500::DevBuf<uint64_t> item_start;        // heavy work items: prefix by vertex (h+1)
   g500::DevBuf<uint32_t> item_vertex;       // owner of each heavy work item
