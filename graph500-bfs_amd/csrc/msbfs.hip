@@ -193,7 +193,7 @@ struct MsLevel {
   int L;
   // split level: roots whose frontier degree sum is below split_thr push;
   // lane_part holds per-block degree sums per lane, split_mask the lanes
-  // that push (written by k_ms_lane_mask before the level's pulls)
+  // that push (written by k_ms_prep before the level's pulls)
   unsigned long long split_thr;  // 0: no split levels
   unsigned long long* lane_part;
   uint64_t* split_mask;
@@ -215,8 +215,9 @@ constexpr int kSplitHubWords = 2;
 
 enum { kModeTopDown = 0, kModeStream = 1, kModePull = 2, kModeSplit = 3 };
 // rows of per-lane degree sums for a split level: block b of a top-down
-// level's count pass adds its sums to row b % kLaneParts
-constexpr int kLaneParts = 512;
+// level's count pass adds its sums to row b % kLaneParts (512 rows took one
+// block 0.2 ms to add up with four lane words)
+constexpr int kLaneParts = 64;
 
 // Adds degree d to the LDS counter of every lane set in x.  A word with more
 // lanes set than clear adds d to the all-lanes counter and subtracts it from
@@ -230,6 +231,17 @@ __device__ inline void lane_add(unsigned long long* lfe, unsigned long long* lal
     for (uint64_t b = x; b; b &= b - 1) atomicAdd(&lfe[__ffsll((long long)b) - 1], d);
   }
 }
+// The degree bins of a level's sweeps and the blocks each one gets.
+struct MsBins {
+  const uint64_t* item_start;
+  const uint32_t* item_vertex;
+  uint64_t* acc;           // the heavy pulls' accumulators
+  int64_t n_items;
+  int64_t medium_end;      // medium rows: [a.hubs, medium_end)
+  int chunk;
+  unsigned heavy, medium, light;
+};
+
 enum { kDenseStream = 1, kDenseHybrid = 2 };
 
 __device__ inline bool ms_active(const MsLevel& a) { return a.cnt[a.L] != 0; }
@@ -291,6 +303,55 @@ __device__ inline void ms_note_lanes(const MsLevel& a, uint64_t (&lanes)[K]) {
   }
 }
 
+// Split level.  A root whose level-L frontier is light (its degree sum below
+// split_thr) would keep almost every vertex's pull scanning its whole row:
+// few vertices have a neighbour in that frontier, and a pull stops only
+// when every lane it lacks is covered.  Those roots push instead, along the
+// rows of their frontier vertices, and the pulls stop once the other lanes
+// are covered.
+//
+// Per-lane degree sums of F_L come from the count pass of the top-down level
+// that produced it (k_ms_td_count).
+//
+// One block: sums the lane_part rows per lane (each wave a quarter of the
+// rows, 16 loads in flight per lane) and sets split_mask to the lanes
+// present in F_L whose frontier degree sum is below split_thr.
+template <int K>
+__device__ inline void lane_mask(const MsLevel& a, int parts) {
+  __shared__ unsigned long long mk[4];
+  __shared__ unsigned long long ws[kWavesPerBlock][64 * K];
+  const int t = threadIdx.x, wave = t / kWave, lane = lane_id();
+  if (t < 4) mk[t] = 0;
+  const int per = (parts + kWavesPerBlock - 1) / kWavesPerBlock;
+  const int p0 = wave * per, p1 = min(parts, p0 + per);
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int lanei = 64 * k + lane;
+    unsigned long long acc[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = 0;
+    for (int p = p0; p < p1; p += 16) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (p + j < p1) acc[j] += a.lane_part[(int64_t)(p + j) * 256 + lanei];
+    }
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) sum += acc[j];
+    ws[wave][lanei] = sum;
+  }
+  __syncthreads();
+  if (t < 64 * K) {
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) sum += ws[w][t];
+    const bool present = (a.act_l[t >> 6] >> (t & 63)) & 1ull;
+    if (present && sum < a.split_thr) atomicOr(&mk[t >> 6], 1ull << (t & 63));
+  }
+  __syncthreads();
+  if (t < 4) a.split_mask[t] = mk[t];
+}
+
 // Level preparation: clear the next bitmap; unless the level only pulls,
 // clear F_{L+1} (pushes fill it by atomicOr; a pulling level stores every
 // vertex's word); when F_L came from a top-down level and this level pushes
@@ -302,6 +363,7 @@ template <int K>
 __global__ __launch_bounds__(kT) void k_ms_prep(MsLevel a, int64_t bm_words) {
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
+  if (mode == kModeSplit && blockIdx.x == gridDim.x - 1) lane_mask<K>(a, kLaneParts);
   const bool clear = mode != kModePull;
   const bool fold = a.L > 0 && ms_top_down(a, a.L - 1) && mode == kModeTopDown;
   const int64_t i0 = (int64_t)blockIdx.x * kT + threadIdx.x;
@@ -410,7 +472,8 @@ __device__ inline bool push_lanes(const MsLevel& a, bool split, uint64_t (&pm)[K
 }
 
 template <int K, int G>
-__global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, int64_t vb, int64_t ve) {
+__device__ inline void push_rows(const MsLevel& a, int64_t vb, int64_t ve, int64_t rank,
+                                 int64_t nblk) {
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModeTopDown && mode != kModeSplit) return;
@@ -418,8 +481,8 @@ __global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, int64_t vb, int64_t v
   uint64_t pm[K];
   if (!push_lanes<K>(a, split, pm)) return;
   const int lig = threadIdx.x % G;
-  const int64_t gid = ((int64_t)blockIdx.x * kT + threadIdx.x) / G;
-  const int64_t ngroups = (int64_t)gridDim.x * (kT / G);
+  const int64_t gid = (rank * kT + threadIdx.x) / G;
+  const int64_t ngroups = nblk * (kT / G);
   for (int64_t v = vb + gid; v < ve; v += ngroups) {
     if (!in_bitmap(a.fb, v)) continue;
     uint64_t f[K];
@@ -446,10 +509,7 @@ __global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, int64_t vb, int64_t v
 
 // The same for heavy vertices: one wave per work item of `chunk` edges.
 template <int K>
-__global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
-                                                     const uint64_t* __restrict__ item_start,
-                                                     const uint32_t* __restrict__ item_vertex,
-                                                     int64_t n_items, int chunk) {
+__device__ inline void push_items(const MsLevel& a, const MsBins& n, int64_t rank, int64_t nblk) {
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModeTopDown && mode != kModeSplit) return;
@@ -459,10 +519,10 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
   uint64_t pm[K];
   if (!push_lanes<K>(a, split, pm)) return;
   const int lane = lane_id();
-  const int64_t wid = ((int64_t)blockIdx.x * kT + threadIdx.x) / kWave;
-  const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
-  for (int64_t it = wid; it < n_items; it += nw) {
-    const int64_t v = item_vertex[it];
+  const int64_t wid = (rank * kT + threadIdx.x) / kWave;
+  const int64_t nw = nblk * kWavesPerBlock;
+  for (int64_t it = wid; it < n.n_items; it += nw) {
+    const int64_t v = n.item_vertex[it];
     if (!in_bitmap(a.fb, v)) continue;
     uint64_t f[K];
     load_lanes<K>(a.fl + v * K, f);
@@ -473,8 +533,8 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
       any = any || f[k] != 0;
     }
     if (!any) continue;
-    const int64_t beg = a.row_off[v] + (int64_t)(it - item_start[v]) * chunk;
-    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)chunk);
+    const int64_t beg = a.row_off[v] + (int64_t)(it - n.item_start[v]) * n.chunk;
+    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)n.chunk);
     for (int64_t e0 = beg + lane; e0 < end; e0 += (int64_t)kWave * kPushIlp) {
       uint32_t w[kPushIlp];
       bool ok[kPushIlp];
@@ -485,6 +545,22 @@ __global__ __launch_bounds__(kT) void k_ms_push_heavy(MsLevel a,
         ms_push_n<K>(a, mark, w, ok, f);
     }
   }
+}
+
+// The pushes of a level, every bin in one launch: blocks [0, n.heavy) take the
+// heavy rows' work items, the next n.medium the medium rows, the rest the
+// light ones.  A launch a bin left ~4.5 us per empty launch, about ten of them
+// a level with the pulls', and each bin's tail to itself: batches at SCALE 20 (64
+// roots) / 24 (256) / 26 (128) 1.18 / 10.25 / 22.1 -> 0.87 / 9.5 / 20.9 ms.
+template <int K, int G>
+__global__ __launch_bounds__(kT) void k_ms_push(MsLevel a, MsBins n) {
+  const unsigned b = blockIdx.x;
+  if (b < n.heavy)
+    push_items<K>(a, n, b, n.heavy);
+  else if (b < n.heavy + n.medium)
+    push_rows<K, G>(a, a.hubs, n.medium_end, b - n.heavy, n.medium);
+  else
+    push_rows<K, 1>(a, n.medium_end, a.n_c, b - n.heavy - n.medium, n.light);
 }
 
 // After a top-down level's pushes: new (vertex, root) pairs = the lanes of
@@ -557,11 +633,11 @@ __global__ __launch_bounds__(kT) void k_ms_td_count(MsLevel a) {
 // G lanes per vertex over new IDs [vb, ve); the words of the hubs stay in the
 // L2, and a word outside the frontier is zero.
 template <int K, int G, int U>
-__global__ __launch_bounds__(kT) void k_ms_hub_pull(MsLevel a, int64_t vb, int64_t ve) {
-  if (!ms_active(a) || !ms_hub_pull(a)) return;
+__device__ inline void hub_pull_rows(const MsLevel& a, int64_t vb, int64_t ve, int64_t rank,
+                                     int64_t nblk) {
   const int lig = threadIdx.x % G;
-  const int64_t gid = ((int64_t)blockIdx.x * kT + threadIdx.x) / G;
-  const int64_t ngroups = (int64_t)gridDim.x * (kT / G);
+  const int64_t gid = (rank * kT + threadIdx.x) / G;
+  const int64_t ngroups = nblk * (kT / G);
   const uint32_t hubs = (uint32_t)a.hubs;
   for (int64_t v = vb + gid; v < ve; v += ngroups) {
     const int64_t beg = a.row_off[v], end = a.row_off[v + 1];
@@ -611,20 +687,17 @@ __global__ __launch_bounds__(kT) void k_ms_hub_pull(MsLevel a, int64_t vb, int64
 
 // The heavy rows' hub pull, one wave per work item of `chunk` edges.
 template <int K>
-__global__ __launch_bounds__(kT) void k_ms_hub_pull_heavy(MsLevel a,
-                                                         const uint64_t* __restrict__ item_start,
-                                                         const uint32_t* __restrict__ item_vertex,
-                                                         int64_t n_items, int chunk) {
-  if (!ms_active(a) || !ms_hub_pull(a)) return;
+__device__ inline void hub_pull_items(const MsLevel& a, const MsBins& n, int64_t rank,
+                                      int64_t nblk) {
   const int lane = lane_id();
-  const int64_t wid = ((int64_t)blockIdx.x * kT + threadIdx.x) / kWave;
-  const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
+  const int64_t wid = (rank * kT + threadIdx.x) / kWave;
+  const int64_t nw = nblk * kWavesPerBlock;
   const uint32_t hubs = (uint32_t)a.hubs;
   constexpr int U = 4;
-  for (int64_t it = wid; it < n_items; it += nw) {
-    const int64_t v = item_vertex[it];
-    const int64_t beg = a.row_off[v] + (int64_t)(it - item_start[v]) * chunk;
-    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)chunk);
+  for (int64_t it = wid; it < n.n_items; it += nw) {
+    const int64_t v = n.item_vertex[it];
+    const int64_t beg = a.row_off[v] + (int64_t)(it - n.item_start[v]) * n.chunk;
+    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)n.chunk);
     uint64_t acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0;
@@ -657,6 +730,18 @@ __global__ __launch_bounds__(kT) void k_ms_hub_pull_heavy(MsLevel a,
       }
     }
   }
+}
+
+template <int K>
+__global__ __launch_bounds__(kT) void k_ms_hub_pull(MsLevel a, MsBins n) {
+  if (!ms_active(a) || !ms_hub_pull(a)) return;
+  const unsigned b = blockIdx.x;
+  if (b < n.heavy)
+    hub_pull_items<K>(a, n, b, n.heavy);
+  else if (b < n.heavy + n.medium)
+    hub_pull_rows<K, 16, 2>(a, a.hubs, n.medium_end, b - n.heavy, n.medium);
+  else
+    hub_pull_rows<K, 1, 4>(a, n.medium_end, a.n_c, b - n.heavy - n.medium, n.light);
 }
 
 // Streaming pull: the edge array is cut into tiles of kTile edges, one block
@@ -964,56 +1049,6 @@ __global__ __launch_bounds__(kT) void k_ms_hyb_push_heavy(MsLevel a,
   }
 }
 
-// Split level.  A root whose level-L frontier is light (its degree sum below
-// split_thr) would keep almost every vertex's pull scanning its whole row:
-// few vertices have a neighbour in that frontier, and a pull stops only
-// when every lane it lacks is covered.  Those roots push instead, along the
-// rows of their frontier vertices, and the pulls stop once the other lanes
-// are covered.
-//
-// Per-lane degree sums of F_L come from the count pass of the top-down level
-// that produced it (k_ms_td_count).
-// One block: sums the lane_part rows per lane (each wave a quarter of the
-// rows, 16 loads in flight per lane) and sets split_mask to the lanes
-// present in F_L whose frontier degree sum is below split_thr.
-template <int K>
-__global__ __launch_bounds__(kT) void k_ms_lane_mask(MsLevel a, int parts) {
-  __shared__ unsigned long long mk[4];
-  __shared__ unsigned long long ws[kWavesPerBlock][64 * K];
-  if (!ms_active(a) || ms_mode(a, a.L) != kModeSplit) return;
-  const int t = threadIdx.x, wave = t / kWave, lane = lane_id();
-  if (t < 4) mk[t] = 0;
-  const int per = (parts + kWavesPerBlock - 1) / kWavesPerBlock;
-  const int p0 = wave * per, p1 = min(parts, p0 + per);
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int lanei = 64 * k + lane;
-    unsigned long long acc[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0;
-    for (int p = p0; p < p1; p += 16) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (p + j < p1) acc[j] += a.lane_part[(int64_t)(p + j) * 256 + lanei];
-    }
-    unsigned long long sum = 0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) sum += acc[j];
-    ws[wave][lanei] = sum;
-  }
-  __syncthreads();
-  if (t < 64 * K) {
-    unsigned long long sum = 0;
-#pragma unroll
-    for (int w = 0; w < kWavesPerBlock; ++w) sum += ws[w][t];
-    const bool present = (a.act_l[t >> 6] >> (t & 63)) & 1ull;
-    if (present && sum < a.split_thr) atomicOr(&mk[t >> 6], 1ull << (t & 63));
-  }
-  __syncthreads();
-  if (t < 4) a.split_mask[t] = mk[t];
-}
-
-
 // After a streaming level: F_{L+1} = gathered lanes & ~seen, seen |= F_{L+1},
 // frontier bitmap, counters.
 template <int K>
@@ -1060,8 +1095,8 @@ __global__ __launch_bounds__(kT) void k_ms_commit(MsLevel a, int want) {
 // frontier is zero): on the levels that pull, most neighbours are in the
 // frontier, and the test cost a round trip per round.
 template <int K, int G, int U>
-__global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve) {
-  __shared__ uint64_t red[kWavesPerBlock];
+__device__ inline void bu_rows(const MsLevel& a, int64_t vb, int64_t ve, int64_t rank,
+                               int64_t nblk, uint64_t* red) {
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModePull && mode != kModeSplit) return;
@@ -1073,8 +1108,8 @@ __global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve)
   const bool hubs_pulled = split && K >= kSplitHubWords;
   const uint32_t hubs = hubs_pulled ? (uint32_t)a.hubs : 0u;
   const int lig = threadIdx.x % G;
-  const int64_t gid0 = ((int64_t)blockIdx.x * kT + threadIdx.x) / G;
-  const int64_t ngroups = (int64_t)gridDim.x * (kT / G);
+  const int64_t gid0 = (rank * kT + threadIdx.x) / G;
+  const int64_t ngroups = nblk * (kT / G);
   uint64_t disc = 0, edges = 0;
   // a lane absent from F_L cannot be found this level: it counts as covered
   // when deciding that a vertex is done (roots whose search has ended, e.g.
@@ -1188,29 +1223,25 @@ __global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, int64_t vb, int64_t ve)
 // the frontier lanes it finds into acc[v]; k_ms_bu_heavy_fin turns acc into
 // F_{L+1} once every item is done.
 template <int K, int U>
-__global__ __launch_bounds__(kT) void k_ms_bu_heavy(MsLevel a,
-                                                   const uint64_t* __restrict__ item_start,
-                                                   const uint32_t* __restrict__ item_vertex,
-                                                   int64_t n_items, int chunk,
-                                                   uint64_t* __restrict__ gacc) {
+__device__ inline void bu_items(const MsLevel& a, const MsBins& n, int64_t rank, int64_t nblk) {
   if (!ms_active(a)) return;
   const int mode = ms_mode(a, a.L);
   if (mode != kModePull && mode != kModeSplit) return;
   const int lane = lane_id();
-  const int64_t wid = ((int64_t)blockIdx.x * kT + threadIdx.x) / kWave;
-  const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
+  const int64_t wid = (rank * kT + threadIdx.x) / kWave;
+  const int64_t nw = nblk * kWavesPerBlock;
   // lanes absent from F_L (and on a split level the pushing lanes) count as
   // covered (as in k_ms_bu)
   uint64_t inact[K];
 #pragma unroll
   for (int k = 0; k < K; ++k)
     inact[k] = ~a.act_l[k] | (mode == kModeSplit ? a.split_mask[k] : 0ull);
-  for (int64_t it = wid; it < n_items; it += nw) {
-    const int64_t v = item_vertex[it];
+  for (int64_t it = wid; it < n.n_items; it += nw) {
+    const int64_t v = n.item_vertex[it];
     uint64_t s[K], g0[K], f[K];
     load_lanes<K>(a.seen + v * K, s);
     load_lanes<K>(a.fl + v * K, f);
-    load_lanes<K>(gacc + v * K, g0);
+    load_lanes<K>(n.acc + v * K, g0);
     bool full = true, hub = false;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
@@ -1220,8 +1251,8 @@ __global__ __launch_bounds__(kT) void k_ms_bu_heavy(MsLevel a,
                     (a.split_mask[k] & ~(s[k] | g0[k])) != 0);
     }
     if (full && !hub) continue;
-    const int64_t beg = a.row_off[v] + (int64_t)(it - item_start[v]) * chunk;
-    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)chunk);
+    const int64_t beg = a.row_off[v] + (int64_t)(it - n.item_start[v]) * n.chunk;
+    const int64_t end = min(a.row_off[v + 1], beg + (int64_t)n.chunk);
     uint64_t acc[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = 0;
@@ -1254,10 +1285,23 @@ __global__ __launch_bounds__(kT) void k_ms_bu_heavy(MsLevel a,
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         const uint64_t nb = acc[k] & ~s[k] & ~g0[k];
-        if (nb) atomicOr((unsigned long long*)&gacc[v * K + k], (unsigned long long)nb);
+        if (nb) atomicOr((unsigned long long*)&n.acc[v * K + k], (unsigned long long)nb);
       }
     }
   }
+}
+
+// The pulls of a level, every bin in one launch (as k_ms_push).
+template <int K, int G, int U>
+__global__ __launch_bounds__(kT) void k_ms_bu(MsLevel a, MsBins n) {
+  __shared__ uint64_t red[kWavesPerBlock];
+  const unsigned b = blockIdx.x;
+  if (b < n.heavy)
+    bu_items<K, 4>(a, n, b, n.heavy);
+  else if (b < n.heavy + n.medium)
+    bu_rows<K, G, U>(a, a.hubs, n.medium_end, b - n.heavy, n.medium, red);
+  else
+    bu_rows<K, 1, 4>(a, n.medium_end, a.n_c, b - n.heavy - n.medium, n.light, red);
 }
 
 template <int K>
@@ -1666,22 +1710,6 @@ MsLevel level_args(const g500_msbfs* b, int L) {
   return a;
 }
 
-template <int K, int G>
-void launch_push(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t ve, hipStream_t s) {
-  if (ve <= vb) return;
-  hipLaunchKernelGGL((k_ms_push<K, G>), dim3(sweep_grid(b, ve - vb, G)), dim3(kT), 0, s, a, vb,
-                     ve);
-  G500_CHECK_LAUNCH();
-}
-
-template <int K, int G, int U>
-void launch_bu(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t ve, hipStream_t s) {
-  if (ve <= vb) return;
-  hipLaunchKernelGGL((k_ms_bu<K, G, U>), dim3(sweep_grid(b, ve - vb, G)), dim3(kT), 0, s, a, vb,
-                     ve);
-  G500_CHECK_LAUNCH();
-}
-
 // One level L -> L+1: preparation, then the top-down and the bottom-up
 // kernels of every bin (the ones of the other direction return at once).
 template <int K, int G>
@@ -1704,12 +1732,15 @@ void launch_hyb_push(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t 
 }
 
 template <int K, int G>
-void launch_hub_pull(const g500_msbfs* b, const MsLevel& a, int64_t vb, int64_t ve,
-                     hipStream_t s) {
-  if (ve <= vb) return;
-  constexpr int U = G == 1 ? 4 : 2;
-  hipLaunchKernelGGL((k_ms_hub_pull<K, G, U>), dim3(sweep_grid(b, ve - vb, G)), dim3(kT), 0, s, a,
-                     vb, ve);
+void launch_push(const MsLevel& a, const MsBins& n, hipStream_t s) {
+  hipLaunchKernelGGL((k_ms_push<K, G>), dim3(n.heavy + n.medium + n.light), dim3(kT), 0, s, a, n);
+  G500_CHECK_LAUNCH();
+}
+
+template <int K, int G, int U>
+void launch_bu(const MsLevel& a, const MsBins& n, hipStream_t s) {
+  hipLaunchKernelGGL((k_ms_bu<K, G, U>), dim3(n.heavy + n.medium + n.light), dim3(kT), 0, s, a,
+                     n);
   G500_CHECK_LAUNCH();
 }
 
@@ -1732,38 +1763,31 @@ void level_kernels(const g500_msbfs* b, int L, hipStream_t s) {
       1, std::min<int64_t>(ceil_div(n_c * K, kT), (int64_t)num_cus(b->g->device) * 8));
   hipLaunchKernelGGL((k_ms_prep<K>), dim3(pgrid), dim3(kT), 0, s, a, bw);
   G500_CHECK_LAUNCH();
-  // a split level's pushing lanes (split levels need split_bp > 0 and come
-  // after a top-down level)
-  if (a.split_thr > 0 && L > 0) {
-    hipLaunchKernelGGL((k_ms_lane_mask<K>), dim3(1), dim3(kT), 0, s, a, kLaneParts);
-    G500_CHECK_LAUNCH();
-  }
   // pushes: every lane at a top-down level, the pushing lanes at a split
   // level (before the pulls, which take the pushed lanes into F_{L+1})
   const unsigned hgrid = (unsigned)std::max<int64_t>(
       1, std::min<int64_t>(ceil_div(b->n_items, kWavesPerBlock),
                            (int64_t)num_cus(b->g->device) * b->tuning.blocks_per_cu));
+  const int group = b->tuning.medium_group;
+  MsBins bins{b->item_start.get(), b->item_vertex.get(), b->acc.get(), b->n_items, m, chunk,
+              b->n_items > 0 ? hgrid : 0u,
+              m > h ? sweep_grid(b, m - h, group) : 0u,
+              n_c > m ? sweep_grid(b, n_c - m, 1) : 0u};
   // hub pulls follow a top-down level (whose count pass takes the degree sums)
   if (b->n_items > 0 && L > 0 && L <= kHubLevels) {
-    hipLaunchKernelGGL((k_ms_hub_pull_heavy<K>), dim3(hgrid), dim3(kT), 0, s, a,
-                       b->item_start.get(), b->item_vertex.get(), b->n_items, chunk);
-    G500_CHECK_LAUNCH();
-    launch_hub_pull<K, 16>(b, a, h, m, s);
-    launch_hub_pull<K, 1>(b, a, m, n_c, s);
-  }
-  if (b->n_items > 0) {
-    hipLaunchKernelGGL((k_ms_push_heavy<K>), dim3(hgrid), dim3(kT), 0, s, a,
-                       b->item_start.get(), b->item_vertex.get(), b->n_items, chunk);
+    MsBins pull = bins;
+    if (m > h) pull.medium = sweep_grid(b, m - h, 16);
+    hipLaunchKernelGGL((k_ms_hub_pull<K>), dim3(pull.heavy + pull.medium + pull.light), dim3(kT),
+                       0, s, a, pull);
     G500_CHECK_LAUNCH();
   }
-  switch (b->tuning.medium_group) {
-    case 2: launch_push<K, 2>(b, a, h, m, s); break;
-    case 4: launch_push<K, 4>(b, a, h, m, s); break;
-    case 8: launch_push<K, 8>(b, a, h, m, s); break;
-    case 16: launch_push<K, 16>(b, a, h, m, s); break;
-    default: launch_push<K, 32>(b, a, h, m, s); break;
+  if (n_c > 0) switch (group) {
+    case 2: launch_push<K, 2>(a, bins, s); break;
+    case 4: launch_push<K, 4>(a, bins, s); break;
+    case 8: launch_push<K, 8>(a, bins, s); break;
+    case 16: launch_push<K, 16>(a, bins, s); break;
+    default: launch_push<K, 32>(a, bins, s); break;
   }
-  launch_push<K, 1>(b, a, m, n_c, s);
   hipLaunchKernelGGL((k_ms_td_count<K>), dim3(sweep_grid(b, n_c, 1)), dim3(kT), 0, s, a);
   G500_CHECK_LAUNCH();
   // Every kernel below is queued for every level and returns at once unless
@@ -1810,23 +1834,18 @@ void level_kernels(const g500_msbfs* b, int L, hipStream_t s) {
                        (int)kModeStream);
     G500_CHECK_LAUNCH();
   }
+  if (n_c > 0) switch (group) {
+    case 2: launch_bu<K, 2, 4>(a, bins, s); break;
+    case 4: launch_bu<K, 4, 4>(a, bins, s); break;
+    case 8: launch_bu<K, 8, 4>(a, bins, s); break;
+    case 16: launch_bu<K, 16, 2>(a, bins, s); break;
+    default: launch_bu<K, 32, 2>(a, bins, s); break;
+  }
   if (b->n_items > 0) {
-    hipLaunchKernelGGL((k_ms_bu_heavy<K, 4>), dim3(hgrid), dim3(kT), 0, s, a,
-                       b->item_start.get(), b->item_vertex.get(), b->n_items, chunk,
-                       b->acc.get());
-    G500_CHECK_LAUNCH();
     hipLaunchKernelGGL((k_ms_bu_heavy_fin<K>), dim3(sweep_grid(b, h, 1)), dim3(kT), 0, s, a, h,
                        b->acc.get());
     G500_CHECK_LAUNCH();
   }
-  switch (b->tuning.medium_group) {
-    case 2: launch_bu<K, 2, 4>(b, a, h, m, s); break;
-    case 4: launch_bu<K, 4, 4>(b, a, h, m, s); break;
-    case 8: launch_bu<K, 8, 4>(b, a, h, m, s); break;
-    case 16: launch_bu<K, 16, 2>(b, a, h, m, s); break;
-    default: launch_bu<K, 32, 2>(b, a, h, m, s); break;
-  }
-  launch_bu<K, 1, 4>(b, a, m, n_c, s);
 }
 
 void enqueue_level(const g500_msbfs* b, int K, int L, hipStream_t s) {
