@@ -35,13 +35,14 @@
 //                 vertices with edges and starts on a second stream at the
 //                 bottom-up -> top-down switch, against a bitmap snapshot;
 //                 k_pred_fixup adds the vertices the last levels reach.
-//   k_level_decide, k_queue_decide   one block closing each step: the
-//                 step's totals, the direction rule, the next step's code.
+//   last_of, close_level, close_queue   the last block of a step's last
+//                 kernel closes it: the step's totals, the direction rule,
+//                 the next step's code.
 //
 // The level loop is a sequence of steps (a level, or the bitmap -> queue
 // conversion at the bottom-up -> top-down switch).  Every block of a step's
-// kernels writes its totals to a per-block slot; the one-block closing
-// kernel sums the slots, applies the reference's direction rule on the
+// kernels writes its totals to a per-block slot; the last block of the
+// last kernel sums the slots, applies the reference's direction rule on the
 // device, writes the code of the step that must run next into the loop
 // state and posts the totals with that code to pinned host memory.  Every
 // kernel of a step first compares its own code with that state and returns
@@ -147,9 +148,12 @@ __device__ inline void post_report(HostReport* ring, const unsigned long long v[
 }
 
 // Every kernel of a step starts with this test: the step runs only if the
-// level loop's state names it as the next one.  The closing kernel of the
+// level loop's state names it as the next one.  The last kernel of the
 // step before wrote that code (kernels of one stream see the writes of the
-// kernels before them), and nothing writes it while the step runs.
+// kernels before them).  While the step runs only its closing block writes
+// the state: blocks that start after that see another code and return, and a
+// block that still saw the step's code reads the step's own frontier entry,
+// which the closing leaves alone (it writes the other level's).
 __device__ inline bool step_is_next(const LevelSync* ls, uint32_t code) {
   return __builtin_amdgcn_readfirstlane(ls->step) == code;
 }
@@ -182,8 +186,9 @@ __device__ inline uint32_t decide_next(const LevelSync& cur, LevelSync* ls, uint
     ls->prev_nq = nq_size;
     if (td && next_td) {
       next = td_step_mode(nq_size, nq_edges, cur.exec_thr);
-      ls->qlen = nq_size;
-      ls->qedges = nq_edges;
+      Frontier& f = next_frontier(ls, code);
+      f.qlen = nq_size;
+      f.qedges = nq_edges;
     } else if (td) {
       // a top-down expansion leaves the unvisited lists behind, a sweep
       // (also one that ran a top-down level) refreshes them
@@ -197,41 +202,77 @@ __device__ inline uint32_t decide_next(const LevelSync& cur, LevelSync* ls, uint
   return nc;
 }
 
-// One block, launched after a level's kernels (step `code`): sums the
-// blocks' partial totals (counts in cpart, degree sums in epart) plus what
-// queue reservations took from ls->cnt, clears ls->cnt, decides the next
-// step and posts the totals with its code.  The blocks of a level kernel
-// finish together, so summing their totals here replaces same-address
-// atomics, which serialize.  Thread 0 reads the loop state at the start
-// (the earlier kernels' atomics are complete at this kernel's start), so
-// its loads overlap the partial sums'.
-__global__ __launch_bounds__(kT) void k_level_decide(const uint64_t* __restrict__ cpart,
-                                                    int nc,
-                                                    const uint64_t* __restrict__ epart,
-                                                    int ne, LevelSync* ls, HostReport* hr,
-                                                    unsigned long long seq, uint32_t code) {
-  if (!step_is_next(ls, code)) return;
-  __shared__ uint64_t red[kWavesPerBlock];
+// Closing a step.  The block of its last kernel that finishes last sums the
+// blocks' totals, decides the next step and posts both, which took a launch
+// of its own before, seven times a run; a run at SCALE 16 / 18 / 20 / 24:
+// 156 / 182 / 226 / 477 us with those launches, 147 / 176 / 214 / 466
+// without; SCALE 26 the same within the noise.  Every block leaves its total in its slot with a
+// device-scope store, waits until that has arrived and takes a ticket; the
+// last block reads the slots with device-scope loads.  No fence: one would
+// write back the block's whole L2, dirty with pred entries.  Tickets of one
+// address serialize at ~12 ns, so they are taken from kTicketSlots counters
+// (the last of a slot goes on to the common one): 2048 blocks pass in ~1 us.
+constexpr int kTicketSlots = 64;
+constexpr int kTicketPad = 32;  // a counter per 128-byte line
+constexpr int kTickets = (kTicketSlots + 1) * kTicketPad;
+
+struct Closing {
+  unsigned int* tickets;
+  HostReport* report;
+  unsigned long long seq;
+};
+
+// True (in all threads) in the last of `blocks` blocks (blockIdx < blocks)
+// to come here; thread 0 stores the block's total in *slot first.  Its own
+// earlier atomics returned their results, so they are complete.
+__device__ inline bool last_of(const Closing& cl, unsigned blocks, uint64_t* slot,
+                               uint64_t total) {
+  __shared__ bool last;
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(slot, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned slots = min(blocks, (unsigned)kTicketSlots), mine = blockIdx.x % slots;
+    const unsigned members = blocks / slots + (mine < blocks % slots ? 1u : 0u);
+    unsigned int* t = cl.tickets + (1 + mine) * kTicketPad;
+    last = false;
+    if (atomicAdd(t, 1u) + 1 == members) {
+      *t = 0;
+      if (atomicAdd(cl.tickets, 1u) + 1 == slots) {
+        *cl.tickets = 0;
+        last = true;
+      }
+    }
+  }
+  __syncthreads();
+  return last;
+}
+
+__device__ inline uint64_t sum_slots(const uint64_t* part, int n, uint64_t* red) {
+  uint64_t x = 0;
+  for (int i = threadIdx.x; i < n; i += kT)
+    x += __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();  // red may still be read by thread 0
+  return block_sum(x, red);
+}
+
+// The last block of a level (step `code`) closes it.  Top-down: the slots
+// hold degree sums and the queue's reservations the count; bottom-up: the
+// slots hold counts.  Thread 0 reads the loop state first, so its loads
+// overlap the slots'.
+__device__ inline void close_level(const uint64_t* part, int n, bool top_down, LevelSync* ls,
+                                   const Closing& cl, uint32_t code, uint64_t* red) {
   LevelSync cur;
   if (threadIdx.x == 0) cur = *ls;
-  uint64_t c = 0, d = 0;
-  for (int i = threadIdx.x; i < nc; i += kT) c += cpart[i];
-  for (int i = threadIdx.x; i < ne; i += kT) d += epart[i];
-  c = block_sum(c, red);
-  __syncthreads();  // thread 0 has read red
-  d = block_sum(d, red);
+  const uint64_t x = sum_slots(part, n, red);
   if (threadIdx.x == 0) {
-    unsigned long long v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = cur.cnt[i];
-      ls->cnt[i] = 0;
+    unsigned long long v[4] = {x, 0, 0, 0};
+    if (top_down) {
+      v[0] = atomicExch(&ls->cnt[0], 0ull);
+      v[1] = x;
     }
-    v[0] += c;
-    v[1] += d;
+    ls->cnt[2] = 0;
     v[2] = decide_next(cur, ls, code, (long long)v[0], (long long)v[1]);
-    v[3] = 0;
-    post_report(hr, v, seq);
+    post_report(cl.report, v, cl.seq);
   }
 }
 
@@ -254,7 +295,8 @@ __global__ __launch_bounds__(kT) void k_bfs_init(uint64_t* __restrict__ vis,
                                                 int64_t* pred_new,
                                                 int64_t entry, uint32_t* q, LevelSync* ls,
                                                 LoopInit li,
-                                                const int64_t* __restrict__ row_off) {
+                                                const int64_t* __restrict__ row_off,
+                                                unsigned int* tickets) {
   // root: an original ID with an edge, or -1
   const int64_t root_new = root >= 0 ? (int64_t)o2n[root] : -1;
   for (int64_t w = (int64_t)blockIdx.x * kT + threadIdx.x; w < words;
@@ -266,13 +308,15 @@ __global__ __launch_bounds__(kT) void k_bfs_init(uint64_t* __restrict__ vis,
     if (root_new >= lo && root_new < lo + 64) word |= 1ull << (root_new - lo);
     vis[w] = word;
   }
+  if (blockIdx.x == 0 && threadIdx.x <= kTicketSlots) tickets[threadIdx.x * kTicketPad] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) ls->cnt[i] = 0;
+    Frontier& f = frontier(ls, li.first);
     ls->step = li.first;
     ls->growing = 1u;
-    ls->qlen = li.qlen;
-    ls->qedges = li.qedges;
+    f.qlen = li.qlen;
+    f.qedges = li.qedges;
     ls->prev_nq = 0;
     ls->alpha_thr = li.alpha_thr;
     ls->beta_thr = li.beta_thr;
@@ -281,7 +325,7 @@ __global__ __launch_bounds__(kT) void k_bfs_init(uint64_t* __restrict__ vis,
     if (root_new >= 0 && root_new < n_c) {
       pred_new[root_new] = entry;
       q[0] = (uint32_t)root_new;
-      ls->qedges = row_off[root_new + 1] - row_off[root_new];
+      f.qedges = row_off[root_new + 1] - row_off[root_new];
     }
   }
 }
@@ -335,7 +379,7 @@ __global__ __launch_bounds__(kT) void k_td_prep_sums(
     const int64_t* __restrict__ row_off, uint64_t* __restrict__ dsum,
     uint64_t* __restrict__ bsum, uint64_t* __restrict__ boff, unsigned int* ticket) {
   if (!step_is_next(ls, code)) return;
-  const int64_t qlen = ls->qlen;
+  const int64_t qlen = frontier(ls, code).qlen;
   if (qlen <= kTdWin) return;
   __shared__ uint64_t wsum[kWavesPerBlock];
   __shared__ bool last;
@@ -389,7 +433,7 @@ __global__ __launch_bounds__(kT) void k_td_prep_tiles(
     const uint64_t* __restrict__ bsum, const uint64_t* __restrict__ boff,
     uint32_t* __restrict__ tile_owner) {
   if (!step_is_next(ls, code)) return;
-  const int64_t qlen = ls->qlen;
+  const int64_t qlen = frontier(ls, code).qlen;
   if (qlen <= kTdWin) return;
   const int t = threadIdx.x;
   const int64_t nb = ceil_div(qlen, (int64_t)kPrepTile);
@@ -424,7 +468,8 @@ __global__ __launch_bounds__(kT) void k_td_prep_tiles(
 // block stages the whole frontier (prefix sum of degrees, row base, original
 // ID) in LDS itself.
 // The grid is fixed (kMaxGrid); blocks past the frontier's degree sum (an
-// upper bound of its row entries) write a zero total and return.
+// upper bound of its row entries) return at once and take no part in closing
+// the level.
 __global__ __launch_bounds__(kT) void k_td_expand(
     const uint32_t* __restrict__ q, uint32_t code,
     const uint64_t* __restrict__ dsum, const uint32_t* __restrict__ tile_owner,
@@ -432,13 +477,13 @@ __global__ __launch_bounds__(kT) void k_td_expand(
     const uint32_t* __restrict__ col, const uint32_t* __restrict__ n2o,
     const uint32_t* __restrict__ deg_new, unsigned long long* vis,
     int64_t* __restrict__ pred_new, uint32_t* __restrict__ nq, LevelSync* ls,
-    uint64_t* __restrict__ epart, uint64_t level_bits) {
+    uint64_t* __restrict__ epart, uint64_t level_bits, Closing cl) {
   if (!step_is_next(ls, code)) return;
-  if ((uint64_t)blockIdx.x * kTdTile >= (uint64_t)ls->qedges) {
-    if (threadIdx.x == 0) epart[blockIdx.x] = 0;
-    return;
-  }
-  const int64_t qlen = ls->qlen;
+  const Frontier front = frontier(ls, code);
+  const unsigned active = (unsigned)min(
+      max(ceil_div((int64_t)front.qedges, (int64_t)kTdTile), (int64_t)1), (int64_t)gridDim.x);
+  if (blockIdx.x >= active) return;
+  const int64_t qlen = front.qlen;
   // the tile's owners, staged once per tile: prefix sum, col offset of edge
   // 0 of the owner's range (row_off[u] - dsum[i]) and original ID.  On heavy
   // levels a tile has one or two owners (hubs) shared by every block at
@@ -595,7 +640,8 @@ __global__ __launch_bounds__(kT) void k_td_expand(
     __syncthreads();
   }
   const uint64_t s = block_sum(my_edges, red);
-  if (t == 0) epart[blockIdx.x] = s;
+  if (last_of(cl, active, epart + blockIdx.x, s))
+    close_level(epart, (int)active, true, ls, cl, code, red);
 }
 
 // Bottom-up levels.  A wave owns a chunk of cw bitmap words (64 cw vertices)
@@ -939,8 +985,9 @@ __global__ __launch_bounds__(kBuT) void k_bu_long(
     const int64_t* __restrict__ row_off, const uint32_t* __restrict__ col,
     const uint32_t* __restrict__ n2o, int64_t* __restrict__ pred_new,
     uint32_t* __restrict__ unv, uint32_t* unv_cnt,
-    const uint32_t* __restrict__ longv, const LevelSync* ls, uint32_t code,
-    uint64_t* __restrict__ cpart, uint64_t level_bits, uint64_t* __restrict__ wacc) {
+    const uint32_t* __restrict__ longv, LevelSync* ls, uint32_t code,
+    uint64_t* __restrict__ cpart, int nsweep, uint64_t level_bits, uint64_t* __restrict__ wacc,
+    Closing cl) {
   if (!step_is_next(ls, code)) return;
   __shared__ uint64_t red[kBuWaves];
   __shared__ uint64_t hub[kHubWords];
@@ -996,12 +1043,15 @@ __global__ __launch_bounds__(kBuT) void k_bu_long(
     }
   }
   const uint64_t s = block_sum<kBuWaves>(nfound, red);
-  if (threadIdx.x == 0) cpart[blockIdx.x] = s;
   if (count) {
     __syncthreads();
     const uint64_t sb = block_sum<kBuWaves>(scan_b, red);
     if (threadIdx.x == 0) wacc[blockIdx.x] += sb;
   }
+  // a top-down level run as a sweep is closed behind its conversion
+  if (step_mode(code) != kModeBUSweep) return;
+  if (last_of(cl, gridDim.x, cpart + nsweep + blockIdx.x, s))
+    close_level(cpart, nsweep + (int)gridDim.x, false, ls, cl, code, red);
 }
 
 // Four waves per SIMD (128 VGPRs, a 12-byte spill) rather than the three its
@@ -1013,8 +1063,8 @@ __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void 
     const uint32_t* __restrict__ col, const uint2* __restrict__ first,
     const uint64_t* __restrict__ multi, const uint32_t* __restrict__ n2o,
     int64_t* __restrict__ pred_new, uint32_t* __restrict__ unv,
-    uint32_t* __restrict__ unv_cnt, const LevelSync* ls, uint32_t code,
-    uint64_t* __restrict__ cpart, uint64_t level_bits, uint64_t* __restrict__ wacc) {
+    uint32_t* __restrict__ unv_cnt, LevelSync* ls, uint32_t code,
+    uint64_t* __restrict__ cpart, uint64_t level_bits, uint64_t* __restrict__ wacc, Closing cl) {
   if (!step_is_next(ls, code)) return;
   __shared__ unsigned long long fw[kBuWaves][kWave];
   __shared__ uint64_t red[kBuWaves];
@@ -1098,12 +1148,13 @@ __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void 
     wave_sync();
   }
   const uint64_t s = block_sum<kBuWaves>(nfound, red);
-  if (threadIdx.x == 0) cpart[blockIdx.x] = s;
   if (count) {
     __syncthreads();
     const uint64_t sb = block_sum<kBuWaves>(scan_b, red);
     if (threadIdx.x == 0) wacc[blockIdx.x] += sb;
   }
+  if (last_of(cl, gridDim.x, cpart + blockIdx.x, s))
+    close_level(cpart, (int)gridDim.x, false, ls, cl, code, red);
 }
 
 // queue <- bits set in cur but not in prev; reports (count, degree sum).
@@ -1145,6 +1196,41 @@ __global__ __launch_bounds__(kT) void k_queue_count(const uint64_t* __restrict__
   if (lane_id() == 0) wcnt[(int64_t)blockIdx.x * kWavesPerBlock + threadIdx.x / kWave] = (uint32_t)c;
 }
 
+// The last block of k_queue_write closes a step whose frontier came from the
+// bitmap: sums the conversion's totals (count, degree sum) and clears ls->cnt
+// (a top-down level run as a sweep leaves the long-row count there).  After a
+// top-down level run as a sweep the totals are the level's and the direction
+// rule decides the next step; after the conversion at the switch to top-down
+// they are the first top-down frontier's, which runs next (as a sweep if its
+// degree sum passes the execution threshold).
+__device__ inline void close_queue(const uint32_t* __restrict__ wcnt, const uint64_t* bedges,
+                                   LevelSync* ls, const Closing& cl, uint32_t code,
+                                   uint64_t* red) {
+  LevelSync cur;
+  if (threadIdx.x == 0) cur = *ls;
+  uint64_t c = 0;
+  for (int i = threadIdx.x; i < (int)gridDim.x * kWavesPerBlock; i += kT) c += wcnt[i];
+  const uint64_t d = sum_slots(bedges, (int)gridDim.x, red);
+  __syncthreads();  // thread 0 has read red
+  c = block_sum(c, red);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ls->cnt[i] = 0;
+    uint32_t next;
+    if (step_mode(code) == kModeConv) {
+      Frontier& f = frontier(ls, code);
+      f.qlen = (long long)c;
+      f.qedges = (long long)d;
+      next = step_code(step_level(code), td_step_mode((long long)c, (long long)d, cur.exec_thr));
+      ls->step = next;
+    } else {
+      next = decide_next(cur, ls, code, (long long)c, (long long)d);
+    }
+    const unsigned long long v[4] = {c, d, next, 0ull};
+    post_report(cl.report, v, cl.seq);
+  }
+}
+
 __global__ __launch_bounds__(kT) void k_queue_write(const uint64_t* __restrict__ cur,
                                                    const uint64_t* __restrict__ prev,
                                                    int64_t words,
@@ -1152,7 +1238,7 @@ __global__ __launch_bounds__(kT) void k_queue_write(const uint64_t* __restrict__
                                                    const uint32_t* __restrict__ wcnt,
                                                    uint32_t* __restrict__ out,
                                                    uint64_t* __restrict__ bedges,
-                                                   const LevelSync* ls, uint32_t code) {
+                                                   LevelSync* ls, uint32_t code, Closing cl) {
   if (!step_is_next(ls, code)) return;
   __shared__ uint64_t red[kWavesPerBlock];
   const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
@@ -1196,47 +1282,8 @@ __global__ __launch_bounds__(kT) void k_queue_write(const uint64_t* __restrict__
   }
   __syncthreads();  // red is reused
   const uint64_t s = block_sum(edges, red);
-  if (t == 0) bedges[blockIdx.x] = s;
-}
-
-// One block, closing a step whose frontier came from the bitmap: sums the
-// conversion's totals (count, degree sum) -- all blocks of k_queue_write
-// finish together, so here rather than by atomics on one address, which
-// serialize -- and clears ls->cnt (a top-down level run as a sweep leaves
-// the long-row count there).  After a top-down level run as a sweep the
-// totals are the level's and the direction rule decides the next step; after
-// the conversion at the switch to top-down they are the first top-down
-// frontier's, which runs next (as a sweep if its degree sum passes the
-// execution threshold).
-__global__ __launch_bounds__(kT) void k_queue_decide(const uint32_t* __restrict__ wcnt,
-                                                    const uint64_t* __restrict__ bedges,
-                                                    int blocks, LevelSync* ls, HostReport* hr,
-                                                    unsigned long long seq, uint32_t code) {
-  if (!step_is_next(ls, code)) return;
-  __shared__ uint64_t red[kWavesPerBlock];
-  LevelSync cur;
-  if (threadIdx.x == 0) cur = *ls;
-  uint64_t c = 0, d = 0;
-  for (int i = threadIdx.x; i < blocks * kWavesPerBlock; i += kT) c += wcnt[i];
-  for (int i = threadIdx.x; i < blocks; i += kT) d += bedges[i];
-  c = block_sum(c, red);
-  __syncthreads();  // thread 0 has read red
-  d = block_sum(d, red);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ls->cnt[i] = 0;
-    uint32_t next;
-    if (step_mode(code) == kModeConv) {
-      ls->qlen = (long long)c;
-      ls->qedges = (long long)d;
-      next = step_code(step_level(code), td_step_mode((long long)c, (long long)d, cur.exec_thr));
-      ls->step = next;
-    } else {
-      next = decide_next(cur, ls, code, (long long)c, (long long)d);
-    }
-    const unsigned long long v[4] = {c, d, next, 0ull};
-    post_report(hr, v, seq);
-  }
+  if (last_of(cl, gridDim.x, bedges + blockIdx.x, s))
+    close_queue(wcnt, bedges, ls, cl, code, red);
 }
 
 // pred[o] for every original ID: the level-written entry of its new ID if
@@ -1449,8 +1496,7 @@ __global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t roo
     q[0] = (uint16_t)r;
     ls.step = li.first;
     ls.growing = 1u;
-    ls.qlen = 1;
-    ls.qedges = g.row_off[r + 1] - g.row_off[r];
+    frontier(&ls, li.first) = {1, g.row_off[r + 1] - g.row_off[r]};
     ls.prev_nq = 0;
     ls.alpha_thr = li.alpha_thr;
     ls.beta_thr = li.beta_thr;
@@ -1512,7 +1558,7 @@ __global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t roo
     if (mode == kModeDone || step == kSmallSteps) break;
     uint64_t count = 0, edges = 0;  // this thread's share
     if (mode == kModeTD || mode == kModeTDS) {
-      const int qlen = (int)ls.qlen;
+      const int qlen = (int)frontier(&ls, code).qlen;
       if (t == 0) fill = 0;
       for (int w0 = 0; w0 < qlen; w0 += kSmallT) {
         const int nwin = min(qlen - w0, kSmallT);
@@ -1630,8 +1676,7 @@ __global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t roo
       const LevelSync cur = ls;
       uint32_t next;
       if (mode == kModeConv) {
-        ls.qlen = (long long)sc;
-        ls.qedges = (long long)se;
+        frontier(&ls, code) = {(long long)sc, (long long)se};
         next = step_code(level, td_step_mode((long long)sc, (long long)se, cur.exec_thr));
         ls.step = next;
       } else {
@@ -1709,6 +1754,7 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
                              ceil_div(chunks, kBuWaves)));
   b->lpart.alloc((size_t)std::max<int64_t>(
       kMaxGrid, std::max<int64_t>(b->bu_grid[0] + b->bu_grid[2], b->bu_grid[1])));
+  b->tickets.alloc((size_t)kTickets);
   b->wacc.alloc((size_t)b->bu_grid[0] + b->bu_grid[2] + b->bu_grid[1]);
   b->lsync.alloc(1);
   G500_CHECK_HIP(hipMemset(b->lsync.get(), 0, sizeof(LevelSync)));
@@ -1896,6 +1942,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
     G500_CHECK_HIP(hipEventRecord(pool_event(b->level_events, st.ev), s));
   }
   // counting runs: per-block scan bytes, sweep / long-row / list slots
+  const Closing cl{b->tickets.get(), b->d_report, st.seq};
   uint64_t* wsweep = b->counting ? b->wacc.get() : nullptr;
   uint64_t* wlong = b->counting ? b->wacc.get() + b->bu_grid[0] : nullptr;
   uint64_t* wlist = b->counting ? b->wacc.get() + b->bu_grid[0] + b->bu_grid[2] : nullptr;
@@ -1912,8 +1959,8 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
     hipLaunchKernelGGL(k_bu_long, dim3(b->bu_grid[2]), dim3(kBuT), 0, s, in.vis,
                        (unsigned long long*)in.vis_alt, b->words, b->chunk_words, g->row_off.get(),
                        g->col.get(), g->new2orig.get(), b->pred_new.get(), b->unv.get(),
-                       b->unv_cnt.get(), in.nq, ls, code, b->lpart.get() + b->bu_grid[0],
-                       level_bits, wlong);
+                       b->unv_cnt.get(), in.nq, ls, code, b->lpart.get(), (int)b->bu_grid[0],
+                       level_bits, wlong, cl);
     G500_CHECK_LAUNCH();
     st.after.vis = in.vis_alt;
     st.after.vis_alt = in.vis;
@@ -1927,10 +1974,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
     G500_CHECK_LAUNCH();
     if (snap) G500_CHECK_HIP(hipEventRecord(b->ev_snap, s));
     hipLaunchKernelGGL(k_queue_write, grid, dim3(kT), 0, s, cur, prev, b->words,
-                       g->deg_new.get(), b->qcnt.get(), out, b->qedges.get(), ls, code);
-    G500_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_queue_decide, dim3(1), dim3(kT), 0, s, b->qcnt.get(), b->qedges.get(),
-                       (int)grid.x, ls, b->d_report, st.seq, code);
+                       g->deg_new.get(), b->qcnt.get(), out, b->qedges.get(), ls, code, cl);
     G500_CHECK_LAUNCH();
   };
   switch (mode) {
@@ -1948,10 +1992,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       hipLaunchKernelGGL(k_td_expand, dim3(kMaxGrid), dim3(kT), 0, s, in.q, code,
                          b->dsum.get(), b->tile_owner.get(), g->row_off.get(), g->col.get(),
                          g->new2orig.get(), g->deg_new.get(), (unsigned long long*)in.vis,
-                         b->pred_new.get(), in.nq, ls, b->lpart.get(), level_bits);
-      G500_CHECK_LAUNCH();
-      hipLaunchKernelGGL(k_level_decide, dim3(1), dim3(kT), 0, s, (const uint64_t*)nullptr, 0,
-                         b->lpart.get(), kMaxGrid, ls, b->d_report, st.seq, code);
+                         b->pred_new.get(), in.nq, ls, b->lpart.get(), level_bits, cl);
       G500_CHECK_LAUNCH();
       std::swap(st.after.q, st.after.nq);
       break;
@@ -1962,20 +2003,12 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       break;
     case kModeBUSweep:
       sweep();
-      hipLaunchKernelGGL(k_level_decide, dim3(1), dim3(kT), 0, s, b->lpart.get(),
-                         (int)(b->bu_grid[0] + b->bu_grid[2]), (const uint64_t*)nullptr, 0, ls,
-                         b->d_report, st.seq, code);
-      G500_CHECK_LAUNCH();
       break;
     case kModeBUList:
       hipLaunchKernelGGL(k_bu_list, dim3(b->bu_grid[1]), dim3(kBuT), 0, s, in.vis, in.vis_alt,
                          b->words, b->chunk_words, g->row_off.get(), g->col.get(), g->first.get(),
                          g->multi.get(), g->new2orig.get(), b->pred_new.get(), b->unv.get(),
-                         b->unv_cnt.get(), ls, code, b->lpart.get(), level_bits, wlist);
-      G500_CHECK_LAUNCH();
-      hipLaunchKernelGGL(k_level_decide, dim3(1), dim3(kT), 0, s, b->lpart.get(),
-                         (int)b->bu_grid[1], (const uint64_t*)nullptr, 0, ls, b->d_report,
-                         st.seq, code);
+                         b->unv_cnt.get(), ls, code, b->lpart.get(), level_bits, wlist, cl);
       G500_CHECK_LAUNCH();
       st.after.vis = in.vis_alt;
       st.after.vis_alt = in.vis;
@@ -2378,7 +2411,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
                      (int64_t)(((uint64_t)root_level << 48) | ((uint64_t)b->epoch << 32) |
                                (uint64_t)bfs_root),
                      b->q.get(),
-                     b->lsync.get(), li, g->row_off.get());
+                     b->lsync.get(), li, g->row_off.get(), b->tickets.get());
   G500_CHECK_LAUNCH();
 
   int64_t qlen = root_in ? 1 : 0;

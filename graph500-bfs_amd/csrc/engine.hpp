@@ -29,9 +29,8 @@ __host__ __device__ inline int step_level(uint32_t code) { return (int)(code >> 
 
 // Device-side state of the level loop.  cnt[] are the counters that queue
 // reservations take within a level (top-down next-queue slots in cnt[0],
-// long-row slots in cnt[2]); the step's closing kernel adds them to the
-// blocks' totals and clears them.  The closing kernel also applies the
-// direction rule and writes the code of the step that must run next into
+// long-row slots in cnt[2]); the block that closes the step adds them to the
+// blocks' totals and clears them.  It also applies the direction rule and writes the code of the step that must run next into
 // `step`; every kernel of a step compares that code with its own and returns
 // at once when they differ.  So the host may queue a predicted step behind
 // the running one: a wrong prediction costs its empty launches, never a
@@ -40,12 +39,28 @@ struct LevelSync {
   unsigned long long cnt[4];
   uint32_t step;       // code of the step to run next
   uint32_t growing;    // the frontier has grown at every level so far
-  long long qlen;      // top-down frontier queue length
-  long long qedges;    // its degree sum (>= its CSR entries)
+  // the top-down frontiers of even and odd levels: a level's closing block
+  // writes the next level's while other blocks may still read their own
+  struct Frontier {
+    long long qlen;    // queue length
+    long long qedges;  // its degree sum (>= its CSR entries)
+  } front[2];
   long long prev_nq;   // frontier size of the previous level
   long long alpha_thr, beta_thr, exec_thr;  // int64(m/alpha), int64(n_c/(beta*ef*2)), m/exec_alpha
   uint32_t snap_tag;   // code of the conversion that wrote the gather's bitmap snapshot (0: none)
 };
+
+using Frontier = LevelSync::Frontier;
+// the frontier a top-down step reads, and the one its closing writes
+__host__ __device__ inline Frontier& frontier(LevelSync* ls, uint32_t code) {
+  return ls->front[step_level(code) & 1];
+}
+__host__ __device__ inline const Frontier& frontier(const LevelSync* ls, uint32_t code) {
+  return ls->front[step_level(code) & 1];
+}
+__host__ __device__ inline Frontier& next_frontier(LevelSync* ls, uint32_t code) {
+  return ls->front[(step_level(code) + 1) & 1];
+}
 
 // Host-visible (pinned, coherent, mapped) step reports: a ring of slots, the
 // step with sequence number s posting to slot s % kReportSlots, so a step
@@ -110,6 +125,7 @@ struct g500_bfs {
   // run one at a time (as under a counter profiler)
   hipEvent_t ev_snap = nullptr;
   g500::DevBuf<uint64_t> lpart;   // per-block totals of a level's kernels
+  g500::DevBuf<unsigned int> tickets;  // blocks done in a step's last kernel (see last_of)
   g500::DevBuf<uint32_t> qcnt;    // per-wave counts of the bitmap -> queue conversion
   g500::DevBuf<uint64_t> qedges;  // its per-block degree sums
   // without CoreBFS: (original ID, new ID) of the vertices with edges, in
