@@ -1347,51 +1347,82 @@ __global__ __launch_bounds__(kT) void k_pred_gather(const uint32_t* __restrict__
   }
 }
 
-// Without CoreBFS, a vertex without edges is never reached and its pred
-// entry is always -1: the engine fills pred once and the gather walks only
-// core, the (original ID, new ID) pairs of the vertices with edges in
-// ascending original-ID order.  One pair per thread: per vertex one
-// random 8-byte read (its entry), the rest streams.  Started at the switch
-// back to top-down (snap_level > 0: the level of that conversion), it writes
-// only the vertices inside the bitmap snapshot -- this run's entries below
-// that level, which nothing writes again -- and leaves the rest to
-// k_pred_fixup, so the two write disjoint entries and need no order between
-// them.  An entry the top-down levels write while the gather reads it is
-// outside the snapshot whether it is read before (another epoch) or after
-// (its level).
-__global__ __launch_bounds__(kT) void k_pred_gather_core(const uint2* __restrict__ core,
-                                                        int64_t n_core, uint32_t epoch,
-                                                        const int64_t* __restrict__ pred_new,
-                                                        int64_t root,
-                                                        int64_t* __restrict__ pred,
-                                                        uint32_t snap_level,
-                                                        const LevelSync* ls, uint32_t snap_code) {
+// Without CoreBFS the gather needs no original -> new map: `bits` marks the
+// original IDs with edges, `off` their number before each word, and core lists
+// the new IDs of all of them in ascending original-ID order.  A wave takes
+// kGatherWords words at a time, a lane per vertex: the list streams and one
+// random 8-byte read per vertex with edges (its entry) is left.  Vertices
+// without edges are written too, as the -1 they always hold: leaving them out
+// halves the bytes written but leaves every cache line partly written, and a
+// run took as long at SCALE 26 and 2 % longer at SCALE 24.  The kernel at
+// SCALE 26: 261 us (3.5 TB/s); 284 with a (original ID, new ID) pair per
+// vertex read and only those vertices written.  A run at SCALE 26: 1075 us
+// before, 1027 with 4 words at a time, 1005 with 8; 2 words 1034.
+// Started at the switch back to top-down (snap_level > 0: the level of that
+// conversion), it writes of the vertices with edges only those inside the bitmap snapshot -- this
+// run's entries below that level, which nothing writes again -- and leaves
+// the rest to k_pred_fixup, so the two write disjoint entries and need no
+// order between them.  An entry the top-down levels write while the gather
+// reads it is outside the snapshot whether it is read before (another epoch)
+// or after (its level).
+constexpr int kGatherWords = 8;
+
+__global__ __launch_bounds__(kT) void k_pred_gather_core(
+    const uint64_t* __restrict__ bits, const uint64_t* __restrict__ off,
+    const uint32_t* __restrict__ core, int64_t n, uint32_t epoch,
+    const int64_t* __restrict__ pred_new, int64_t root, int64_t* __restrict__ pred,
+    uint32_t snap_level, const LevelSync* ls, uint32_t snap_code) {
   if (!snapshot_is(ls, snap_code)) return;
-  const XcdSpan xs = xcd_span(n_core);
-  for (int64_t i = xs.lo + xs.rank * kT + threadIdx.x; i < xs.hi; i += xs.nblk * kT) {
-    const uint2 ov = get_pair(core + i);
-    const int64_t raw = pred_new[ov.y];
-    if (snap_level != 0 && (run_entry(raw, epoch) == -1 ||
-                            (uint32_t)((uint64_t)raw >> 48) >= snap_level))
-      continue;
-    int64_t e = run_entry(raw, epoch);
-    if ((int64_t)ov.x == root) e = root;
-    __builtin_nontemporal_store(e, pred + ov.x);
+  const int lane = lane_id();
+  const uint64_t below = lanemask_lt();
+  const int64_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const XcdSpan xs = xcd_span(ceil_div(n, (int64_t)64));
+  for (int64_t w0 = xs.lo + (xs.rank * kWavesPerBlock + wave) * kGatherWords; w0 < xs.hi;
+       w0 += xs.nblk * kWavesPerBlock * kGatherWords) {
+    bool has[kGatherWords];
+    uint32_t v[kGatherWords];
+    int64_t raw[kGatherWords];
+#pragma unroll
+    for (int j = 0; j < kGatherWords; ++j) {
+      const uint64_t b = w0 + j < xs.hi ? bits[w0 + j] : 0ull;
+      const uint64_t o = w0 + j < xs.hi ? off[w0 + j] : 0ull;
+      has[j] = (b >> lane) & 1ull;
+      v[j] = has[j] ? __builtin_nontemporal_load(core + o + __popcll(b & below)) : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kGatherWords; ++j) raw[j] = has[j] ? pred_new[v[j]] : -1;
+#pragma unroll
+    for (int j = 0; j < kGatherWords; ++j) {
+      const int64_t o = (w0 + j) * 64 + lane;
+      int64_t e = has[j] ? run_entry(raw[j], epoch) : (int64_t)-1;
+      const bool outside = has[j] && (e == -1 || (uint32_t)((uint64_t)raw[j] >> 48) >= snap_level);
+      if (w0 + j >= xs.hi || o >= n || (snap_level != 0 && outside)) continue;
+      if (o == root) e = root;
+      __builtin_nontemporal_store(e, pred + o);
+    }
   }
 }
 
-__global__ __launch_bounds__(kT) void k_core_flags(const uint32_t* __restrict__ o2n, int64_t n,
-                                                  int64_t n_c, uint32_t* __restrict__ flag) {
+// bits, and per word the number of vertices with edges in it
+__global__ __launch_bounds__(kT) void k_core_bits(const uint32_t* __restrict__ o2n, int64_t n,
+                                                 int64_t n_c, uint64_t* __restrict__ bits,
+                                                 uint32_t* __restrict__ cnt) {
   const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (o < n) flag[o] = (int64_t)o2n[o] < n_c ? 1u : 0u;
+  const uint64_t b = __ballot(o < n && (int64_t)o2n[o] < n_c);
+  if (lane_id() == 0 && o < n) {
+    bits[o >> 6] = b;
+    cnt[o >> 6] = (uint32_t)__popcll(b);
+  }
 }
 
-__global__ __launch_bounds__(kT) void k_core_list(const uint32_t* __restrict__ flag,
+__global__ __launch_bounds__(kT) void k_core_list(const uint64_t* __restrict__ bits,
                                                  const uint64_t* __restrict__ off,
                                                  const uint32_t* __restrict__ o2n, int64_t n,
-                                                 uint2* __restrict__ core) {
+                                                 uint32_t* __restrict__ core) {
   const int64_t o = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (o < n && flag[o]) core[off[o]] = make_uint2((uint32_t)o, o2n[o]);
+  if (o >= n) return;
+  const uint64_t b = bits[o >> 6];
+  if ((b >> lane_id()) & 1ull) core[off[o >> 6] + __popcll(b & lanemask_lt())] = o2n[o];
 }
 
 // pred entries of the vertices outside the snapshot the early gather used:
@@ -1778,21 +1809,23 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
     // the core's original IDs in ascending order; pred starts at -1, which
     // the vertices without edges keep
     hipStream_t s = b->stream;
-    DevBuf<uint32_t> flag;
-    DevBuf<uint64_t> off;
-    flag.alloc((size_t)g->n);
-    off.alloc((size_t)g->n + 1);
-    hipLaunchKernelGGL(k_core_flags, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, s,
-                       g->orig2new.get(), g->n, g->n_c, flag.get());
+    const int64_t owords = ceil_div(g->n, 64);
+    DevBuf<uint32_t> cnt;
+    cnt.alloc_raw((size_t)owords);
+    b->core_bits.alloc_raw((size_t)owords);
+    b->core_off.alloc_raw((size_t)owords + 1);
+    hipLaunchKernelGGL(k_core_bits, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, s,
+                       g->orig2new.get(), g->n, g->n_c, b->core_bits.get(), cnt.get());
     G500_CHECK_LAUNCH();
     ScanWorkspace ws;
-    exclusive_scan<uint32_t>(flag.get(), off.get(), g->n, ws, s);
-    b->core.alloc((size_t)g->n_c);
+    exclusive_scan<uint32_t>(cnt.get(), b->core_off.get(), owords, ws, s);
+    b->core.alloc_raw((size_t)g->n_c);
     hipLaunchKernelGGL(k_core_list, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, s,
-                       flag.get(), off.get(), g->orig2new.get(), g->n, b->core.get());
+                       b->core_bits.get(), b->core_off.get(), g->orig2new.get(), g->n,
+                       b->core.get());
     G500_CHECK_LAUNCH();
     uint64_t total = 0;
-    G500_CHECK_HIP(hipMemcpyAsync(&total, off.get() + g->n, sizeof(total),
+    G500_CHECK_HIP(hipMemcpyAsync(&total, b->core_off.get() + owords, sizeof(total),
                                   hipMemcpyDeviceToHost, s));
     G500_CHECK_HIP(hipStreamSynchronize(s));
     if ((int64_t)total != g->n_c)
@@ -1872,9 +1905,10 @@ void launch_gather(g500_bfs* b, int64_t root, hipStream_t st, uint32_t snap_code
     return (unsigned)std::min<int64_t>(ceil_div(ceil_div(items, kT), kXcds) * kXcds, 65536);
   };
   if (b->n_core > 0)
-    hipLaunchKernelGGL(k_pred_gather_core, dim3(grid(b->n_core)), dim3(kT), 0, st,
-                       b->core.get(), b->n_core, b->epoch, b->pred_new.get(), root,
-                       b->pred.get(), snap_level, b->lsync.get(), snap_code);
+    hipLaunchKernelGGL(k_pred_gather_core, dim3(grid(ceil_div(g->n, kGatherWords))), dim3(kT), 0,
+                       st, b->core_bits.get(), b->core_off.get(), b->core.get(), g->n, b->epoch,
+                       b->pred_new.get(), root, b->pred.get(), snap_level, b->lsync.get(),
+                       snap_code);
   else
     hipLaunchKernelGGL(k_pred_gather, dim3(grid(g->n)),
                        dim3(kT), 0, st, g->orig2new.get(), b->epoch, b->pred_new.get(), g->n,
@@ -2522,10 +2556,12 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   // the steps still queued (guesses past the last level) return at once
   if (b->vis.get() != cur.vis) b->vis.swap(b->vis_alt);
   if (b->q.get() != cur.q) b->q.swap(b->nq);
-  // the gather: per vertex with edges its original ID, new ID, entry read and
-  // written; with CoreBFS every original ID (new ID and entry written) and
-  // every vertex with edges' entry
-  int64_t gather_bytes = b->n_core > 0 ? 24 * b->n_core : 12 * g->n + 8 * n_c;
+  // the gather: per vertex with edges its new ID and entry read, per 64
+  // original IDs two words, per original ID the entry written; with CoreBFS
+  // every original ID (new ID and entry written) and every vertex with edges'
+  // entry
+  int64_t gather_bytes =
+      b->n_core > 0 ? 12 * b->n_core + g->n / 4 + 8 * g->n : 12 * g->n + 8 * n_c;
   const bool disjoint = early_gather && disjoint_fixup(b);
   if (early_gather) {
     // unless the guessed fixup followed the step that ended the run

@@ -128,9 +128,11 @@ struct g500_bfs {
   g500::DevBuf<unsigned int> tickets;  // blocks done in a step's last kernel (see last_of)
   g500::DevBuf<uint32_t> qcnt;    // per-wave counts of the bitmap -> queue conversion
   g500::DevBuf<uint64_t> qedges;  // its per-block degree sums
-  // without CoreBFS: (original ID, new ID) of the vertices with edges, in
-  // ascending original ID (the gather's domain; every other pred entry stays -1)
-  g500::DevBuf<uint2> core;
+  // without CoreBFS: the original IDs with edges as bits, their number before
+  // each word of these, and the new ID of each in ascending original ID (every
+  // other pred entry stays -1)
+  g500::DevBuf<uint64_t> core_bits, core_off;
+  g500::DevBuf<uint32_t> core;
   int64_t n_core = 0;
   int64_t iso_root = -1;  // a root without edges whose entry the last run wrote
   uint32_t epoch = 0;     // the run's epoch in bits 32-47 of its pred_new entries
