@@ -1319,10 +1319,15 @@ __device__ inline int64_t run_entry(int64_t e, uint32_t epoch) {
                                                      : (int64_t)-1;
 }
 
-// A gather queued on a guess that a conversion runs (snap_code != 0) returns
-// at once unless that conversion wrote the bitmap snapshot.
-__device__ inline bool snapshot_is(const LevelSync* ls, uint32_t snap_code) {
-  return snap_code == 0 || __builtin_amdgcn_readfirstlane(ls->snap_tag) == snap_code;
+// A gather queued on a guess returns at once unless the guess holds: that a
+// conversion runs (snap_code != 0: it wrote the bitmap snapshot) or that the
+// run ends (done_code != 0: the loop state says so).
+struct GatherGuess {
+  uint32_t snap_code, done_code;
+};
+__device__ inline bool guess_holds(const LevelSync* ls, const GatherGuess& g) {
+  return (g.snap_code == 0 || __builtin_amdgcn_readfirstlane(ls->snap_tag) == g.snap_code) &&
+         (g.done_code == 0 || step_is_next(ls, g.done_code));
 }
 
 __global__ __launch_bounds__(kT) void k_pred_gather(const uint32_t* __restrict__ o2n,
@@ -1332,8 +1337,8 @@ __global__ __launch_bounds__(kT) void k_pred_gather(const uint32_t* __restrict__
                                                    const uint32_t* __restrict__ tree_parent,
                                                    const uint64_t* __restrict__ has_parent,
                                                    int64_t* __restrict__ pred,
-                                                   const LevelSync* ls, uint32_t snap_code) {
-  if (!snapshot_is(ls, snap_code)) return;
+                                                   const LevelSync* ls, GatherGuess guess) {
+  if (!guess_holds(ls, guess)) return;
   const XcdSpan xs = xcd_span(n);
   for (int64_t o = xs.lo + xs.rank * kT + threadIdx.x; o < xs.hi; o += xs.nblk * kT) {
     const uint32_t v = o2n[o];
@@ -1371,8 +1376,8 @@ __global__ __launch_bounds__(kT) void k_pred_gather_core(
     const uint64_t* __restrict__ bits, const uint64_t* __restrict__ off,
     const uint32_t* __restrict__ core, int64_t n, uint32_t epoch,
     const int64_t* __restrict__ pred_new, int64_t root, int64_t* __restrict__ pred,
-    uint32_t snap_level, const LevelSync* ls, uint32_t snap_code) {
-  if (!snapshot_is(ls, snap_code)) return;
+    uint32_t snap_level, const LevelSync* ls, GatherGuess guess) {
+  if (!guess_holds(ls, guess)) return;
   const int lane = lane_id();
   const uint64_t below = lanemask_lt();
   const int64_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -1735,6 +1740,14 @@ __global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t roo
                          : (int64_t)(((uint64_t)lev[v] << 48) | (uint64_t)g.n2o[par[v]]);
 }
 
+// Graphs from this many vertices on have their gather run beside the last
+// top-down levels, on a second stream; smaller ones have it follow them.  The
+// gather itself takes 4 us at SCALE 18 and 20 at SCALE 22, the hand-offs to the
+// other stream and back ~20: a run at SCALE 15 / 18 / 20 / 22 / 23 / 24 takes
+// 153 / 180 / 220 / 304 / 366 / 462 us with the second stream and 133 / 166 /
+// 210 / 297 / 365 / 473 without.
+constexpr int64_t kOverlapVerts = 1 << 23;
+
 unsigned grid_for(int64_t work_items, int64_t per_block) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ceil_div(work_items, per_block)));
 }
@@ -1802,7 +1815,8 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   G500_CHECK_HIP(hipEventCreateWithFlags(&b->ev_g0, hipEventDisableSystemFence));
   G500_CHECK_HIP(hipEventCreate(&b->ev_g1));
   G500_CHECK_HIP(hipStreamCreate(&b->gstream));
-  b->vis_snap.alloc((size_t)b->words);
+  b->overlap_gather = g->n >= kOverlapVerts;
+  if (b->overlap_gather) b->vis_snap.alloc((size_t)b->words);
   b->qcnt.alloc((size_t)kQueueGrid * kWavesPerBlock);
   b->qedges.alloc((size_t)kQueueGrid);
   if (!g->corebfs && g->n_c > 0) {
@@ -1894,9 +1908,9 @@ void wait_report(g500_bfs* b, unsigned long long seq, unsigned long long out[4])
 
 // pred by original ID from this run's level entries (a smaller grid beside
 // the last top-down levels measured slower: the random reads need every
-// wave the chip holds).  snap_code != 0: queued before the conversion of
-// that code is known to run (the kernel checks).
-void launch_gather(g500_bfs* b, int64_t root, hipStream_t st, uint32_t snap_code,
+// wave the chip holds).  A code in `guess`: queued before that conversion is
+// known to run, or the run to have ended (the kernel checks).
+void launch_gather(g500_bfs* b, int64_t root, hipStream_t st, GatherGuess guess,
                    uint32_t snap_level) {
   g500_graph* g = b->g;
   G500_CHECK_HIP(hipEventRecord(b->ev_g0, st));
@@ -1908,13 +1922,13 @@ void launch_gather(g500_bfs* b, int64_t root, hipStream_t st, uint32_t snap_code
     hipLaunchKernelGGL(k_pred_gather_core, dim3(grid(ceil_div(g->n, kGatherWords))), dim3(kT), 0,
                        st, b->core_bits.get(), b->core_off.get(), b->core.get(), g->n, b->epoch,
                        b->pred_new.get(), root, b->pred.get(), snap_level, b->lsync.get(),
-                       snap_code);
+                       guess);
   else
     hipLaunchKernelGGL(k_pred_gather, dim3(grid(g->n)),
                        dim3(kT), 0, st, g->orig2new.get(), b->epoch, b->pred_new.get(), g->n,
                        g->n_c, root, g->corebfs ? g->tree_parent.get() : nullptr,
                        g->corebfs ? g->has_parent.get() : nullptr, b->pred.get(),
-                       b->lsync.get(), snap_code);
+                       b->lsync.get(), guess);
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipEventRecord(b->ev_g1, st));
   if (st != b->stream) b->gather_pending = true;
@@ -2048,7 +2062,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       st.after.vis_alt = in.vis;
       break;
     case kModeConv:
-      to_queue(in.vis, in.vis_alt, in.q, b->vis_snap.get());
+      to_queue(in.vis, in.vis_alt, in.q, b->overlap_gather ? b->vis_snap.get() : nullptr);
       break;
     default:
       fail(G500_ERR_STATE, "no step of mode %u", mode);
@@ -2152,15 +2166,15 @@ uint32_t predict_next(const Step& last, HostLoop hl, const std::vector<g500_leve
 }
 
 // The end of a run queued on guesses: the pred gather behind a guessed
-// conversion (k_pred_gather* checks that the conversion ran) and the fixup
-// behind the step guessed to be the last (k_pred_fixup checks that the loop
-// ended there).
+// conversion (k_pred_gather* checks that the conversion ran) and the fixup --
+// on graphs below kOverlapVerts the gather itself -- behind the step guessed
+// to be the last (the kernel checks that the loop ended there).
 struct EndGuess {
   int64_t root = 0;
   bool gather_confirmed = false;     // a gather follows the conversion that ran
   unsigned long long conv_seq = 0;   // the guessed conversion the last guessed gather follows
-  unsigned long long fixup_seq = 0;  // the step the guessed fixup follows
-  uint32_t fixup_code = 0;           // the final code it waits for
+  unsigned long long end_seq = 0;    // the step the guessed fixup or gather follows
+  uint32_t end_code = 0;             // the final code it waits for
 };
 
 // The engine stream waits until every gather queued so far has ended.
@@ -2182,7 +2196,7 @@ bool disjoint_fixup(const g500_bfs* b) { return b->n_core > 0; }
 // it, is what the engine stream waits on.
 void queue_gather(g500_bfs* b, int64_t root, uint32_t snap_code, uint32_t conv_code) {
   G500_CHECK_HIP(hipStreamWaitEvent(b->gstream, b->ev_snap, 0));
-  launch_gather(b, root, b->gstream, snap_code,
+  launch_gather(b, root, b->gstream, GatherGuess{snap_code, 0},
                 disjoint_fixup(b) ? (uint32_t)step_level(conv_code) : 0u);
 }
 
@@ -2238,10 +2252,11 @@ void speculate(g500_bfs* b, std::deque<Step>& pend, const HostLoop& hl, size_t d
     uint32_t next = predict_next(last, h, tr);
     if (b->guess_wrong) next = wrong_guess(next);
     if (step_mode(next) == kModeDone) {
-      if (eg->gather_confirmed && eg->fixup_seq != last.seq) {
-        queue_fixup(b, last.after.vis, next);
-        eg->fixup_seq = last.seq;
-        eg->fixup_code = next;
+      if ((eg->gather_confirmed || !b->overlap_gather) && eg->end_seq != last.seq) {
+        if (b->overlap_gather) queue_fixup(b, last.after.vis, next);
+        else launch_gather(b, eg->root, b->stream, GatherGuess{0, next}, 0u);
+        eg->end_seq = last.seq;
+        eg->end_code = next;
       }
       return;
     }
@@ -2256,7 +2271,7 @@ void speculate(g500_bfs* b, std::deque<Step>& pend, const HostLoop& hl, size_t d
       tr.push_back(t);
     }
     pend.push_back(launch_step(b, next, last.after, nlev_ev, nsweep_ev));
-    if (step_mode(next) == kModeConv && !eg->gather_confirmed) {
+    if (step_mode(next) == kModeConv && !eg->gather_confirmed && b->overlap_gather) {
       // ev_snap was just recorded behind this conversion's snapshot
       queue_gather(b, eg->root, next, next);
       eg->conv_seq = pend.back().seq;
@@ -2540,7 +2555,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
       pend.clear();
       pend.push_back(launch_step(b, next, cur, &nlev_ev, &nsweep_ev));
     }
-    if (step_mode(next) == kModeConv) {
+    if (step_mode(next) == kModeConv && b->overlap_gather) {
       // switching to top-down: the remaining top-down levels are short and
       // latency-bound, so the pred gather of every vertex reached so far
       // starts on the second stream once the conversion has written the
@@ -2565,7 +2580,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   const bool disjoint = early_gather && disjoint_fixup(b);
   if (early_gather) {
     // unless the guessed fixup followed the step that ended the run
-    if (!(eg.fixup_seq == ran.back().seq && eg.fixup_code == final_code))
+    if (!(eg.end_seq == ran.back().seq && eg.end_code == final_code))
       queue_fixup(b, b->vis.get(), 0);
     // both bitmaps; per vertex its new -> original ID, entry read and written
     alg += 16 * words + 20 * after_snap;
@@ -2576,8 +2591,8 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
       alg += 12 * unreached;
       gather_bytes -= 8 * (after_snap + unreached);
     }
-  } else {
-    launch_gather(b, root, s, 0, 0u);
+  } else if (!(eg.end_seq == ran.back().seq && eg.end_code == final_code)) {
+    launch_gather(b, root, s, GatherGuess{0, 0}, 0u);
   }
   alg += gather_bytes;
   if (b->n_core > 0) {

@@ -116,6 +116,7 @@ struct g500_bfs {
   // the pred gather of the vertices reached by the last bottom-up level runs
   // on gstream during the remaining top-down levels; vis_snap is the bitmap
   // it covers (copied by the conversion's count pass), the fixup adds the rest
+  bool overlap_gather = false;  // (large graphs only; else the gather ends the run)
   hipStream_t gstream = nullptr;
   g500::DevBuf<uint64_t> vis_snap;
   // ev_snap follows the last conversion's count pass (the gather waits on

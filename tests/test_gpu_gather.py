@@ -44,3 +44,30 @@ def test_pred_of_a_path(n, step):
 def g_pred(b, root):
     b.run(root)
     return b.pred()
+
+
+@pytest.mark.parametrize("guess", ["", "wrong"])
+@pytest.mark.parametrize("corebfs", [False, True])
+@pytest.mark.parametrize("stride", [1, 64, 128, 129])  # vertices: 2^16, 2^22, 2^23, over 2^23
+def test_gather_beside_and_behind_the_levels(stride, corebfs, guess, monkeypatch):
+    """The same tree whether the gather runs beside the last levels (large graphs) or ends the
+    run."""
+    if guess:
+        monkeypatch.setenv("G500_GUESS", guess)
+    small = G.Graph.generate(16)
+    v0, v1 = small.edges()
+    g = G.Graph.from_edges(v0 * stride, v1 * stride).construct(corebfs=corebfs)
+    small.construct(corebfs=corebfs)
+    b, ref = G.Bfs(g), G.Bfs(small)
+    for root in small.find_roots(4):
+        ref.run(int(root))
+        for _ in range(2):
+            b.run(int(root) * stride)
+            levels = b.levels()
+            np.testing.assert_array_equal(levels[:stride << 16:stride], ref.levels())
+            assert (np.delete(levels, np.s_[:stride << 16:stride]) == 0xFFFF).all()
+            assert b.validate(int(root) * stride)[0]
+    for x in (b, ref):
+        x.destroy()
+    for x in (g, small):
+        x.free()
