@@ -87,6 +87,11 @@ __host__ __device__ inline uint32_t td_step_mode(long long qlen, long long qedge
   return qedges > exec_thr ? kModeTDX : (qlen <= kTdWin ? kModeTDS : kModeTD);
 }
 
+// A bottom-up level over the unvisited lists, by the vertices left in them.
+__host__ __device__ inline uint32_t list_mode(long long left, long long rest_thr) {
+  return left < rest_thr ? kModeBURest : kModeBUList;
+}
+
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -184,6 +189,8 @@ __device__ inline uint32_t decide_next(const LevelSync& cur, LevelSync* ls, uint
     }
     ls->growing = growing ? 1u : 0u;
     ls->prev_nq = nq_size;
+    const long long left = cur.left - nq_size;
+    ls->left = left;
     if (td && next_td) {
       next = td_step_mode(nq_size, nq_edges, cur.exec_thr);
       Frontier& f = next_frontier(ls, code);
@@ -192,9 +199,9 @@ __device__ inline uint32_t decide_next(const LevelSync& cur, LevelSync* ls, uint
     } else if (td) {
       // a top-down expansion leaves the unvisited lists behind, a sweep
       // (also one that ran a top-down level) refreshes them
-      next = mode == kModeTDX ? kModeBUList : kModeBUSweep;
+      next = mode == kModeTDX ? list_mode(left, cur.rest_thr) : kModeBUSweep;
     } else {
-      next = next_td ? kModeConv : kModeBUList;
+      next = next_td ? kModeConv : list_mode(left, cur.rest_thr);
     }
   }
   const uint32_t nc = step_code(step_level(code) + 1, next);
@@ -280,7 +287,7 @@ __device__ inline void close_level(const uint64_t* part, int n, bool top_down, L
 // first frontier's degree sum is the root's row length, set on the device).
 struct LoopInit {
   uint32_t first;  // code of the first step
-  long long qlen, qedges, alpha_thr, beta_thr, exec_thr;
+  long long qlen, qedges, alpha_thr, beta_thr, exec_thr, left, rest_thr;
 };
 
 // Bits of vertices >= n_c are pre-set so they are never searched
@@ -321,6 +328,8 @@ __global__ __launch_bounds__(kT) void k_bfs_init(uint64_t* __restrict__ vis,
     ls->alpha_thr = li.alpha_thr;
     ls->beta_thr = li.beta_thr;
     ls->exec_thr = li.exec_thr;
+    ls->left = li.left;
+    ls->rest_thr = li.rest_thr;
     ls->snap_tag = 0;
     if (root_new >= 0 && root_new < n_c) {
       pred_new[root_new] = entry;
@@ -1157,6 +1166,134 @@ __global__ __launch_bounds__(kBuT) __attribute__((amdgpu_waves_per_eu(4))) void 
     close_level(cpart, (int)gridDim.x, false, ls, cl, code, red);
 }
 
+// A list level with few vertices left: a wave takes the entries of up to 64
+// chunks together, a lane per entry, and reads the visited bits from memory.
+// What remains after the first list level lies mostly in other components, one
+// or two vertices a chunk, and chunk by chunk such a level was a chain of four
+// or five dependent reads per chunk behind the copy of the hub bits: 30 us at
+// SCALE 26, 21 at 24, 11.5 at 18; here 15.6, 11.3 and 7.6.  Levels of more than
+// one vertex in kRestShare (the first after a sweep: a tenth to a third of
+// all) stay with k_bu_list, whose batches keep eight a lane in flight.
+// A branch in k_bu_list instead cost its full levels 4 % in spills.
+constexpr int64_t kRestShare = 64;
+
+__global__ __launch_bounds__(kBuT) void k_bu_rest(
+    const uint64_t* __restrict__ vis_old, unsigned long long* vis_new, int64_t words, int cw,
+    const int64_t* __restrict__ row_off, const uint32_t* __restrict__ col,
+    const uint2* __restrict__ first, const uint64_t* __restrict__ multi,
+    const uint32_t* __restrict__ n2o, int64_t* __restrict__ pred_new, uint32_t* __restrict__ unv,
+    uint32_t* __restrict__ unv_cnt, LevelSync* ls, uint32_t code, uint64_t* __restrict__ cpart,
+    uint64_t level_bits, uint64_t* __restrict__ wacc, Closing cl) {
+  if (!step_is_next(ls, code)) return;
+  __shared__ uint64_t red[kBuWaves];
+  const int lane = lane_id(), wave = threadIdx.x / kWave;
+  const int64_t nchunks = ceil_div(words, cw);
+  const uint32_t cverts = (uint32_t)cw * 64u;
+  const bool count = wacc != nullptr;
+  const uint64_t below = lanemask_lt();
+  uint64_t nfound = 0, scan_b = 0;
+  auto visited = [&](uint32_t u) { return (vis_old[u >> 6] >> (u & 63)) & 1ull; };
+  // the wave's chunks are c0, c0 + step, ..., 64 of them at a time
+  const int64_t step = (int64_t)gridDim.x * kBuWaves;
+  for (int64_t c0 = (int64_t)blockIdx.x * kBuWaves + wave; c0 < nchunks; c0 += kWave * step) {
+    const int chunks = (int)min(ceil_div(nchunks - c0, step), (int64_t)kWave);
+    const uint32_t held = lane < chunks ? unv_cnt[c0 + lane * step] : 0u;  // lane l: the l-th's
+    uint32_t kept = 0;                                                     // misses among them
+    // the new bitmap's words first; the found bits are added to them
+    constexpr int kIlp = 4;
+    for (int k0 = 0; k0 < chunks; k0 += kIlp) {
+      uint64_t word[kIlp];
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j) {
+        const int64_t w = (c0 + (k0 + j) * step) * cw + lane;
+        word[j] = k0 + j < chunks && lane < cw && w < words ? vis_old[w] : 0ull;
+      }
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j) {
+        const int64_t w = (c0 + (k0 + j) * step) * cw + lane;
+        if (k0 + j < chunks && lane < cw && w < words) vis_new[w] = word[j];
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they arrive before the atomics below
+    uint32_t total = held;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, kWave);
+    for (uint32_t e0 = 0; e0 < total; e0 += kWave) {
+      int mine = -1;  // the lane's chunk and its entry there
+      uint32_t idx = 0, run = 0;
+      for (int k = 0; k < chunks; ++k) {
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)held, k), e = e0 + lane;
+        if (e >= run && e < run + n) {
+          mine = k;
+          idx = e - run;
+        }
+        run += n;
+      }
+      const int64_t c = c0 + (mine < 0 ? 0 : mine) * step;
+      uint32_t v = 0, par = 0;
+      bool hit = false;
+      if (mine >= 0) {
+        v = unv[c * cverts + idx];
+        const uint2 f = get_pair(first + v);
+        const bool more = multi_bit(multi, v);
+        hit = visited(f.x);
+        par = f.y;
+        if (!hit && more) {
+          int64_t k = row_off[v] + 1;
+          const int64_t k1 = row_off[v + 1];
+          if (count) scan_b += 16;
+          while (!hit && k < k1) {
+            uint32_t u[4];
+            bool h[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) u[t] = k + t < k1 ? col[k + t] : 0u;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) h[t] = k + t < k1 && visited(u[t]);
+            int used = (int)min<int64_t>(4, k1 - k);
+#pragma unroll
+            for (int t = 3; t >= 0; --t)
+              if (h[t]) {
+                hit = true;
+                par = u[t];
+                used = t + 1;
+              }
+            if (count) scan_b += 4u * (uint64_t)used + (hit ? 4u : 0u);
+            k += 4;
+          }
+          if (hit) par = n2o[par];
+        }
+        if (hit) {
+          put_pred(pred_new + v, (uint64_t)par | level_bits);
+          atomicOr(vis_new + (v >> 6), 1ull << (v & 63));
+          ++nfound;
+        }
+        if (count) scan_b += hit ? 8u : 4u;
+      }
+      // a round's misses go where earlier rounds' ended, never past an entry
+      // not yet read: all of the round's entries are in registers
+      const bool miss = mine >= 0 && !hit;
+      uint64_t open = __ballot(miss);
+      while (open) {
+        const int k = __builtin_amdgcn_readlane(mine, __ffsll((long long)open) - 1);
+        const uint64_t m = __ballot(miss && mine == k);
+        const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)kept, k);
+        if (miss && mine == k) unv[c * cverts + base + (uint32_t)__popcll(m & below)] = v;
+        if (lane == k) kept += (uint32_t)__popcll(m);
+        open &= ~m;
+      }
+    }
+    if (lane < chunks && held) unv_cnt[c0 + lane * step] = kept;
+  }
+  const uint64_t s = block_sum<kBuWaves>(nfound, red);
+  if (count) {
+    __syncthreads();
+    const uint64_t sb = block_sum<kBuWaves>(scan_b, red);
+    if (threadIdx.x == 0) wacc[blockIdx.x] += sb;
+  }
+  if (last_of(cl, gridDim.x, cpart + blockIdx.x, s))
+    close_level(cpart, (int)gridDim.x, false, ls, cl, code, red);
+}
+
 // queue <- bits set in cur but not in prev; reports (count, degree sum).
 // Two launches over one partition of the words: block b owns a contiguous
 // range and each of its waves a contiguous quarter of it.  k_queue_count
@@ -1537,6 +1674,8 @@ __global__ __launch_bounds__(kSmallT) void k_bfs_small(SmallGraph g, int64_t roo
     ls.alpha_thr = li.alpha_thr;
     ls.beta_thr = li.beta_thr;
     ls.exec_thr = li.exec_thr;
+    ls.left = li.left;
+    ls.rest_thr = li.rest_thr;
   }
   __syncthreads();
   // two block sums, valid in thread 0
@@ -2061,6 +2200,16 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       st.after.vis = in.vis_alt;
       st.after.vis_alt = in.vis;
       break;
+    case kModeBURest:
+      hipLaunchKernelGGL(k_bu_rest, dim3(b->bu_grid[1]), dim3(kBuT), 0, s, in.vis,
+                         (unsigned long long*)in.vis_alt, b->words, b->chunk_words,
+                         g->row_off.get(), g->col.get(), g->first.get(), g->multi.get(),
+                         g->new2orig.get(), b->pred_new.get(), b->unv.get(), b->unv_cnt.get(), ls,
+                         code, b->lpart.get(), level_bits, wlist, cl);
+      G500_CHECK_LAUNCH();
+      st.after.vis = in.vis_alt;
+      st.after.vis_alt = in.vis;
+      break;
     case kModeConv:
       to_queue(in.vis, in.vis_alt, in.q, b->overlap_gather ? b->vis_snap.get() : nullptr);
       break;
@@ -2078,7 +2227,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
 struct HostLoop {
   bool growing = true;
   int64_t prev_nq = 0;
-  int64_t alpha_thr = 0, beta_thr = 0, exec_thr = 0;
+  int64_t alpha_thr = 0, beta_thr = 0, exec_thr = 0, rest_thr = 0;
   int64_t n_c = 0, m = 0;
   // for the guesses: vertices with edges reached so far, and how many of
   // them the engine's previous run left unreached (other components)
@@ -2117,8 +2266,8 @@ struct HostLoop {
     prev_nq = nq_size;
     uint32_t next;
     if (td && next_td) next = td_step_mode(nq_size, nq_edges, exec_thr);
-    else if (td) next = mode == kModeTDX ? kModeBUList : kModeBUSweep;
-    else next = next_td ? kModeConv : kModeBUList;
+    else if (td) next = mode == kModeTDX ? list_mode(n_c - visited, rest_thr) : kModeBUSweep;
+    else next = next_td ? kModeConv : list_mode(n_c - visited, rest_thr);
     return step_code(level + 1, next);
   }
 };
@@ -2162,7 +2311,12 @@ uint32_t predict_next(const Step& last, HostLoop hl, const std::vector<g500_leve
                      td_step_mode(tr.empty() ? 0 : tr.back().nq_size, 0, hl.exec_thr));
   int64_t nq, fe, at[G500_AT_NUM];
   estimate_level(mode, tr, hl, &nq, &fe);
-  return hl.after_level(last.code, nq, fe, at);
+  const uint32_t next = hl.after_level(last.code, nq, fe, at);
+  // the first list level finds nearly all that its component has left (the
+  // estimate stays below that: it must not take the run to be over)
+  if (step_mode(next) == kModeBUList && mode == kModeBUList)
+    return step_code(step_level(next), kModeBURest);
+  return next;
 }
 
 // The end of a run queued on guesses: the pred gather behind a guessed
@@ -2220,6 +2374,7 @@ uint32_t wrong_guess(uint32_t code) {
     case kModeDone: return step_code(l, kModeTD);
     case kModeConv: return step_code(l, kModeBUList);
     case kModeBUList:
+    case kModeBURest:
     case kModeBUSweep: return step_code(l, kModeConv);
     default: return step_code(l, kModeDone);
   }
@@ -2448,10 +2603,12 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   hl.beta_thr = (int64_t)((double)n_c / (beta * edgefactor * 2.0));
   hl.exec_thr = b->exec_alpha > 0 ? (int64_t)std::floor((double)g->m / b->exec_alpha)
                                   : INT64_MAX;
+  hl.rest_thr = n_c / kRestShare;
   hl.visited = root_in ? 1 : 0;
   hl.unreach = b->unreach;
   const uint32_t first = step_code(root_level + 1, kModeTDS);
-  LoopInit li{first, root_in ? 1 : 0, 0, hl.alpha_thr, hl.beta_thr, hl.exec_thr};
+  LoopInit li{first, root_in ? 1 : 0, 0, hl.alpha_thr, hl.beta_thr, hl.exec_thr,
+              n_c - hl.visited, hl.rest_thr};
   if (run_small(b, root, li, hl, at)) return;
   G500_CHECK_HIP(hipEventRecord(b->ev_begin, s));
   hipLaunchKernelGGL(k_bfs_init, dim3(grid_for(words, kT)), dim3(kT), 0, s,
@@ -2521,7 +2678,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
           sweep_host += sw;
           alg += sw;
           if (td) alg += 16 * words + 8 * nq_size;  // bitmap -> queue (queue + degree)
-        } else if (mode == kModeBUList) {
+        } else if (mode == kModeBUList || mode == kModeBURest) {
           // list level: old and new bitmap; a list entry and a pair per listed vertex
           alg += 16 * words + 12 * unvisited;
         } else {

@@ -17,6 +17,7 @@ enum StepMode : uint32_t {
   kModeConv = 5,     // bitmap -> queue at the bottom-up -> top-down switch
   kModeDone = 6,
   kModeTDS = 7,      // top-down, small frontier staged by the expansion itself
+  kModeBURest = 8,   // bottom-up over the unvisited lists, few vertices left in them
 };
 __host__ __device__ inline bool mode_is_td(uint32_t m) {
   return m == kModeTD || m == kModeTDS || m == kModeTDX;
@@ -46,6 +47,8 @@ struct LevelSync {
     long long qedges;  // its degree sum (>= its CSR entries)
   } front[2];
   long long prev_nq;   // frontier size of the previous level
+  long long left;      // vertices with edges not reached yet
+  long long rest_thr;  // a list level of fewer runs as kModeBURest
   long long alpha_thr, beta_thr, exec_thr;  // int64(m/alpha), int64(n_c/(beta*ef*2)), m/exec_alpha
   uint32_t snap_tag;   // code of the conversion that wrote the gather's bitmap snapshot (0: none)
 };
