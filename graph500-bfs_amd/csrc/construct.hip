@@ -265,9 +265,10 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
 
 }  // namespace
 
-void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
+void build_csr(g500_graph* g, const uint2* edges, int64_t ne, DegreeMode mode,
                int force_log_n) {
   hipStream_t s = g->stream;
+  const bool symmetric = mode != DegreeMode::kBothEnds;
   const int64_t nv = (int64_t)1 << g->id_bits;  // covers every input ID
 
   DevBuf<unsigned long long> stats;
@@ -277,8 +278,7 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
   deg.alloc_raw((size_t)nv);
   G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, nv * sizeof(uint32_t), s));
   if (ne > 0)
-    count_degrees(edges, ne, symmetric ? DegreeMode::kSourceNoLoops : DegreeMode::kBothEnds, nv,
-                  deg.get(), stats.get(), s);
+    count_degrees(edges, ne, mode, nv, deg.get(), stats.get(), s);
   {
     const int64_t blocks = std::min<int64_t>(ceil_div(nv, kT * 8), 1024);
     hipLaunchKernelGGL(k_deg_stats, dim3((unsigned)blocks), dim3(kT), 0, s,
@@ -341,7 +341,8 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
 }
 
 void construct_graph(g500_graph* g, int corebfs) {
-  build_csr(g, g->edges.get(), g->nedges, g->symmetric_input, -1);
+  build_csr(g, g->edges.get(), g->nedges,
+            g->symmetric_input ? DegreeMode::kSourceNoLoops : DegreeMode::kBothEnds, -1);
   g->corebfs = corebfs;
   g->constructed = true;
 }

