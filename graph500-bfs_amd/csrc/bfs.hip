@@ -229,29 +229,38 @@ struct Closing {
   unsigned long long seq;
 };
 
+// A block's total, for the block that comes last; thread 0.
+__device__ inline void leave_total(uint64_t* slot, uint64_t total) {
+  __hip_atomic_store(slot, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // True (in all threads) in the last of `blocks` blocks (blockIdx < blocks)
-// to come here; thread 0 stores the block's total in *slot first.  Its own
-// earlier atomics returned their results, so they are complete.
-__device__ inline bool last_of(const Closing& cl, unsigned blocks, uint64_t* slot,
-                               uint64_t total) {
+// to come here, once what thread 0 of each left with leave_total has arrived.
+// (Its atomics that returned a result are complete as well.)
+__device__ inline bool comes_last(unsigned int* tickets, unsigned blocks) {
   __shared__ bool last;
   if (threadIdx.x == 0) {
-    __hip_atomic_store(slot, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const unsigned slots = min(blocks, (unsigned)kTicketSlots), mine = blockIdx.x % slots;
     const unsigned members = blocks / slots + (mine < blocks % slots ? 1u : 0u);
-    unsigned int* t = cl.tickets + (1 + mine) * kTicketPad;
+    unsigned int* t = tickets + (1 + mine) * kTicketPad;
     last = false;
     if (atomicAdd(t, 1u) + 1 == members) {
       *t = 0;
-      if (atomicAdd(cl.tickets, 1u) + 1 == slots) {
-        *cl.tickets = 0;
+      if (atomicAdd(tickets, 1u) + 1 == slots) {
+        *tickets = 0;
         last = true;
       }
     }
   }
   __syncthreads();
   return last;
+}
+
+__device__ inline bool last_of(const Closing& cl, unsigned blocks, uint64_t* slot,
+                               uint64_t total) {
+  if (threadIdx.x == 0) leave_total(slot, total);
+  return comes_last(cl.tickets, blocks);
 }
 
 __device__ inline uint64_t sum_slots(const uint64_t* part, int n, uint64_t* red) {
@@ -382,18 +391,23 @@ constexpr int kPrepTile = kT * kPrepItems;
 constexpr int kPrepGrid = 256;
 
 // Block-local prefix sums into dsum, block totals into bsum; the last block
-// to finish (atomic ticket, which it resets) scans the totals into boff.
+// to finish scans the totals into boff.  The totals pass as a step's do
+// (leave_total, comes_last): with a fence in every block the launch took 13 us
+// before the first sweep and 36 beside the gather, whose output the fences
+// wrote back; now 10 and 22.  (SCALE 24: beside the gather this launch is on
+// the run's longest path.)
 __global__ __launch_bounds__(kT) void k_td_prep_sums(
     const uint32_t* __restrict__ q, const LevelSync* ls, uint32_t code,
     const int64_t* __restrict__ row_off, uint64_t* __restrict__ dsum,
-    uint64_t* __restrict__ bsum, uint64_t* __restrict__ boff, unsigned int* ticket) {
+    uint64_t* __restrict__ bsum, uint64_t* __restrict__ boff, unsigned int* tickets) {
   if (!step_is_next(ls, code)) return;
   const int64_t qlen = frontier(ls, code).qlen;
   if (qlen <= kTdWin) return;
   __shared__ uint64_t wsum[kWavesPerBlock];
-  __shared__ bool last;
   const int t = threadIdx.x;
   const int64_t nb = ceil_div(qlen, (int64_t)kPrepTile);
+  const unsigned active = (unsigned)min(nb, (int64_t)gridDim.x);
+  if (blockIdx.x >= active) return;
   for (int64_t blk = blockIdx.x; blk < nb; blk += gridDim.x) {
     const int64_t i0 = blk * kPrepTile + (int64_t)t * kPrepItems;
     uint32_t u[kPrepItems];
@@ -413,30 +427,33 @@ __global__ __launch_bounds__(kT) void k_td_prep_sums(
       if (i0 + j < qlen) dsum[i0 + j] = a;
       a += d[j];
     }
-    if (t == 0) bsum[blk] = tot;
+    if (t == 0) leave_total(bsum + blk, tot);
   }
-  if (t == 0) {
-    __threadfence();
-    last = atomicAdd(ticket, 1u) == gridDim.x - 1;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
+  if (!comes_last(tickets, active)) return;
   uint64_t carry = 0;
   for (int64_t b0 = 0; b0 < nb; b0 += kT) {
-    const uint64_t x = b0 + t < nb ? __atomic_load_n(&bsum[b0 + t], __ATOMIC_RELAXED) : 0;
+    const uint64_t x = b0 + t < nb ? __hip_atomic_load(bsum + b0 + t, __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT)
+                                   : 0;
     uint64_t ctot;
     const uint64_t ex = block_excl_scan(x, wsum, &ctot);
     if (b0 + t < nb) boff[b0 + t] = carry + ex;
     carry += ctot;
   }
-  if (t == 0) {
-    dsum[qlen] = carry;
-    *ticket = 0u;
-  }
+  if (t == 0) dsum[qlen] = carry;
 }
 
-// Adds the block offsets and writes the tile owners.
+__device__ inline uint64_t readlane64(uint64_t x, int l) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l);
+  return ((uint64_t)hi << 32) | lo;
+}
+
+// Adds the block offsets and writes the tile owners: the tiles of a vertex that
+// owns more than kOwnTiles are written by its whole wave.  (By one thread a hub
+// of 10^6 edges held the launch for 500 stores in a row: nine in ten launches
+// within 23 us at SCALE 24 and 34 at 26, now within 12 and 15.)
+constexpr int kOwnTiles = 8;
 __global__ __launch_bounds__(kT) void k_td_prep_tiles(
     const LevelSync* ls, uint32_t code, uint64_t* __restrict__ dsum,
     const uint64_t* __restrict__ bsum, const uint64_t* __restrict__ boff,
@@ -462,13 +479,20 @@ __global__ __launch_bounds__(kT) void k_td_prep_tiles(
 #pragma unroll
     for (int j = 0; j < kPrepItems; ++j) {
       const int64_t i = i0 + j;
-      if (i >= bend) break;
       const uint64_t a = off + loc[j], b = off + loc[j + 1];
-      dsum[i] = a;
-      if (b <= a) continue;
-      const uint64_t t0 = (a + kTdTile - 1) / kTdTile, t1 = (b - 1) / kTdTile;
-      for (uint64_t tt = t0; tt <= t1; ++tt) tile_owner[tt] = (uint32_t)i;
-      if (i == qlen - 1) tile_owner[t1 + 1] = (uint32_t)i;
+      const bool edges = i < bend && b > a;
+      if (i < bend) dsum[i] = a;
+      const uint64_t t0 = (a + kTdTile - 1) / kTdTile, t1 = edges ? (b - 1) / kTdTile : 0;
+      const bool many = edges && t1 >= t0 + kOwnTiles;
+      if (edges && !many)
+        for (uint64_t tt = t0; tt <= t1; ++tt) tile_owner[tt] = (uint32_t)i;
+      if (edges && i == qlen - 1) tile_owner[t1 + 1] = (uint32_t)i;
+      for (uint64_t m = __ballot(many); m; m &= m - 1) {
+        const int l = __ffsll((long long)m) - 1;
+        const uint64_t w0 = readlane64(t0, l), w1 = readlane64(t1, l);
+        const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)i, l);
+        for (uint64_t tt = w0 + lane_id(); tt <= w1; tt += kWave) tile_owner[tt] = o;
+      }
     }
   }
 }
@@ -704,12 +728,6 @@ __device__ inline VisProbe stage_hubs(uint64_t* hub, const uint64_t* vis, int64_
   for (int i = threadIdx.x; i < hw; i += kBuT) hub[i] = vis[i];
   __syncthreads();
   return VisProbe{hub, vis, (uint32_t)hw * 64u};
-}
-
-__device__ inline uint64_t readlane64(uint64_t x, int l) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), l);
-  return ((uint64_t)hi << 32) | lo;
 }
 
 // Rows with more than max_rest entries left are not scanned: long[j] is set
@@ -1910,8 +1928,6 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   b->tile_owner.alloc((size_t)ceil_div(std::max<int64_t>(g->m, 1), kTdTile) + 2);
   b->bsum.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile));
   b->boff.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile));
-  b->prep_ticket.alloc(1);
-  G500_CHECK_HIP(hipMemset(b->prep_ticket.get(), 0, sizeof(unsigned int)));
   // bottom-up grids: what stays resident (each block stages the hub bits
   // once), never more blocks than chunk groups
   int cus = 0, per_cu[3] = {0, 0, 0};
@@ -2170,7 +2186,7 @@ Step launch_step(g500_bfs* b, uint32_t code, const Bufs& in, size_t* nlev_ev,
       if (mode == kModeTD) {
         hipLaunchKernelGGL(k_td_prep_sums, dim3(kPrepGrid), dim3(kT), 0, s, in.q, ls, code,
                            g->row_off.get(), b->dsum.get(), b->bsum.get(), b->boff.get(),
-                           b->prep_ticket.get());
+                           b->tickets.get());
         G500_CHECK_LAUNCH();
         hipLaunchKernelGGL(k_td_prep_tiles, dim3(kPrepGrid), dim3(kT), 0, s, ls, code,
                            b->dsum.get(), b->bsum.get(), b->boff.get(), b->tile_owner.get());

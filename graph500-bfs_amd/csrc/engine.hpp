@@ -89,7 +89,6 @@ struct g500_bfs {
   g500::DevBuf<uint64_t> dsum;      // frontier degree prefix sums
   g500::DevBuf<uint32_t> tile_owner; // frontier index owning each top-down tile's first edge
   g500::DevBuf<uint64_t> bsum, boff;  // per prep block: degree total, its offset
-  g500::DevBuf<unsigned int> prep_ticket;  // blocks done in the prep's first launch
   // unvisited vertices after a bottom-up level: an entry per vertex of each
   // chunk of chunk_words bitmap words, unv_cnt[chunk] of them in use
   int chunk_words = 64;
@@ -129,7 +128,7 @@ struct g500_bfs {
   // run one at a time (as under a counter profiler)
   hipEvent_t ev_snap = nullptr;
   g500::DevBuf<uint64_t> lpart;   // per-block totals of a level's kernels
-  g500::DevBuf<unsigned int> tickets;  // blocks done in a step's last kernel (see last_of)
+  g500::DevBuf<unsigned int> tickets;  // blocks done in a kernel whose last block goes on (comes_last)
   g500::DevBuf<uint32_t> qcnt;    // per-wave counts of the bitmap -> queue conversion
   g500::DevBuf<uint64_t> qedges;  // its per-block degree sums
   // without CoreBFS: the original IDs with edges as bits, their number before
