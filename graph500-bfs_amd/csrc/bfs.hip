@@ -17,24 +17,28 @@
 //                 there (every lane gets eight edges, whatever the degree
 //                 skew).  Winners of the visited-bit atomicOr write pred and
 //                 are appended to an LDS queue that is flushed with one global
-//                 atomic per tile.
-//   k_bu_sweep    first bottom-up level after top-down ones: a wave owns 64
-//                 bitmap words; lane l takes bit l of each word, so the
+//                 atomic per half tile of winners.
+//   k_bu_sweep    first bottom-up level after top-down ones: a wave owns up to
+//                 64 bitmap words; lane l takes bit l of each word, so the
 //                 first-neighbour probes read `first` coalesced, eight
 //                 vertices per lane in flight.  The still-unvisited vertices
 //                 go to per-chunk lists.
 //   k_bu_list     later bottom-up levels: the same probes over those lists,
 //                 compacted in place as vertices are found.  New bits are
-//                 written once per bitmap word either way.
+//                 written once per bitmap word either way.  k_bu_rest takes
+//                 their place once few vertices are left, k_bu_long the rows
+//                 too long for the sweep's lanes.
 //   k_queue_count, k_queue_write   bitmap -> queue at the bottom-up ->
 //                 top-down switch and after top-down levels run as sweeps.
 //   k_pred_gather_core / k_pred_gather   pred[o] by original ID, gathered
 //                 from the entries the levels wrote by new ID (levels write
 //                 densely by new ID; one pass in original-ID order then
-//                 produces pred).  Without CoreBFS it walks only the
-//                 vertices with edges and starts on a second stream at the
-//                 bottom-up -> top-down switch, against a bitmap snapshot;
-//                 k_pred_fixup adds the vertices the last levels reach.
+//                 produces pred).  Without CoreBFS it walks a bitmap of the
+//                 vertices with edges; on large graphs it starts on a second
+//                 stream at the bottom-up -> top-down switch, against a bitmap
+//                 snapshot, and k_pred_fixup adds the vertices the last levels
+//                 reach.
+//   k_bfs_small   a whole run of a small graph in one block.
 //   last_of, close_level, close_queue   the last block of a step's last
 //                 kernel closes it: the step's totals, the direction rule,
 //                 the next step's code.
@@ -2328,10 +2332,12 @@ uint32_t predict_next(const Step& last, HostLoop hl, const std::vector<g500_leve
   int64_t nq, fe, at[G500_AT_NUM];
   estimate_level(mode, tr, hl, &nq, &fe);
   const uint32_t next = hl.after_level(last.code, nq, fe, at);
-  // the first list level finds nearly all that its component has left (the
-  // estimate stays below that: it must not take the run to be over)
-  if (step_mode(next) == kModeBUList && mode == kModeBUList)
-    return step_code(step_level(next), kModeBURest);
+  // a sweep leaves a list level's worth, and that one finds nearly all that
+  // the component has left (the estimates are too rough to tell: a top-down
+  // sweep's takes everything, a bottom-up level's must not end the run)
+  if (step_mode(next) == kModeBUList || step_mode(next) == kModeBURest)
+    return step_code(step_level(next), mode == kModeBUList || mode == kModeBURest ? kModeBURest
+                                                                                 : kModeBUList);
   return next;
 }
 
