@@ -703,7 +703,7 @@ constexpr int kBuBatch = kWave * kBuIlp;
 // else down to 8 (one batch of vertices per lane): with 64 everywhere the 2^18
 // vertices of SCALE 18 kept 42 waves busy on 256 CUs, and SCALE 24 half the
 // resident ones.  A run at SCALE 18 / 22 / 24 / 26: 0.24 / 0.40 / 0.535 / 1.07
-// ms before, 0.18 / 0.31 / 0.475 / 1.05 now; one or two chunks per wave cost
+// ms with 64, 0.18 / 0.31 / 0.475 / 1.05 with this rule; one or two chunks per wave cost
 // 1-3 % at SCALE 24 and 26, eight 3 % at SCALE 26 (shorter deferred lists).
 constexpr int kMaxChunkWords = kWave;
 constexpr int kMinChunkWords = kBuIlp;
@@ -1646,8 +1646,8 @@ __global__ __launch_bounds__(kT) void k_levels(const int64_t* __restrict__ pred,
 // them and writes pred by original ID at the end.  It takes the same
 // directions (decide_next) and leaves the host a record per step; a run of
 // more than kSmallSteps steps leaves none and the level loop runs instead.
-// A run at SCALE 10 / 12 / 13 / 14: 150 / 186 / 201 / 201 us as a level loop, 38 / 46 /
-// 58 / 72 here (SCALE 15: 157 in the loop, past the LDS of one block).
+// A run at SCALE 10 / 12 / 13 / 14: 104 / 115 / 128 / 121 us as a level loop, 38 / 46 /
+// 59 / 73 here (SCALE 15: 135 in the loop, past the LDS of one block).
 constexpr int kSmallT = 1024;
 constexpr int kSmallVerts = 16384;
 constexpr int64_t kSmallEdges = 1 << 19;
