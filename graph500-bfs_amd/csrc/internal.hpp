@@ -89,9 +89,10 @@ struct g500_graph {
   int64_t core_vertices = 0, tree_vertices = 0, removed_parents = 0;
   int64_t hd_root = -1;                   // highest-degree core vertex
 
-  // the input edges once more, in the validator's order (made by the first
+  // the input edges once more, in the validator's order (made by the second
   // validation of a graph large enough, empty otherwise)
   std::mutex order_mu;  // engines of one graph may validate at the same time
+  int64_t edge_passes = 0;  // validations that came to the edges before there was an order
   bool order_tried = false;
   g500::DevBuf<uint64_t> ordered;
   g500::DevBuf<g500::EdgeChunk> edge_chunks;

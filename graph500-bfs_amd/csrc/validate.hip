@@ -18,7 +18,11 @@
 // few lines, the window staying in the L2; pred itself is read only where those
 // bits say an edge may be a tree edge.  1.2 ms at SCALE 24, bound by the
 // L2 requests still left (with parts of 16 KB instead of 1 KB, which leaves
-// nearly one per edge: 1.9); ordering takes 5 ms once per graph.
+// nearly one per edge: 1.9).  The second edge pass over a graph orders the
+// edges, the first is direct: ordering takes 6 ms at SCALE 24, so a program that
+// validates one tree of a graph would lose by it.  The first, second and third
+// call take 8.0, 7.6 and 1.4 ms there (8.4 each when all are direct), 1.5, 2.0 and
+// 0.45 at SCALE 22 (1.6 each).
 // Graphs of fewer edges, or trees deeper than a byte's four bits hold, take
 // the direct form.
 #include "engine.hpp"
@@ -79,10 +83,8 @@ __global__ __launch_bounds__(kT) void k_v_tree(const int64_t* __restrict__ pred,
     const bool out = p < -1 || p >= nglobal;
     if (out) ++range;
     if (i != root && p != -1 && p == i) ++self;
-    if (code) {
-      code[i] = (uint8_t)((d < kCodeNone ? d : kCodeNone) << 4 | ((uint32_t)p & 15u));
-      if (d >= kCodeNone && d != 0xFFFF) ++deep;
-    }
+    if (d >= kCodeNone && d != 0xFFFF) ++deep;
+    if (code) code[i] = (uint8_t)((d < kCodeNone ? d : kCodeNone) << 4 | ((uint32_t)p & 15u));
     if (!check_depth) continue;
     if (p == -1 && d != 0xFFFF) ++bad;
     else if (p != -1 && d == 0xFFFF) ++bad;
@@ -304,24 +306,25 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   *ok = 0;
   G500_CHECK_HIP(hipMemsetAsync(cnt, 0, sizeof(h), s));
 
-  {
-    std::lock_guard<std::mutex> lock(g->order_mu);
-    if (!g->order_tried) (void)order_edges(g, s);
-    g->order_tried = true;
-  }
-  const bool tiles = g->n_edge_chunks > 0;
-  if (tiles && !b->vcode.get()) {
+  const auto code_room = [&] {
+    if (b->vcode.get()) return;
     // IDs past the last vertex (loops may name them) have no depth
     const int64_t ids = ceil_div((int64_t)1 << g->id_bits, 1 << kEdgeWindowBits)
                         << kEdgeWindowBits;
     b->vcode.alloc_raw((size_t)ids);
     G500_CHECK_HIP(hipMemsetAsync(b->vcode.get(), 0xFF, (size_t)ids, s));
+  };
+  bool tiles;
+  {
+    std::lock_guard<std::mutex> lock(g->order_mu);
+    tiles = g->n_edge_chunks > 0;
   }
-  uint8_t* code = tiles ? b->vcode.get() : nullptr;
+  if (tiles) code_room();
+  const bool coded = tiles && !g->corebfs;  // the first pass makes the codes
 
   // stage 1-4: ranges, root, self parents, depth map
   hipLaunchKernelGGL(k_v_tree, dim3(grid(nlocal)), dim3(kT), 0, s, b->pred.get(), nlocal,
-                     nglobal, root, g->corebfs ? 0 : 1, g->corebfs ? nullptr : code, cnt);
+                     nglobal, root, g->corebfs ? 0 : 1, coded ? b->vcode.get() : nullptr, cnt);
   G500_CHECK_LAUNCH();
   fetch();
   if (h[G500_VERR_RANGE]) {
@@ -352,12 +355,6 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
       fetch();
       if (!h[kChanged]) break;
     }
-    if (tiles) {  // the codes of the rebuilt depths
-      hipLaunchKernelGGL(k_v_tree, dim3(grid(nlocal)), dim3(kT), 0, s, b->pred.get(), nlocal,
-                         nglobal, root, 0, code, cnt);
-      G500_CHECK_LAUNCH();
-      fetch();
-    }
   } else if (pe_depth(proot) != 0 || h[G500_VERR_DEPTH_MAP]) {
     errs[G500_VERR_ROOT] = pe_depth(proot) != 0;
     errs[G500_VERR_DEPTH_MAP] = (int64_t)h[G500_VERR_DEPTH_MAP];
@@ -365,11 +362,26 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   }
 
   // stage 5: every input edge, then parent edges
+  if (!tiles && h[kDeep] == 0) {
+    std::lock_guard<std::mutex> lock(g->order_mu);
+    if (g->edge_passes++ > 0 && !g->order_tried) {
+      g->order_tried = true;
+      (void)order_edges(g, s);
+    }
+    tiles = g->n_edge_chunks > 0;
+  }
+  if (tiles && !coded) {
+    code_room();
+    hipLaunchKernelGGL(k_v_tree, dim3(grid(nlocal)), dim3(kT), 0, s, b->pred.get(), nlocal,
+                       nglobal, root, 0, b->vcode.get(), cnt);
+    G500_CHECK_LAUNCH();
+    fetch();
+  }
   G500_CHECK_HIP(hipMemsetAsync(b->pred_valid.get(), 0, nlocal, s));
   if (tiles && h[kDeep] == 0) {
     hipLaunchKernelGGL(k_v_tiles, dim3((unsigned)g->n_edge_chunks), dim3(kTileT), 0, s,
                        g->ordered.get(), g->edge_chunks.get(),
-                       g->edge_part_bits, code, b->pred.get(), nlocal,
+                       g->edge_part_bits, b->vcode.get(), b->pred.get(), nlocal,
                        g->corebfs ? 0 : 1, b->pred_valid.get(), cnt);
     G500_CHECK_LAUNCH();
   } else if (g->nedges > 0) {
