@@ -70,7 +70,21 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
   *device = 0;
   (void)hipGetDevice(device);
   void* p = nullptr;
-  if (bytes < kKeepMin) return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+  const auto fresh = [&](size_t size) {
+    *got = size;
+    if (hipMalloc(&p, size) == hipSuccess) return true;
+    (void)hipGetLastError();
+    p = nullptr;
+    return false;
+  };
+  const auto fresh_after_all = [&](size_t size) {
+    device_trim();
+    return fresh(size);
+  };
+  if (bytes < kKeepMin) {
+    if (!fresh(bytes)) (void)fresh_after_all(bytes);
+    return p;
+  }
   size_t want = (bytes + kGranule - 1) / kGranule * kGranule;
   if (scratch) {
     // sizes that differ a little (another seed's graph) share a block
@@ -103,14 +117,8 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
   }
   free_blocks(old);
   if (p) return p;
-  *got = want;
-  if (hipMalloc(&p, want) == hipSuccess) return p;
-  (void)hipGetLastError();
-  device_trim();
-  if (hipMalloc(&p, want) == hipSuccess) return p;
-  (void)hipGetLastError();
-  *got = bytes;
-  return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+  if (!fresh(want) && !fresh_after_all(want)) (void)fresh(bytes);
+  return p;
 }
 
 void device_release(void* p, size_t bytes, int device) {

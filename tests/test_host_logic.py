@@ -45,3 +45,10 @@ def test_result_block_matches_reference_log(tmp_path):
         tol = 2e-6 if "validate" in k else 1e-9 * max(1.0, abs(v))
         assert abs(got[k] - v) <= tol, (k, got[k], v)
     assert abs(got["harmonic_mean_TEPS"] - 1169336659.98) < 0.01
+
+
+def test_kept_device_blocks(tmp_path):
+    exe = _build(tmp_path, "test_devmem.cc",
+                 ["-I" + os.path.join(ROOT, "tests", "cpp", "fake_device")])
+    out = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout
+    assert "devmem ok" in out
