@@ -139,6 +139,7 @@ g500_graph* new_graph_with_capacity(int device, int64_t capacity) {
 }  // namespace
 
 g500_graph::~g500_graph() {
+  g500::forget_ordered_edges(this);
   if (stream) (void)hipStreamDestroy(stream);
 }
 

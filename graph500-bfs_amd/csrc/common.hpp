@@ -55,6 +55,9 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
 void device_release(void* p, size_t bytes, int device);
 // Gives all kept blocks back to the device.
 void device_trim();
+// Releases the edge orders of graphs on the device that no validation is using
+// (edgeorder.hip): they only save time, so an allocation that fails takes them.
+void drop_ordered_edges(int device);
 
 // Device allocation owned by a host object.
 template <typename T>
@@ -75,6 +78,10 @@ struct DevBuf {
   void alloc_raw(size_t count) {
     bool used;
     reserve(count, false, &used);
+  }
+  bool try_raw(size_t count) {
+    bool used;
+    return take(count, false, &used);
   }
   // scratch that is written before it is read; false where the device has no
   // room, for a caller that can do without

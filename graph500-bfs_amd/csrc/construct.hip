@@ -365,10 +365,16 @@ void ensure_edge_bits(g500_graph* g) {
 }  // namespace g500
 
 int64_t g500_graph::device_bytes() const {
-  return (int64_t)(edges.n * sizeof(uint2) + row_off.n * sizeof(int64_t) +
+  int64_t order = 0;
+  {
+    std::lock_guard<std::mutex> lock(order_mu);
+    if (ordered)
+      order = (int64_t)(ordered->keys.n * sizeof(uint64_t) +
+                        ordered->chunks.n * sizeof(g500::EdgeChunk));
+  }
+  return order + (int64_t)(edges.n * sizeof(uint2) + row_off.n * sizeof(int64_t) +
                    col.n * sizeof(uint32_t) + first.n * sizeof(uint2) +
                    multi.n * sizeof(uint64_t) +
                    (deg_new.n + new2orig.n + orig2new.n) * sizeof(uint32_t) +
-                   tree_parent.n * sizeof(uint32_t) + has_parent.n * sizeof(uint64_t) +
-                   ordered.n * sizeof(uint64_t) + edge_chunks.n * sizeof(g500::EdgeChunk));
+                   tree_parent.n * sizeof(uint32_t) + has_parent.n * sizeof(uint64_t));
 }

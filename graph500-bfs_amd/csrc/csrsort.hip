@@ -1119,19 +1119,19 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   return true;
 }
 
-bool order_edges(g500_graph* g, hipStream_t s) {
+std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t s) {
   const int64_t ne = g->nedges;
-  if (ne < kOrderedEdgesMin || g->id_bits > kOrderedIdBits) return false;
+  if (ne < kOrderedEdgesMin || g->id_bits > kOrderedIdBits) return nullptr;
   size_t free_b = 0, total_b = 0;
   G500_CHECK_HIP(hipMemGetInfo(&free_b, &total_b));
-  if ((uint64_t)ne * sizeof(uint64_t) > total_b / 16) return false;
+  if ((uint64_t)ne * sizeof(uint64_t) > total_b / 16) return nullptr;
   const int wlog = std::max(0, g->id_bits - kEdgeWindowBits);
   const int slog = std::max(0, g->id_bits - kEdgeSliceBits);
   // as many parts of a window as two passes can tell apart
   int pass_log = 0;
   while ((1 << (pass_log + 1)) <= kMaxParts) ++pass_log;
   const int part_bits = std::min(kEdgePartBits, 2 * pass_log - wlog - slog);
-  if (part_bits < 0) return false;
+  if (part_bits < 0) return nullptr;
   const int tile_shift = kEdgeSliceBits + kEdgeWindowBits - part_bits;
   const int64_t tiles = (int64_t)1 << (wlog + slog + part_bits);
   int step_log = 0;
@@ -1144,11 +1144,12 @@ bool order_edges(g500_graph* g, hipStream_t s) {
   if ((step > 1 && !part.try_scratch((size_t)ne)) || !keys.try_scratch((size_t)ne) ||
       !off.try_scratch((size_t)tiles + 1) || !cnt.try_scratch((size_t)tiles) ||
       !cursor.try_scratch((size_t)tiles))
-    return false;
+    return nullptr;
+  ScanWorkspace ws;
   const unsigned blocks = (unsigned)ceil_div(ne, kPartTile);
   // places of the buckets from their counts
   auto places = [&](int64_t n) {
-    exclusive_scan<uint32_t>(cnt.get(), off.get(), n, g->scan_ws, s);
+    exclusive_scan<uint32_t>(cnt.get(), off.get(), n, ws, s);
     G500_CHECK_HIP(hipMemcpyAsync(cursor.get(), off.get(), n * sizeof(uint64_t),
                                   hipMemcpyDeviceToDevice, s));
   };
@@ -1210,14 +1211,15 @@ bool order_edges(g500_graph* g, hipStream_t s) {
         chunks.push_back({a, (uint32_t)(e - a), w, c, 0});
       }
     }
-  g->edge_chunks.alloc_raw(chunks.size());
-  G500_CHECK_HIP(hipMemcpyAsync(g->edge_chunks.get(), chunks.data(),
+  auto order = std::make_shared<OrderedEdges>();
+  order->chunks.alloc_raw(chunks.size());
+  G500_CHECK_HIP(hipMemcpyAsync(order->chunks.get(), chunks.data(),
                                 chunks.size() * sizeof(EdgeChunk), hipMemcpyHostToDevice, s));
   G500_CHECK_HIP(hipStreamSynchronize(s));
-  g->ordered.swap(keys);
-  g->n_edge_chunks = (int64_t)chunks.size();
-  g->edge_part_bits = part_bits;
-  return true;
+  order->keys.swap(keys);
+  order->n_chunks = (int64_t)chunks.size();
+  order->part_bits = part_bits;
+  return order;
 }
 
 }  // namespace g500

@@ -5,8 +5,8 @@
 // A graph built, searched and freed over and over (13 GB of blocks at SCALE 24)
 // took 170 to 470 ms each time that way, its kernels 40.  So blocks from 1 MiB
 // on are kept when they are released and handed out again, up to an eighth of
-// the device's memory; the oldest are given back first, all of them when an
-// allocation fails, when free memory is asked for (g500_device_memory) and,
+// the device's memory; the oldest are given back first, all of them (and then
+// the validator's edge orders) when an allocation fails, when free memory is asked for (g500_device_memory) and,
 // at the next call, when no one took them for ten seconds.
 //
 // A block is kept only after the device has finished all work queued so far
@@ -78,6 +78,9 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
     return false;
   };
   const auto fresh_after_all = [&](size_t size) {
+    device_trim();
+    if (fresh(size)) return true;
+    drop_ordered_edges(*device);
     device_trim();
     return fresh(size);
   };

@@ -25,6 +25,12 @@ struct EdgeChunk {
   uint64_t first;
   uint32_t count, window, slice, unused;
 };
+struct OrderedEdges {
+  DevBuf<uint64_t> keys;
+  DevBuf<EdgeChunk> chunks;
+  int64_t n_chunks = 0;
+  int part_bits = 0;
+};
 __host__ __device__ inline uint64_t edge_key(uint32_t s, uint32_t t, int slices_log,
                                              int part_bits) {
   const int low = kEdgeWindowBits - part_bits;
@@ -90,14 +96,13 @@ struct g500_graph {
   int64_t hd_root = -1;                   // highest-degree core vertex
 
   // the input edges once more, in the validator's order (made by the second
-  // validation of a graph large enough, empty otherwise)
-  std::mutex order_mu;  // engines of one graph may validate at the same time
+  // validation of a graph large enough, given up where the device runs out of
+  // memory, else null); all under order_mu: engines of one graph may validate
+  // at the same time
+  mutable std::mutex order_mu;
   int64_t edge_passes = 0;  // validations that came to the edges before there was an order
   bool order_tried = false;
-  g500::DevBuf<uint64_t> ordered;
-  g500::DevBuf<g500::EdgeChunk> edge_chunks;
-  int64_t n_edge_chunks = 0;
-  int edge_part_bits = 0;
+  std::shared_ptr<const g500::OrderedEdges> ordered;
 
   g500::ScanWorkspace scan_ws;
   g500::RadixWorkspace radix_ws;
@@ -144,9 +149,17 @@ void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, 
 // them (an unexpected spread of a long row's targets, or too little memory).
 bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric);
 
-// g->ordered and its chunks; false where the edges are few, their IDs too wide
-// or memory is short
-bool order_edges(g500_graph* g, hipStream_t s);
+// The input edges in the validator's order; null where they are few, their IDs
+// too wide or memory is short.
+std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t s);
+
+// edgeorder.hip: the graph's order, or null
+std::shared_ptr<const OrderedEdges> held_order(g500_graph* g);
+// The order for a pass over the edges: none for a graph's first pass, made by
+// the second.  While one engine makes it, others get none.
+std::shared_ptr<const OrderedEdges> order_for_pass(g500_graph* g, hipStream_t s);
+// before a graph that may hold an order goes
+void forget_ordered_edges(g500_graph* g);
 
 // corebfs.hip
 constexpr uint32_t kNoParent = 0xFFFFFFFFu;

@@ -278,6 +278,17 @@ unsigned grid(int64_t n) {
   return (unsigned)(b < 1 ? 1 : (b > 2048 ? 2048 : b));
 }
 
+// The engine's codes; IDs past the last vertex (loops may name them) have no
+// depth.  False where there is no room.
+bool code_room(g500_bfs* b) {
+  if (b->vcode.get()) return true;
+  const int64_t ids = ceil_div((int64_t)1 << b->g->id_bits, 1 << kEdgeWindowBits)
+                      << kEdgeWindowBits;
+  if (!b->vcode.try_raw((size_t)ids)) return false;
+  G500_CHECK_HIP(hipMemsetAsync(b->vcode.get(), 0xFF, (size_t)ids, b->stream));
+  return true;
+}
+
 }  // namespace
 
 void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
@@ -306,21 +317,8 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   *ok = 0;
   G500_CHECK_HIP(hipMemsetAsync(cnt, 0, sizeof(h), s));
 
-  const auto code_room = [&] {
-    if (b->vcode.get()) return;
-    // IDs past the last vertex (loops may name them) have no depth
-    const int64_t ids = ceil_div((int64_t)1 << g->id_bits, 1 << kEdgeWindowBits)
-                        << kEdgeWindowBits;
-    b->vcode.alloc_raw((size_t)ids);
-    G500_CHECK_HIP(hipMemsetAsync(b->vcode.get(), 0xFF, (size_t)ids, s));
-  };
-  bool tiles;
-  {
-    std::lock_guard<std::mutex> lock(g->order_mu);
-    tiles = g->n_edge_chunks > 0;
-  }
-  if (tiles) code_room();
-  const bool coded = tiles && !g->corebfs;  // the first pass makes the codes
+  std::shared_ptr<const OrderedEdges> order = held_order(g);
+  const bool coded = order && !g->corebfs && code_room(b);  // the first pass makes the codes
 
   // stage 1-4: ranges, root, self parents, depth map
   hipLaunchKernelGGL(k_v_tree, dim3(grid(nlocal)), dim3(kT), 0, s, b->pred.get(), nlocal,
@@ -362,16 +360,9 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   }
 
   // stage 5: every input edge, then parent edges
-  if (!tiles && h[kDeep] == 0) {
-    std::lock_guard<std::mutex> lock(g->order_mu);
-    if (g->edge_passes++ > 0 && !g->order_tried) {
-      g->order_tried = true;
-      (void)order_edges(g, s);
-    }
-    tiles = g->n_edge_chunks > 0;
-  }
+  if (!order && h[kDeep] == 0) order = order_for_pass(g, s);
+  const bool tiles = order && (coded || code_room(b));
   if (tiles && !coded) {
-    code_room();
     hipLaunchKernelGGL(k_v_tree, dim3(grid(nlocal)), dim3(kT), 0, s, b->pred.get(), nlocal,
                        nglobal, root, 0, b->vcode.get(), cnt);
     G500_CHECK_LAUNCH();
@@ -379,9 +370,8 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   }
   G500_CHECK_HIP(hipMemsetAsync(b->pred_valid.get(), 0, nlocal, s));
   if (tiles && h[kDeep] == 0) {
-    hipLaunchKernelGGL(k_v_tiles, dim3((unsigned)g->n_edge_chunks), dim3(kTileT), 0, s,
-                       g->ordered.get(), g->edge_chunks.get(),
-                       g->edge_part_bits, b->vcode.get(), b->pred.get(), nlocal,
+    hipLaunchKernelGGL(k_v_tiles, dim3((unsigned)order->n_chunks), dim3(kTileT), 0, s,
+                       order->keys.get(), order->chunks.get(), order->part_bits, b->vcode.get(), b->pred.get(), nlocal,
                        g->corebfs ? 0 : 1, b->pred_valid.get(), cnt);
     G500_CHECK_LAUNCH();
   } else if (g->nedges > 0) {

@@ -1,12 +1,17 @@
-// Kept device blocks against a device of 64 GiB that exists on the host only.
+// Kept device blocks and the validator's edge orders against a device of 64 GiB
+// that exists on the host only.
 #include <cstdio>
 #include <vector>
 
 #include "../../graph500-bfs_amd/csrc/devmem.hip"
+#include "../../graph500-bfs_amd/csrc/edgeorder.hip"
 
 namespace {
 
 constexpr size_t kMiB = size_t(1) << 20, kGiB = size_t(1) << 30, kAll = 64 * kGiB;
+
+int making = 0;  // order_edges: how often it was called, and the error it meets
+int error = 0;
 
 #define CHECK(x)                                                  \
   do {                                                            \
@@ -38,8 +43,17 @@ void fresh_device() {
 
 }  // namespace
 
+g500_graph::~g500_graph() { g500::forget_ordered_edges(this); }
+
 namespace g500 {
-[[noreturn]] void fail(int, const char*, ...) { std::abort(); }
+[[noreturn]] void fail(int code, const char*, ...) { throw Error(code, "fake"); }
+std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t) {
+  ++making;
+  if (error) fail(error, "");
+  auto o = std::make_shared<OrderedEdges>();
+  o->keys.alloc_raw((size_t)g->nedges);
+  return o;
+}
 }  // namespace g500
 
 int main() {
@@ -73,6 +87,62 @@ int main() {
     const Got none = take(kAll);
     CHECK(!none.p);
     for (const Got& g : {a, full, rest}) give(g);
+  }
+  // then the edge orders that no validation uses
+  for (size_t want : {size_t(4096), 512 * kMiB}) {
+    fresh_device();
+    making = 0;
+    g500_graph g, other;
+    g.nedges = other.nedges = kGiB / 8;
+    other.device = 1;
+    for (g500_graph* x : {&g, &other}) {
+      CHECK(!g500::order_for_pass(x, nullptr) && !g500::held_order(x));  // a graph's first pass
+      CHECK(g500::order_for_pass(x, nullptr) && g500::held_order(x));
+    }
+    CHECK(making == 2 && fake_device.used == 2 * kGiB);
+    const Got full = take(kAll - fake_device.used);
+    auto in_use = g500::held_order(&g);
+    CHECK(!take(want).p && g500::held_order(&g) == in_use);
+    in_use.reset();
+    const Got a = take(want);
+    CHECK(a.p && !g500::held_order(&g) && g500::held_order(&other));
+    CHECK(!g500::order_for_pass(&g, nullptr) && making == 2);  // not made again
+    give(a);
+    give(full);
+  }
+  // no room for an order: passes go without, and later ones do not try again
+  fresh_device();
+  {
+    g500_graph g;
+    g.nedges = (int64_t)kAll / 8;
+    const Got full = take(1 * kGiB);
+    making = 0;
+    for (int i = 0; i < 3; ++i) CHECK(!g500::order_for_pass(&g, nullptr));
+    CHECK(making == 1);
+    give(full);
+    g500_graph broken;  // other errors are not swallowed
+    error = G500_ERR_HIP;
+    CHECK(!g500::order_for_pass(&broken, nullptr));
+    bool thrown = false;
+    try {
+      (void)g500::order_for_pass(&broken, nullptr);
+    } catch (const g500::Error& e) {
+      thrown = e.code == G500_ERR_HIP;
+    }
+    CHECK(thrown);
+    error = 0;
+  }
+  {  // a graph that goes takes its order along and is not asked for it later
+    fresh_device();
+    {
+      g500_graph g;
+      g.nedges = kGiB / 8;
+      (void)g500::order_for_pass(&g, nullptr);
+      CHECK(g500::order_for_pass(&g, nullptr));
+    }
+    const Got all = take(kAll);
+    CHECK(all.p);
+    give(all);
   }
   fresh_device();
   {  // released beside a capture that forbids the wait: not kept

@@ -1,4 +1,6 @@
 """When the validator orders a graph's edges: the second pass over them, not the first."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -80,3 +82,27 @@ def test_mistakes_before_and_after(G):
         assert te == te_o and list(errs.values()) == [int(errs_o[k]) for k in errs], errs
         ok, te, errs = bfs.validate(r, host_pred=pred)
         assert ok and te == og.validate(r, pred)[1], errs
+
+
+# engines of one graph: one of them orders while the others pass directly
+def test_engines_side_by_side(G, golden):
+    print("\n[order] threads", flush=True)
+    scale = 20
+    g = G.Graph.generate(scale).construct()
+    engines = [G.Bfs(g) for _ in range(3)]
+    roots = g.find_roots(3).tolist()
+    wrong = []
+
+    def work(bfs, root):
+        for _ in range(4):
+            bfs.run(root)
+            ok, te, errs = bfs.validate(root)
+            if not ok or te != golden["pf_nedge"][scale]:
+                wrong.append((root, te, errs))
+
+    ts = [threading.Thread(target=work, args=x) for x in zip(engines, roots)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong
