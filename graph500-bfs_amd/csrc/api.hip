@@ -394,6 +394,7 @@ int g500_bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
     if (!b) g500::fail(G500_ERR_ARG, "null bfs handle");
     use_device(b->g->device);
     g500::bfs_run(b, root, edgefactor, alpha, beta, at_data);
+    g500::device_release_idle();
   });
 }
 
@@ -423,6 +424,7 @@ int g500_bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
     if (!b || !te || !errs || !ok) g500::fail(G500_ERR_ARG, "null argument");
     use_device(b->g->device);
     g500::bfs_validate(b, root, host_pred, te, errs, ok);
+    g500::device_release_idle();
   });
 }
 
@@ -560,6 +562,7 @@ int g500_msbfs_wait(g500_msbfs* b) {
   return guard([&] {
     need_msbfs(b);
     g500::msbfs_wait(b);
+    g500::device_release_idle();
   });
 }
 
@@ -568,6 +571,7 @@ int g500_msbfs_run(g500_msbfs* b, const int64_t* roots, int nroots) {
     need_msbfs(b);
     g500::msbfs_launch(b, roots, nroots);
     g500::msbfs_wait(b);
+    g500::device_release_idle();
   });
 }
 

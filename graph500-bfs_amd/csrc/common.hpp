@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <stdexcept>
@@ -55,6 +56,11 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
 void device_release(void* p, size_t bytes, int device);
 // Gives all kept blocks back to the device.
 void device_trim();
+// Gives back the kept blocks that no one took for ten seconds; a few
+// nanoseconds where there are none.  For the ends of calls that wait for the
+// device anyway.
+void device_release_idle(
+    std::chrono::steady_clock::time_point now = std::chrono::steady_clock::now());
 // Releases the edge orders of graphs on the device that no validation is using
 // (edgeorder.hip): they only save time, so an allocation that fails takes them.
 void drop_ordered_edges(int device);

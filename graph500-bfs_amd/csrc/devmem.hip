@@ -5,13 +5,16 @@
 // A graph built, searched and freed over and over (13 GB of blocks at SCALE 24)
 // took 170 to 470 ms each time that way, its kernels 40.  So blocks from 1 MiB
 // on are kept when they are released and handed out again, up to an eighth of
-// the device's memory; the oldest are given back first, all of them (and then
-// the validator's edge orders) when an allocation fails, when free memory is asked for (g500_device_memory) and,
-// at the next call, when no one took them for ten seconds.
+// the device's memory; the oldest are given back first.  All of them go when an
+// allocation fails (and then the validator's edge orders) or free memory is
+// asked for (g500_device_memory), and those that no one took for ten seconds at
+// the next call that allocates, frees, searches or validates.  A process that
+// makes no more calls keeps them.
 //
 // A block is kept only after the device has finished all work queued so far
 // (as hipFree waits for it), so whichever thread or stream takes it next has
 // it alone.
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <vector>
@@ -24,13 +27,15 @@ namespace {
 
 constexpr size_t kKeepMin = size_t(1) << 20;
 constexpr size_t kGranule = size_t(2) << 20;
-constexpr int kIdleSeconds = 10;
+constexpr std::chrono::seconds kIdle(10);
+
+using Clock = std::chrono::steady_clock;
 
 struct Block {
   void* p;
   size_t bytes;
   int device;
-  std::chrono::steady_clock::time_point since;
+  Clock::time_point since;
 };
 
 // never destroyed: handles may be released by destructors that run after
@@ -38,6 +43,14 @@ struct Block {
 struct Kept {
   std::mutex mu;
   std::vector<Block> blocks;  // oldest first
+  // when the oldest was released, the far future where there is none: read
+  // without the lock by calls that only look for idle blocks
+  std::atomic<Clock::rep> oldest{Clock::time_point::max().time_since_epoch().count()};
+
+  void changed() {
+    const Clock::time_point t = blocks.empty() ? Clock::time_point::max() : blocks.front().since;
+    oldest.store(t.time_since_epoch().count(), std::memory_order_relaxed);
+  }
 };
 Kept& kept() {
   static Kept* k = new Kept;
@@ -58,8 +71,14 @@ size_t keep_limit(int device) {
   return limit[(size_t)device];
 }
 
+// Idle blocks also go beside work that has nothing to do with them, another
+// thread's capture among it, which a plain hipFree would break.
 void free_blocks(const std::vector<Block>& out) {
+  if (out.empty()) return;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
   for (const Block& b : out) (void)hipFree(b.p);
+  if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 }  // namespace
@@ -85,6 +104,7 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
     return fresh(size);
   };
   if (bytes < kKeepMin) {
+    device_release_idle();
     if (!fresh(bytes)) (void)fresh_after_all(bytes);
     return p;
   }
@@ -95,7 +115,6 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
     want = (want + step - 1) / step * step;
   }
   const size_t most = want + (scratch ? want / 8 : want / 64);
-  std::vector<Block> old;
   {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
@@ -112,13 +131,9 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
       *used = true;
       k.blocks.erase(k.blocks.begin() + (ptrdiff_t)best);
     }
-    const auto limit = std::chrono::steady_clock::now() - std::chrono::seconds(kIdleSeconds);
-    while (!k.blocks.empty() && k.blocks.front().since < limit) {
-      old.push_back(k.blocks.front());
-      k.blocks.erase(k.blocks.begin());
-    }
+    k.changed();
   }
-  free_blocks(old);
+  device_release_idle();
   if (p) return p;
   if (!fresh(want) && !fresh_after_all(want)) (void)fresh(bytes);
   return p;
@@ -134,13 +149,14 @@ void device_release(void* p, size_t bytes, int device) {
       hipDeviceSynchronize() != hipSuccess) {
     (void)hipGetLastError();
     (void)hipFree(p);
+    device_release_idle();
     return;
   }
   std::vector<Block> old;
   {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    k.blocks.push_back({p, bytes, device, std::chrono::steady_clock::now()});
+    k.blocks.push_back({p, bytes, device, Clock::now()});
     size_t total = 0;
     for (const Block& b : k.blocks) total += b.device == device ? b.bytes : 0;
     for (size_t i = 0; i < k.blocks.size() && total > limit;) {
@@ -152,8 +168,10 @@ void device_release(void* p, size_t bytes, int device) {
       old.push_back(k.blocks[i]);
       k.blocks.erase(k.blocks.begin() + (ptrdiff_t)i);
     }
+    k.changed();
   }
   free_blocks(old);
+  device_release_idle();
 }
 
 void device_trim() {
@@ -162,6 +180,23 @@ void device_trim() {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
     old.swap(k.blocks);
+    k.changed();
+  }
+  free_blocks(old);
+}
+
+void device_release_idle(Clock::time_point now) {
+  Kept& k = kept();
+  const auto limit = (now - kIdle).time_since_epoch().count();
+  if (k.oldest.load(std::memory_order_relaxed) >= limit) return;
+  std::vector<Block> old;
+  {
+    std::lock_guard<std::mutex> lock(k.mu);
+    while (!k.blocks.empty() && k.blocks.front().since < now - kIdle) {
+      old.push_back(k.blocks.front());
+      k.blocks.erase(k.blocks.begin());
+    }
+    k.changed();
   }
   free_blocks(old);
 }

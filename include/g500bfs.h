@@ -164,7 +164,13 @@ int g500_find_roots(g500_graph* g, int nroots, int r1, int r2, int64_t* roots,
 int g500_make_random_numbers(int64_t nvalues, uint64_t seed1, uint64_t seed2,
                              int64_t position, double* out);
 
-/* Frees the graph.  Every engine created on it (g500_bfs, g500_msbfs) must be
+/* Frees the graph.  Device memory that handles give up stays with the library
+ * for the next graph or engine: blocks of 1 MiB and more, up to an eighth of the
+ * device.  It goes back to the device when an allocation of the library fails,
+ * when g500_device_memory is called, and, for blocks unused for ten seconds, at
+ * the next call that creates or frees a handle, searches or validates.  A
+ * process that needs the memory itself (or leaves it to another) calls
+ * g500_device_memory.  Every engine created on it (g500_bfs, g500_msbfs) must be
  * destroyed first: with engines still alive the call fails with
  * G500_ERR_STATE and frees nothing. */
 int g500_graph_free(g500_graph* g);
@@ -204,7 +210,11 @@ int g500_bfs_get_levels(g500_bfs* b, uint16_t* levels);
  * host_pred != NULL, that array uploaded first).  nglobalverts is
  * max_used_vertex+1 as in mpi/main.cc:646.  Fills te (traversed edges),
  * errs[G500_VERR_NUM] and *ok.  With CoreBFS the rebuilt depths are written
- * back into the device pred, as the reference does in place. */
+ * back into the device pred, as the reference does in place.
+ * The second validation of a graph of 2^20 edges or more leaves a copy of its
+ * edges on the device (8 bytes each, at most a sixteenth of the device, counted
+ * in g500_graph_info.device_bytes) that makes later ones faster; the graph
+ * keeps it until it is freed or an allocation needs the room. */
 int g500_bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
                       int64_t* te, int64_t* errs, int* ok);
 
@@ -330,7 +340,9 @@ enum {
 /* Device bytes g500_msbfs_create_ex(g, max_roots, flags) will allocate
  * (admission control of a serving loop checks it against g500_device_memory). */
 int g500_msbfs_footprint(const g500_graph* g, int max_roots, int flags, int64_t* bytes);
-/* Free and total device memory (hipMemGetInfo). */
+/* Gives every block kept from freed handles back, on all devices, and returns
+ * free and total device memory (hipMemGetInfo).  Allocations that follow start
+ * from the device again. */
 int g500_device_memory(int device, int64_t* free_bytes, int64_t* total_bytes);
 /* Allocates the engine for batches of up to max_roots roots (1..256). */
 int g500_msbfs_create(g500_graph* g, int max_roots, g500_msbfs** out);

@@ -145,6 +145,21 @@ int main() {
     give(all);
   }
   fresh_device();
+  {  // blocks go back once they are ten seconds old, however the library is called
+    const auto later = std::chrono::steady_clock::now() + std::chrono::seconds(11);
+    const Got a = take(100 * kMiB), b = take(200 * kMiB);
+    give(a);
+    give(b);
+    g500::device_release_idle();
+    CHECK(fake_device.used == 300 * kMiB);
+    g500::device_release_idle(later);
+    CHECK(fake_device.used == 0 && fake_device.frees == 2);
+    const Got c = take(300 * kMiB);
+    give(c);
+    g500::device_release_idle();  // younger
+    CHECK(fake_device.used == 300 * kMiB);
+  }
+  fresh_device();
   {  // released beside a capture that forbids the wait: not kept
     const Got a = take(100 * kMiB);
     fake_device.sync_fails = true;
