@@ -92,10 +92,11 @@ __device__ inline void edge_stats(uint64_t orv, uint64_t cnt, unsigned long long
   }
 }
 
-// Whether an edge counts, and toward which endpoints.
+// Whether an edge counts, and toward which endpoints.  Only loops may name IDs
+// from nv on.
 template <int kMode>
-__device__ inline bool edge_counts(const uint2& x) {
-  return kMode == kSourceAll || x.x != x.y;
+__device__ inline bool edge_counts(const uint2& x, int64_t nv) {
+  return kMode == kSourceAll ? (int64_t)x.x < nv : x.x != x.y;
 }
 
 // Block (chunk, range): counts the endpoints of a chunk of edges that lie in
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(kDegT) void k_deg_direct(const uint2* __restrict__ 
     for (int k = 0; k < kDegBatch; ++k) {
       const int64_t i = i0 + k * kDegT + threadIdx.x;
       x[k] = i < end ? e[i] : make_uint2(0, 0);
-      ok[k] = i < end && edge_counts<kMode>(x[k]);
+      ok[k] = i < end && edge_counts<kMode>(x[k], nv);
     }
 #pragma unroll
     for (int k = 0; k < kDegBatch; ++k) {
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(kDegT) void k_deg_direct(const uint2* __restrict__ 
 // Endpoints per range.
 template <int kMode>
 __global__ __launch_bounds__(kDegT) void k_deg_ranges(const uint2* __restrict__ e, int64_t ne,
-                                                     int ranges,
+                                                     int64_t nv, int ranges,
                                                      unsigned long long* __restrict__ total,
                                                      unsigned long long* stats) {
   __shared__ uint32_t hist[kMaxRanges];
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(kDegT) void k_deg_ranges(const uint2* __restrict__ 
   for (int64_t i = (int64_t)blockIdx.x * kDegT + threadIdx.x; i < ne;
        i += (int64_t)gridDim.x * kDegT) {
     const uint2 x = e[i];
-    if (!edge_counts<kMode>(x)) continue;
+    if (!edge_counts<kMode>(x, nv)) continue;
     atomicAdd(&hist[x.x >> kRangeBits], 1u);
     if (kMode == kBoth) atomicAdd(&hist[x.y >> kRangeBits], 1u);
     orv |= (uint64_t)(x.x | x.y);
@@ -192,7 +193,7 @@ __device__ inline uint32_t block_scan(uint32_t v, uint32_t* wsum, uint32_t* tota
 // atomic per range and tile.  cursor[r] starts at the range's first slot.
 template <int kMode, int kEdges, int kNumRanges>
 __global__ __launch_bounds__(kDegT) void k_deg_scatter(const uint2* __restrict__ e, int64_t ne,
-                                                      int ranges,
+                                                      int64_t nv, int ranges,
                                                       unsigned long long* __restrict__ cursor,
                                                       uint16_t* __restrict__ out) {
   constexpr int kPer = kMode == kBoth ? 2 : 1;
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(kDegT) void k_deg_scatter(const uint2* __restrict__
   for (int k = 0; k < kIt; ++k) {
     const int64_t i = base + k * kDegT + t;
     const uint2 x = i < ne ? e[i] : make_uint2(0, 0);
-    const bool ok = i < ne && edge_counts<kMode>(x);
+    const bool ok = i < ne && edge_counts<kMode>(x, nv);
     use |= (uint32_t)ok << k;
     id[k * kPer] = x.x;
     if (kPer == 2) id[k * kPer + 1] = x.y;
@@ -304,13 +305,13 @@ __global__ __launch_bounds__(kDegT) void k_deg_count(const uint16_t* __restrict_
 // The general form: any ID space, one atomic per endpoint.
 template <int kMode>
 __global__ __launch_bounds__(256) void k_deg_atomic(const uint2* __restrict__ e, int64_t ne,
-                                                   uint32_t* __restrict__ deg,
+                                                   int64_t nv, uint32_t* __restrict__ deg,
                                                    unsigned long long* stats) {
   uint64_t orv = 0, num = 0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < ne;
        i += (int64_t)gridDim.x * 256) {
     const uint2 x = e[i];
-    if (!edge_counts<kMode>(x)) continue;
+    if (!edge_counts<kMode>(x, nv)) continue;
     atomicAdd(&deg[x.x], 1u);
     if (kMode == kBoth) atomicAdd(&deg[x.y], 1u);
     orv |= (uint64_t)(x.x | x.y);
@@ -378,7 +379,7 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   if (!dense || !ep.try_scratch((size_t)(ne * kPer))) {
     hipLaunchKernelGGL(k_deg_atomic<kMode>,
                        dim3((unsigned)std::min<int64_t>(ceil_div(ne, 256), 4096)), dim3(256), 0, s,
-                       edges, ne, deg, stats);
+                       edges, ne, nv, deg, stats);
     G500_CHECK_LAUNCH();
     return;
   }
@@ -390,7 +391,7 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   G500_CHECK_HIP(hipMemsetAsync(total.get(), 0, ranges * sizeof(unsigned long long), s));
   hipLaunchKernelGGL(k_deg_ranges<kMode>,
                      dim3((unsigned)std::min<int64_t>(ceil_div(ne, kDegT * 8), 1024)), dim3(kDegT),
-                     0, s, edges, ne, (int)ranges, total.get(), stats);
+                     0, s, edges, ne, nv, (int)ranges, total.get(), stats);
   G500_CHECK_LAUNCH();
   exclusive_scan<uint64_t>((const uint64_t*)total.get(), off.get(), ranges, ws, s);
   G500_CHECK_HIP(hipMemcpyAsync(total.get(), off.get(), ranges * sizeof(uint64_t),
@@ -398,11 +399,11 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   if (ranges <= 1024) {
     constexpr int kEdges = 16384;
     hipLaunchKernelGGL((k_deg_scatter<kMode, kEdges, 1024>), dim3((unsigned)ceil_div(ne, kEdges)),
-                       dim3(kDegT), 0, s, edges, ne, (int)ranges, total.get(), ep.get());
+                       dim3(kDegT), 0, s, edges, ne, nv, (int)ranges, total.get(), ep.get());
   } else {
     constexpr int kEdges = 8192;
     hipLaunchKernelGGL((k_deg_scatter<kMode, kEdges, kMaxRanges>),
-                       dim3((unsigned)ceil_div(ne, kEdges)), dim3(kDegT), 0, s, edges, ne,
+                       dim3((unsigned)ceil_div(ne, kEdges)), dim3(kDegT), 0, s, edges, ne, nv,
                        (int)ranges, total.get(), ep.get());
   }
   G500_CHECK_LAUNCH();

@@ -127,7 +127,7 @@ enum class DegreeMode {
   kSourceNoLoops,  // the source of every edge that is no loop
   kSourceRuns,     // the source of every edge; there are no loops, and the edges of a source
                    // stand together
-  kSourceEnd       // the source of every edge
+  kSourceEnd       // the source of every edge, if below nv
 };
 // CSR of `edges` into g, counted as `mode` says: both directions of each edge
 // (kBothEnds) or the one the list holds (force_log_n < 0: estimate the vertex
@@ -140,7 +140,7 @@ inline bool has_csr_edge(const g500_graph* g, int64_t v) {
 }
 
 // csrsort.hip
-// deg[v] += edges at v for IDs below nv; stats[0] |= the IDs of the edges
+// deg[v] += edges at v for IDs below nv (every ID counted is, but with kSourceEnd); stats[0] |= the IDs of the edges
 // counted, stats[1] += their number
 void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, uint32_t* deg,
                    unsigned long long* stats, hipStream_t s);

@@ -2060,6 +2060,9 @@ int64_t msbfs_footprint(const g500_graph* g, int max_roots, bool level_arrays) {
   const int64_t bw = std::max<int64_t>(1, ceil_div(g->n_c, 64));
   int64_t bytes = nc * kmax * 8;                      // seen
   bytes += (int64_t)kInitialLevels * nc * kmax * 8;   // level frontiers
+  // before these, beside cnt0: degrees and, where there is room, two bytes an
+  // edge (count_degrees), in blocks a sixteenth larger at most
+  bytes = std::max<int64_t>(bytes, g->n * 4 + g->nedges * 2 + g->nedges / 8);
   if (level_arrays) {
     bytes += (int64_t)max_roots * g->n;                 // level arrays
     bytes += nc * 4 * std::min<int64_t>(kmax, 2) * 8;  // their bit planes (K <= 2)
@@ -2083,13 +2086,13 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
   // first, so that its scratch is gone before the engine's own arrays come
   b->cnt0.alloc((size_t)g->n);
   {
-    const int64_t nv = (int64_t)1 << g->id_bits;  // covers every input ID
+    // only loops name IDs from n on, which no root reaches
     DevBuf<uint32_t> deg;
     DevBuf<unsigned long long> stats;
-    deg.alloc((size_t)nv);
+    deg.alloc_raw((size_t)g->n);
     stats.alloc(2);
-    G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, (size_t)nv * sizeof(uint32_t), b->stream));
-    count_degrees(g->edges.get(), g->nedges, DegreeMode::kSourceEnd, nv, deg.get(), stats.get(),
+    G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, (size_t)g->n * sizeof(uint32_t), b->stream));
+    count_degrees(g->edges.get(), g->nedges, DegreeMode::kSourceEnd, g->n, deg.get(), stats.get(),
                   b->stream);
     hipLaunchKernelGGL(k_ms_cnt0, dim3((unsigned)ceil_div(g->n, kT)), dim3(kT), 0, b->stream,
                        deg.get(), g->n, g->orig2new.get(), b->cnt0.get());

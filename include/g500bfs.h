@@ -337,7 +337,8 @@ typedef struct g500_msbfs_stats {
 enum {
   G500_MSBFS_NO_LEVEL_ARRAYS = 1  /* answer point lookups only: no [roots][N] arrays */
 };
-/* Device bytes g500_msbfs_create_ex(g, max_roots, flags) will allocate
+/* Device bytes g500_msbfs_create_ex(g, max_roots, flags) will allocate, the
+ * scratch it needs meanwhile included
  * (admission control of a serving loop checks it against g500_device_memory). */
 int g500_msbfs_footprint(const g500_graph* g, int max_roots, int flags, int64_t* bytes);
 /* Gives every block kept from freed handles back, on all devices, and returns
