@@ -373,21 +373,22 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
     return;
   }
   // partitioning pays once the ranges hold endpoints enough to be counted in
-  // LDS; a sparse list over a large ID space keeps the atomics
+  // LDS; a sparse list over a large ID space keeps the atomics, and so does
+  // one whose endpoints find no room (asked for last)
+  DevBuf<unsigned long long> total;  // per range, then (off) its first slot and a cursor
+  DevBuf<uint64_t> off;
   DevBuf<uint16_t> ep;
+  ScanWorkspace ws;
   const bool dense = ranges <= kMaxRanges && ne * kPer >= nv;
-  if (!dense || !ep.try_scratch((size_t)(ne * kPer))) {
+  if (dense) ws.reserve(ranges);
+  if (!dense || !total.try_scratch((size_t)ranges) || !off.try_scratch((size_t)ranges + 1) ||
+      !ep.try_scratch((size_t)(ne * kPer))) {
     hipLaunchKernelGGL(k_deg_atomic<kMode>,
                        dim3((unsigned)std::min<int64_t>(ceil_div(ne, 256), 4096)), dim3(256), 0, s,
                        edges, ne, nv, deg, stats);
     G500_CHECK_LAUNCH();
     return;
   }
-  DevBuf<unsigned long long> total;  // per range, then (off) its first slot and a cursor
-  DevBuf<uint64_t> off;
-  total.alloc_raw((size_t)ranges);
-  off.alloc_raw((size_t)ranges + 1);
-  ScanWorkspace ws;
   G500_CHECK_HIP(hipMemsetAsync(total.get(), 0, ranges * sizeof(unsigned long long), s));
   hipLaunchKernelGGL(k_deg_ranges<kMode>,
                      dim3((unsigned)std::min<int64_t>(ceil_div(ne, kDegT * 8), 1024)), dim3(kDegT),
@@ -1008,21 +1009,17 @@ void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, 
   }
 }
 
-// g->col and g->row_off for m entries; false where the device has no room.
-// The last entries of col are padding: bottom-up scans read aligned 16-byte
-// groups, which may run a few entries past the last row.
-static bool take_rows(g500_graph* g, int64_t m) {
-  try {
-    g->col.alloc_raw((size_t)m + kColPad);
-    g->row_off.alloc_raw((size_t)g->n_c + 1);
-  } catch (const Error&) {
-    return false;
-  }
+// g->col and g->row_off for m entries.  The last entries of col are padding:
+// bottom-up scans read aligned 16-byte groups, which may run a few entries past
+// the last row.
+static void take_rows(g500_graph* g, int64_t m) {
+  g->col.alloc_raw((size_t)m + kColPad);
+  g->row_off.alloc_raw((size_t)g->n_c + 1);
   G500_CHECK_HIP(hipMemsetAsync(g->col.get() + m, 0, kColPad * sizeof(uint32_t), g->stream));
-  return true;
 }
 
-bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
+// build_rows; throws NOMEM where something small finds no room.
+static bool rows_by_buckets(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   hipStream_t s = g->stream;
   const int64_t keys = g->m_sym, n_c = g->n_c;
   const int lg = g->log_n;
@@ -1107,8 +1104,8 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   G500_CHECK_HIP(hipMemcpyAsync(&m, ubase.get() + buckets, sizeof(m), hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipMemcpyAsync(&over, flag.get(), sizeof(over), hipMemcpyDeviceToHost, s));
   G500_CHECK_HIP(hipStreamSynchronize(s));
-  if (over || !take_rows(g, (int64_t)m))
-    return false;
+  if (over) return false;
+  take_rows(g, (int64_t)m);
   g->m = (int64_t)m;
   hipLaunchKernelGGL(k_collect, dim3((unsigned)buckets), dim3(256), 0, s, un, off.get(),
                      ucnt.get(), ubase.get(), g->col.get());
@@ -1118,6 +1115,17 @@ bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
   return true;
+}
+
+bool build_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
+  try {
+    if (rows_by_buckets(g, edges, ne, symmetric)) return true;
+  } catch (const Error& e) {
+    if (e.code != G500_ERR_NOMEM) throw;
+  }
+  g->col.release();
+  g->row_off.release();
+  return false;
 }
 
 std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t s) {
