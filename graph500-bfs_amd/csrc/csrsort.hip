@@ -1025,13 +1025,10 @@ static bool rows_by_buckets(g500_graph* g, const uint2* edges, int64_t ne, bool 
   const int lg = g->log_n;
   if (keys <= 0 || n_c <= 0) return false;
   const int64_t buckets = ceil_div(keys, kBucketMean);
-  // one pass up to kMaxParts buckets; above that groups of `step` buckets
-  // first, one to four times as many groups as buckets in each
-  int64_t step = 1;
-  if (buckets > kMaxParts)
-    while (4 * step * step <= buckets) step *= 2;
+  // one pass up to kMaxParts buckets; above that groups of `step` buckets first
+  const int64_t step = group_buckets(buckets, kMaxParts);
+  if (step == 0 || lg > 31) return false;
   const int64_t groups = ceil_div(buckets, step);
-  if (groups > kMaxParts || step > kMaxParts || lg > 31) return false;
   const bool two = step > 1;
   const int64_t group_keys = step * kBucketMean;
   const int64_t group_cap = group_keys + group_keys / 8 + kPartTile;

@@ -144,6 +144,17 @@ inline bool has_csr_edge(const g500_graph* g, int64_t v) {
 // counted, stats[1] += their number
 void count_degrees(const uint2* edges, int64_t ne, DegreeMode mode, int64_t nv, uint32_t* deg,
                    unsigned long long* stats, hipStream_t s);
+// Buckets in each group of the first of two partition passes, which make at most
+// `most` parts each: one to four times as many groups as buckets in each (long
+// runs in the second pass), more buckets in each where that would be more groups
+// than a pass makes.  1 where one pass makes all the buckets, 0 where two do not.
+inline int64_t group_buckets(int64_t buckets, int64_t most) {
+  if (buckets <= most) return 1;
+  int64_t step = 1;
+  while (4 * step * step <= buckets || ceil_div(buckets, step) > most) step *= 2;
+  return step <= most ? step : 0;
+}
+
 // Sorted rows without repeated entries (g->m, col, row_off) from the edges,
 // g's maps and degrees.  False, with nothing kept, where this form cannot sort
 // them (an unexpected spread of a long row's targets, or too little memory).

@@ -52,3 +52,10 @@ def test_kept_device_blocks(tmp_path):
                  ["-I" + os.path.join(ROOT, "tests", "cpp", "fake_device")])
     out = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout
     assert "devmem ok" in out
+
+
+def test_partition_groups(tmp_path):
+    exe = _build(tmp_path, "test_partition.cc",
+                 ["-I" + os.path.join(ROOT, "tests", "cpp", "fake_device")])
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=60).stdout
+    assert "partition ok" in out, out
