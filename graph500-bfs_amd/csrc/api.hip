@@ -115,8 +115,8 @@ void append_edges(g500_graph* g, const int64_t* v0, const int64_t* v1, int64_t c
       packed[(size_t)i] = make_uint2((uint32_t)a, (uint32_t)c);
       ors |= (uint64_t)(a | c);
     }
-    G500_CHECK_HIP(hipMemcpy(g->edges.get() + g->nedges, packed.data(), nb * sizeof(uint2),
-                             hipMemcpyHostToDevice));
+    g500::copy_now(g->edges.get() + g->nedges, packed.data(), nb * sizeof(uint2),
+                   hipMemcpyHostToDevice, g->stream);
     g->nedges += nb;
     g->id_or |= ors;
   }
@@ -240,8 +240,7 @@ int g500_graph_copy_forest(const g500_graph* g, int64_t* tree_parent, uint8_t* h
     if (!g->corebfs) g500::fail(G500_ERR_STATE, "graph was not built with CoreBFS");
     use_device(g->device);
     std::vector<uint32_t> tp((size_t)g->n);
-    G500_CHECK_HIP(hipMemcpy(tp.data(), g->tree_parent.get(), g->n * sizeof(uint32_t),
-                             hipMemcpyDeviceToHost));
+    g500::copy_to_host(tp.data(), g->tree_parent.get(), g->n, g->stream);
     for (int64_t o = 0; o < g->n; ++o) {
       if (tree_parent) tree_parent[o] = tp[(size_t)o] == g500::kNoParent ? -1 : (int64_t)tp[(size_t)o];
       if (has_parent) has_parent[o] = g500::has_parent_host(g, o) ? 1 : 0;
@@ -267,9 +266,7 @@ int g500_graph_copy_edges(const g500_graph* g, int64_t start, int64_t count,
     if (count && (!v0 || !v1)) g500::fail(G500_ERR_ARG, "null output arrays");
     use_device(g->device);
     std::vector<uint2> tmp((size_t)count);
-    if (count)
-      G500_CHECK_HIP(hipMemcpy(tmp.data(), g->edges.get() + start, count * sizeof(uint2),
-                               hipMemcpyDeviceToHost));
+    if (count) g500::copy_to_host(tmp.data(), g->edges.get() + start, count, g->stream);
     for (int64_t i = 0; i < count; ++i) {
       v0[i] = tmp[(size_t)i].x;
       v1[i] = tmp[(size_t)i].y;
@@ -283,25 +280,17 @@ int g500_graph_copy_csr(const g500_graph* g, int64_t* row_off, uint32_t* col,
     need_graph(g, true);
     use_device(g->device);
     if (row_off) {
-      G500_CHECK_HIP(hipMemcpy(row_off, g->row_off.get(), (g->n_c + 1) * sizeof(int64_t),
-                               hipMemcpyDeviceToHost));
+      g500::copy_to_host(row_off, g->row_off.get(), g->n_c + 1, g->stream);
       for (int64_t v = g->n_c + 1; v <= g->n; ++v) row_off[v] = g->m;
     }
-    if (col && g->m)
-      G500_CHECK_HIP(hipMemcpy(col, g->col.get(), g->m * sizeof(uint32_t),
-                               hipMemcpyDeviceToHost));
+    if (col && g->m) g500::copy_to_host(col, g->col.get(), g->m, g->stream);
     if (deg_new) {
       std::vector<uint32_t> d((size_t)g->n);
-      G500_CHECK_HIP(hipMemcpy(d.data(), g->deg_new.get(), g->n * sizeof(uint32_t),
-                               hipMemcpyDeviceToHost));
+      g500::copy_to_host(d.data(), g->deg_new.get(), g->n, g->stream);
       for (int64_t i = 0; i < g->n; ++i) deg_new[i] = d[(size_t)i];
     }
-    if (new2orig)
-      G500_CHECK_HIP(hipMemcpy(new2orig, g->new2orig.get(), g->n * sizeof(uint32_t),
-                               hipMemcpyDeviceToHost));
-    if (orig2new)
-      G500_CHECK_HIP(hipMemcpy(orig2new, g->orig2new.get(), g->n * sizeof(uint32_t),
-                               hipMemcpyDeviceToHost));
+    if (new2orig) g500::copy_to_host(new2orig, g->new2orig.get(), g->n, g->stream);
+    if (orig2new) g500::copy_to_host(orig2new, g->orig2new.get(), g->n, g->stream);
   });
 }
 
@@ -584,8 +573,7 @@ int g500_msbfs_get_levels(g500_msbfs* b, int index, uint8_t* host_levels) {
     if (index < 0 || index >= b->nroots)
       g500::fail(G500_ERR_ARG, "root index %d outside [0, %d)", index, b->nroots);
     const size_t n = (size_t)b->g->n;
-    G500_CHECK_HIP(hipMemcpy(host_levels, b->out.get() + (size_t)index * n, n,
-                             hipMemcpyDeviceToHost));
+    g500::copy_to_host(host_levels, b->out.get() + (size_t)index * n, (int64_t)n, b->stream);
   });
 }
 
@@ -635,8 +623,8 @@ int g500_msbfs_get_te(g500_msbfs* b, int64_t* te) {
   return guard([&] {
     need_result(b);
     if (!te) g500::fail(G500_ERR_ARG, "null output buffer");
-    G500_CHECK_HIP(hipMemcpy(te, b->te.get(), (size_t)b->nroots * sizeof(int64_t),
-                             hipMemcpyDeviceToHost));
+    g500::copy_now(te, b->te.get(), (size_t)b->nroots * sizeof(int64_t), hipMemcpyDeviceToHost,
+                   b->stream);
   });
 }
 

@@ -1918,20 +1918,21 @@ unsigned grid_for(int64_t work_items, int64_t per_block) {
 void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   g500_graph* g = b->g;
   b->words = ceil_div(std::max<int64_t>(g->n_c, 1), 64);
-  b->pred.alloc((size_t)g->n);
-  b->pred_new.alloc((size_t)std::max<int64_t>(g->n_c, 1));
+  b->pred.alloc((size_t)g->n, b->stream);
+  b->pred_new.alloc((size_t)std::max<int64_t>(g->n_c, 1), b->stream);
   // every entry starts with the epoch no run uses (run_entry)
-  G500_CHECK_HIP(hipMemset(b->pred_new.get(), 0xFF, b->pred_new.n * sizeof(int64_t)));
+  G500_CHECK_HIP(
+      hipMemsetAsync(b->pred_new.get(), 0xFF, b->pred_new.n * sizeof(int64_t), b->stream));
   b->epoch = 0xFFFFFFFFu;  // the first run's epoch is 0
-  b->vis.alloc((size_t)b->words);
-  b->vis_alt.alloc((size_t)b->words);
-  b->q.alloc((size_t)std::max<int64_t>(g->n_c, 1));
-  b->nq.alloc((size_t)std::max<int64_t>(g->n_c, 1));
-  b->dsum.alloc((size_t)std::max<int64_t>(g->n_c, 1) + 1);
+  b->vis.alloc((size_t)b->words, b->stream);
+  b->vis_alt.alloc((size_t)b->words, b->stream);
+  b->q.alloc((size_t)std::max<int64_t>(g->n_c, 1), b->stream);
+  b->nq.alloc((size_t)std::max<int64_t>(g->n_c, 1), b->stream);
+  b->dsum.alloc((size_t)std::max<int64_t>(g->n_c, 1) + 1, b->stream);
   // a frontier's edges never exceed m
-  b->tile_owner.alloc((size_t)ceil_div(std::max<int64_t>(g->m, 1), kTdTile) + 2);
-  b->bsum.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile));
-  b->boff.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile));
+  b->tile_owner.alloc((size_t)ceil_div(std::max<int64_t>(g->m, 1), kTdTile) + 2, b->stream);
+  b->bsum.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile), b->stream);
+  b->boff.alloc((size_t)ceil_div(std::max<int64_t>(g->n_c, 1), kPrepTile), b->stream);
   // bottom-up grids: what stays resident (each block stages the hub bits
   // once), never more blocks than chunk groups
   int cus = 0, per_cu[3] = {0, 0, 0};
@@ -1949,18 +1950,19 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
              (int64_t)cus * std::max(per_cu[0], 1) * kBuWaves * kChunksPerWave)
     b->chunk_words /= 2;
   const int64_t chunks = ceil_div(b->words, b->chunk_words);
-  b->unv.alloc((size_t)(chunks * b->chunk_words * 64));
-  b->unv_cnt.alloc((size_t)chunks);
+  b->unv.alloc((size_t)(chunks * b->chunk_words * 64), b->stream);
+  b->unv_cnt.alloc((size_t)chunks, b->stream);
   for (int i = 0; i < 3; ++i)
     b->bu_grid[i] = (unsigned)std::max<int64_t>(
         1, std::min<int64_t>((int64_t)std::max(cus, 1) * std::max(per_cu[i], 1),
                              ceil_div(chunks, kBuWaves)));
   b->lpart.alloc((size_t)std::max<int64_t>(
-      kMaxGrid, std::max<int64_t>(b->bu_grid[0] + b->bu_grid[2], b->bu_grid[1])));
-  b->tickets.alloc((size_t)kTickets);
-  b->wacc.alloc((size_t)b->bu_grid[0] + b->bu_grid[2] + b->bu_grid[1]);
-  b->lsync.alloc(1);
-  G500_CHECK_HIP(hipMemset(b->lsync.get(), 0, sizeof(LevelSync)));
+                     kMaxGrid, std::max<int64_t>(b->bu_grid[0] + b->bu_grid[2], b->bu_grid[1])),
+                 b->stream);
+  b->tickets.alloc((size_t)kTickets, b->stream);
+  b->wacc.alloc((size_t)b->bu_grid[0] + b->bu_grid[2] + b->bu_grid[1], b->stream);
+  b->lsync.alloc(1, b->stream);
+  G500_CHECK_HIP(hipMemsetAsync(b->lsync.get(), 0, sizeof(LevelSync), b->stream));
   // the level loop's ring, then the one-block run's header and steps
   constexpr size_t kReports = kReportSlots + 1 + kSmallSteps;
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_report, kReports * sizeof(HostReport),
@@ -1975,9 +1977,9 @@ void bfs_init(g500_bfs* b, int edgefactor, double alpha, double beta) {
   G500_CHECK_HIP(hipEventCreate(&b->ev_g1));
   G500_CHECK_HIP(hipStreamCreate(&b->gstream));
   b->overlap_gather = g->n >= kOverlapVerts;
-  if (b->overlap_gather) b->vis_snap.alloc((size_t)b->words);
-  b->qcnt.alloc((size_t)kQueueGrid * kWavesPerBlock);
-  b->qedges.alloc((size_t)kQueueGrid);
+  if (b->overlap_gather) b->vis_snap.alloc((size_t)b->words, b->stream);
+  b->qcnt.alloc((size_t)kQueueGrid * kWavesPerBlock, b->stream);
+  b->qedges.alloc((size_t)kQueueGrid, b->stream);
   if (!g->corebfs && g->n_c > 0) {
     // the core's original IDs in ascending order; pred starts at -1, which
     // the vertices without edges keep
@@ -2606,8 +2608,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
     if (root_in) {
       int64_t ro[2];
       uint32_t root_new = 0;
-      G500_CHECK_HIP(hipMemcpy(&root_new, g->orig2new.get() + bfs_root, sizeof(root_new),
-                               hipMemcpyDeviceToHost));
+      copy_to_host(&root_new, g->orig2new.get() + bfs_root, 1, s);
       G500_CHECK_HIP(hipMemcpyAsync(ro, g->row_off.get() + root_new, sizeof(ro),
                                     hipMemcpyDeviceToHost, s));
       G500_CHECK_HIP(hipStreamSynchronize(s));
@@ -2814,8 +2815,7 @@ void bfs_run(g500_bfs* b, int64_t root, int edgefactor, double alpha,
   }
   if (b->counting) {
     std::vector<uint64_t> w(b->wacc.n);
-    G500_CHECK_HIP(hipMemcpy(w.data(), b->wacc.get(), w.size() * sizeof(uint64_t),
-                             hipMemcpyDeviceToHost));
+    copy_to_host(w.data(), b->wacc.get(), (int64_t)w.size(), s);
     uint64_t sweep_dev = 0, other_dev = 0;
     for (size_t i = 0; i < w.size(); ++i) (i < b->bu_grid[0] ? sweep_dev : other_dev) += w[i];
     b->stats.counted = 1;

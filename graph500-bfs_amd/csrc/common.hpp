@@ -65,6 +65,19 @@ void device_release_idle(
 // (edgeorder.hip): they only save time, so an allocation that fails takes them.
 void drop_ordered_edges(int device);
 
+// A copy behind the work of s, done on return.  Nothing here uses the default
+// stream: its every use, in any thread, ends the captures that other threads'
+// engines make of their batches, and fails itself.
+inline void copy_now(void* dst, const void* src, size_t bytes, hipMemcpyKind kind,
+                     hipStream_t s) {
+  G500_CHECK_HIP(hipMemcpyAsync(dst, src, bytes, kind, s));
+  G500_CHECK_HIP(hipStreamSynchronize(s));
+}
+template <class T>
+void copy_to_host(T* dst, const T* src, int64_t n, hipStream_t s) {
+  copy_now(dst, src, (size_t)n * sizeof(T), hipMemcpyDeviceToHost, s);
+}
+
 // Device allocation owned by a host object.
 template <typename T>
 struct DevBuf {
@@ -74,11 +87,11 @@ struct DevBuf {
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   ~DevBuf() { release(); }
-  // a block that held other data is cleared, as the driver clears new ones
-  void alloc(size_t count) {
+  // a block that held other data is cleared on s, as the driver clears new ones
+  void alloc(size_t count, hipStream_t s) {
     bool used;
     reserve(count, false, &used);
-    if (used) G500_CHECK_HIP(hipMemset(p, 0, n * sizeof(T)));
+    if (used) G500_CHECK_HIP(hipMemsetAsync(p, 0, n * sizeof(T), s));
   }
   // for arrays that are written before they are read
   void alloc_raw(size_t count) {

@@ -252,8 +252,8 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   g->m = (int64_t)m_total;
   // padding: bottom-up scans read aligned 16-byte groups, which may run a
   // few entries past the last row
-  g->col.alloc((size_t)g->m + kColPad);
-  g->row_off.alloc((size_t)g->n_c + 1);
+  g->col.alloc((size_t)g->m + kColPad, s);
+  g->row_off.alloc((size_t)g->n_c + 1, s);
   hipLaunchKernelGGL(k_dedup_write, dim3((unsigned)tiles), dim3(kT), 0, s,
                      sorted, ms, lg, toff.get(), g->col.get(), g->row_off.get());
   G500_CHECK_LAUNCH();
@@ -272,7 +272,7 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, DegreeMode mode,
   const int64_t nv = (int64_t)1 << g->id_bits;  // covers every input ID
 
   DevBuf<unsigned long long> stats;
-  stats.alloc(8);
+  stats.alloc(8, s);
   G500_CHECK_HIP(hipMemsetAsync(stats.get(), 0, 8 * sizeof(unsigned long long), s));
   DevBuf<uint32_t> deg;
   deg.alloc_raw((size_t)nv);

@@ -310,7 +310,7 @@ void corebfs_prune(g500_graph* g) {
   leaves.alloc_raw((size_t)nn);
   twig.alloc_raw((size_t)nn);
   alive.alloc_raw((size_t)nn);
-  cnt.alloc(4);
+  cnt.alloc(4, s);
   if (n_c > 0) {
     hipLaunchKernelGGL(k_core_init, dim3(blocks(n_c)), dim3(kT), 0, s, g->row_off.get(),
                        n_c, deg.get(), alive.get(), par.get());
@@ -407,14 +407,13 @@ void corebfs_prune(g500_graph* g) {
   g->max_used = (int64_t)read_u64(cnt.get(), s);
 
   g->h_has_parent.resize((size_t)ceil_div(n, 64));
-  G500_CHECK_HIP(hipMemcpy(g->h_has_parent.data(), g->has_parent.get(),
-                           g->h_has_parent.size() * sizeof(uint64_t), hipMemcpyDeviceToHost));
+  copy_to_host(g->h_has_parent.data(), g->has_parent.get(), (int64_t)g->h_has_parent.size(), s);
   g->corebfs = 1;
   g->core_reset_done = false;
   g->hd_root = g->n_c > 0 ? -2 : -1;  // resolved after the new2orig copy below
   if (g->n_c > 0) {
     uint32_t r = 0;
-    G500_CHECK_HIP(hipMemcpy(&r, g->new2orig.get(), sizeof(uint32_t), hipMemcpyDeviceToHost));
+    copy_to_host(&r, g->new2orig.get(), 1, s);
     g->hd_root = r;  // new ID 0: highest core degree, ties by lowest original ID
   }
   g->constructed = true;
@@ -425,7 +424,7 @@ void corebfs_reset_unreachable(g500_graph* g, const uint64_t* visited, hipStream
   DevBuf<uint8_t> reach;
   DevBuf<unsigned long long> cnt;
   reach.alloc_raw((size_t)n);
-  cnt.alloc(1);
+  cnt.alloc(1, s);
   hipLaunchKernelGGL(k_reach_init, dim3(blocks(n)), dim3(kT), 0, s, g->orig2new.get(),
                      visited, n, g->n_c, reach.get());
   G500_CHECK_LAUNCH();
@@ -443,8 +442,7 @@ void corebfs_reset_unreachable(g500_graph* g, const uint64_t* visited, hipStream
   G500_CHECK_LAUNCH();
   g->removed_parents = (int64_t)read_u64(cnt.get(), s);
   g->h_tree_parent.resize((size_t)n);
-  G500_CHECK_HIP(hipMemcpy(g->h_tree_parent.data(), g->tree_parent.get(),
-                           n * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  copy_to_host(g->h_tree_parent.data(), g->tree_parent.get(), n, s);
   g->core_reset_done = true;
 }
 

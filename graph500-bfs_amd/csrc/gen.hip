@@ -197,7 +197,7 @@ void generate_edges(g500_graph* g, int scale, int edgefactor, uint64_t seed1,
   const int64_t ne = ((int64_t)1 << scale) * edgefactor;
   const MrgTable& t = mrg_table();
   DevBuf<Mat5> tab;
-  tab.alloc(8 * 256);
+  tab.alloc(8 * 256, g->stream);
   G500_CHECK_HIP(hipMemcpyAsync(tab.get(), &t.t[8][0], sizeof(Mat5) * 8 * 256,
                                 hipMemcpyHostToDevice, g->stream));
   GenArgs a;

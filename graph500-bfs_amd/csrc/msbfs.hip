@@ -1930,15 +1930,14 @@ void enqueue_batch(const g500_msbfs* b, int K, int cap, hipStream_t s) {
 void add_level_buffer(g500_msbfs* b) {
   auto* f = new DevBuf<uint64_t>;
   try {
-    f->alloc((size_t)std::max<int64_t>(1, b->g->n_c) * b->kmax);
+    f->alloc((size_t)std::max<int64_t>(1, b->g->n_c) * b->kmax, b->stream);
   } catch (...) {
     delete f;
     throw;
   }
   b->F.push_back(f);
   const uint64_t* p = f->get();
-  G500_CHECK_HIP(hipMemcpy(b->fptr.get() + (b->F.size() - 1), &p, sizeof(p),
-                           hipMemcpyHostToDevice));
+  copy_now(b->fptr.get() + (b->F.size() - 1), &p, sizeof(p), hipMemcpyHostToDevice, b->stream);
 }
 
 void drop_graphs(g500_msbfs* b) {
@@ -1979,7 +1978,7 @@ void update_bins(g500_msbfs* b) {
   g500_graph* g = b->g;
   hipStream_t s = b->stream;
   DevBuf<int64_t> d;
-  d.alloc(2);
+  d.alloc(2, b->stream);
   hipLaunchKernelGGL(k_ms_bins, dim3(1), dim3(1), 0, s, g->deg_new.get(), g->n_c,
                      b->tuning.heavy_degree, b->tuning.medium_degree, d.get());
   G500_CHECK_LAUNCH();
@@ -1989,15 +1988,14 @@ void update_bins(g500_msbfs* b) {
   b->bin_heavy = hm[0];
   b->bin_medium = std::max(hm[0], hm[1]);
   const int64_t h = b->bin_heavy;
-  G500_CHECK_HIP(hipMemcpy(&b->heavy_edges, g->row_off.get() + h, sizeof(int64_t),
-                           hipMemcpyDeviceToHost));
-  b->item_start.alloc((size_t)h + 1);
-  b->acc.alloc((size_t)std::max<int64_t>(1, h) * b->kmax);
+  copy_to_host(&b->heavy_edges, g->row_off.get() + h, 1, s);
+  b->item_start.alloc((size_t)h + 1, b->stream);
+  b->acc.alloc((size_t)std::max<int64_t>(1, h) * b->kmax, b->stream);
   G500_CHECK_HIP(hipMemsetAsync(b->acc.get(), 0, b->acc.n * sizeof(uint64_t), s));
   b->n_items = 0;
   if (h > 0) {
     DevBuf<uint32_t> items;
-    items.alloc((size_t)h);
+    items.alloc((size_t)h, b->stream);
     hipLaunchKernelGGL(k_ms_item_counts, dim3((unsigned)ceil_div(h, kT)), dim3(kT), 0, s,
                        g->row_off.get(), h, b->tuning.heavy_chunk, items.get());
     G500_CHECK_LAUNCH();
@@ -2008,9 +2006,8 @@ void update_bins(g500_msbfs* b) {
     G500_CHECK_HIP(hipStreamSynchronize(s));
     b->n_items = (int64_t)total;
     b->h_item_start.resize((size_t)h + 1);
-    G500_CHECK_HIP(hipMemcpy(b->h_item_start.data(), b->item_start.get(),
-                             ((size_t)h + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost));
-    b->item_vertex.alloc((size_t)std::max<int64_t>(1, b->n_items));
+    copy_to_host(b->h_item_start.data(), b->item_start.get(), h + 1, s);
+    b->item_vertex.alloc((size_t)std::max<int64_t>(1, b->n_items), b->stream);
     hipLaunchKernelGGL(k_ms_item_vertex, dim3((unsigned)ceil_div(h, kT)), dim3(kT), 0, s,
                        b->item_start.get(), h, b->item_vertex.get());
     G500_CHECK_LAUNCH();
@@ -2084,13 +2081,13 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
   G500_CHECK_HIP(hipEventCreate(&b->ev_begin));
   G500_CHECK_HIP(hipEventCreate(&b->ev_end));
   // first, so that its scratch is gone before the engine's own arrays come
-  b->cnt0.alloc((size_t)g->n);
+  b->cnt0.alloc((size_t)g->n, b->stream);
   {
     // only loops name IDs from n on, which no root reaches
     DevBuf<uint32_t> deg;
     DevBuf<unsigned long long> stats;
     deg.alloc_raw((size_t)g->n);
-    stats.alloc(2);
+    stats.alloc(2, b->stream);
     G500_CHECK_HIP(hipMemsetAsync(deg.get(), 0, (size_t)g->n * sizeof(uint32_t), b->stream));
     count_degrees(g->edges.get(), g->nedges, DegreeMode::kSourceEnd, g->n, deg.get(), stats.get(),
                   b->stream);
@@ -2100,23 +2097,23 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
     G500_CHECK_HIP(hipStreamSynchronize(b->stream));
   }
   const int64_t nc = std::max<int64_t>(1, g->n_c);
-  b->seen.alloc((size_t)nc * b->kmax);
-  b->fptr.alloc(kMaxLevels + 1);  // F_0..F_255
-  b->cnt.alloc(kMaxLevels + 2);
-  b->te.alloc(G500_MSBFS_MAX_ROOTS);
-  b->lane_part.alloc((size_t)kLaneParts * 256);
-  b->split_mask.alloc(4);
-  G500_CHECK_HIP(hipMemset(b->split_mask.get(), 0, 4 * sizeof(uint64_t)));
-  b->roots.alloc(G500_MSBFS_MAX_ROOTS + 1);
+  b->seen.alloc((size_t)nc * b->kmax, b->stream);
+  b->fptr.alloc(kMaxLevels + 1, b->stream);  // F_0..F_255
+  b->cnt.alloc(kMaxLevels + 2, b->stream);
+  b->te.alloc(G500_MSBFS_MAX_ROOTS, b->stream);
+  b->lane_part.alloc((size_t)kLaneParts * 256, b->stream);
+  b->split_mask.alloc(4, b->stream);
+  G500_CHECK_HIP(hipMemsetAsync(b->split_mask.get(), 0, 4 * sizeof(uint64_t), b->stream));
+  b->roots.alloc(G500_MSBFS_MAX_ROOTS + 1, b->stream);
   b->level_arrays = level_arrays;
   if (level_arrays) {
-    b->out.alloc((size_t)max_roots * (size_t)g->n);
-    b->planes.alloc((size_t)nc * 4 * std::min(b->kmax, 2));
+    b->out.alloc((size_t)max_roots * (size_t)g->n, b->stream);
+    b->planes.alloc((size_t)nc * 4 * std::min(b->kmax, 2), b->stream);
   }
-  b->fb[0].alloc((size_t)bitmap_words(b));
-  b->fb[1].alloc((size_t)bitmap_words(b));
-  b->fe.alloc(2 * (kMaxLevels + 2));  // of all the frontier, of its heavy vertices
-  b->act.alloc((size_t)(kMaxLevels + 2) * 4);
+  b->fb[0].alloc((size_t)bitmap_words(b), b->stream);
+  b->fb[1].alloc((size_t)bitmap_words(b), b->stream);
+  b->fe.alloc(2 * (kMaxLevels + 2), b->stream);  // of all the frontier, of its heavy vertices
+  b->act.alloc((size_t)(kMaxLevels + 2) * 4, b->stream);
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_roots, (G500_MSBFS_MAX_ROOTS + 1) * sizeof(int64_t),
                                hipHostMallocDefault));
   G500_CHECK_HIP(hipHostMalloc((void**)&b->h_cnt, (kMaxLevels + 2) * sizeof(unsigned long long),
@@ -2125,7 +2122,7 @@ void msbfs_init(g500_msbfs* b, int max_roots, bool level_arrays) {
 
   if (g->m > 0) {
     // tiles of 2048 edges read entries 2t and 2t+2: room for both past the end
-    b->stream_tile_v0.alloc((size_t)ceil_div(g->m, kStreamUnit) + 3);
+    b->stream_tile_v0.alloc((size_t)ceil_div(g->m, kStreamUnit) + 3, b->stream);
     hipLaunchKernelGGL(k_ms_stream_tiles, dim3((unsigned)ceil_div(g->n_c, kT)), dim3(kT), 0,
                        b->stream, g->row_off.get(), g->n_c, b->stream_tile_v0.get());
     G500_CHECK_LAUNCH();
@@ -2339,8 +2336,8 @@ void msbfs_gather(g500_msbfs* b, const int64_t* pairs, int64_t count, uint8_t* l
   if (count <= 0) return;
   check_pairs(b, pairs, count);
   if ((int64_t)b->gather_pairs.n < 2 * count) {
-    b->gather_pairs.alloc((size_t)2 * count);
-    b->gather_levels.alloc((size_t)count);
+    b->gather_pairs.alloc((size_t)2 * count, b->stream);
+    b->gather_levels.alloc((size_t)count, b->stream);
   }
   gather_staged(b, pairs, count, levels, b->gather_pairs.get(), b->gather_levels.get());
 }

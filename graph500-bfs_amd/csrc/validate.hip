@@ -304,8 +304,8 @@ void bfs_validate(g500_bfs* b, int64_t root, const int64_t* host_pred,
   } else if (!b->have_result) {
     fail(G500_ERR_STATE, "validate: no BFS result on the device");
   }
-  if (!b->vcount.get()) b->vcount.alloc(kCounters);
-  if (!b->pred_valid.get()) b->pred_valid.alloc((size_t)nlocal);
+  if (!b->vcount.get()) b->vcount.alloc(kCounters, s);
+  if (!b->pred_valid.get()) b->pred_valid.alloc((size_t)nlocal, s);
   unsigned long long* cnt = b->vcount.get();
   unsigned long long h[kCounters];
   auto fetch = [&]() {
