@@ -71,14 +71,30 @@ size_t keep_limit(int device) {
   return limit[(size_t)device];
 }
 
-// Idle blocks also go beside work that has nothing to do with them, another
-// thread's capture among it, which a plain hipFree would break.
-void free_blocks(const std::vector<Block>& out) {
-  if (out.empty()) return;
+// Calls made in its scope leave the captures of other threads alone.
+struct BesideCaptures {
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~BesideCaptures() {
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+
+void free_blocks(const std::vector<Block>& out) {
+  if (out.empty()) return;
+  BesideCaptures scope;
   for (const Block& b : out) (void)hipFree(b.p);
-  if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
+// Waits for all work queued on the device.  hipDeviceSynchronize does that too,
+// but beside a capture in any thread, an engine's of its batch for one, it fails
+// and ends that capture, whatever its mode; hipFree waits as well and does not.
+// About 2 us where nothing is queued.
+bool device_wait() {
+  BesideCaptures scope;
+  void* p = nullptr;
+  if (hipMalloc(&p, 4096) != hipSuccess) return false;
+  return hipFree(p) == hipSuccess;
 }
 
 }  // namespace
@@ -143,10 +159,8 @@ void device_release(void* p, size_t bytes, int device) {
   int current = 0;
   (void)hipGetDevice(&current);
   const size_t limit = keep_limit(device);
-  // the wait fails only beside a capture that forbids it or after a fault:
-  // the block then goes back at once
-  if (bytes < kKeepMin || bytes > limit || current != device ||
-      hipDeviceSynchronize() != hipSuccess) {
+  // where the wait fails (no memory left, or a fault), the block goes back at once
+  if (bytes < kKeepMin || bytes > limit || current != device || !device_wait()) {
     (void)hipGetLastError();
     (void)hipFree(p);
     device_release_idle();

@@ -14,7 +14,7 @@
 struct FakeDevice {
   size_t capacity = 0, used = 0, most = 0;  // most: the largest `used` so far
   int mallocs = 0, frees = 0, current = 0;
-  bool sync_fails = false;
+  int waits = 0;  // hipFree waits for the device
   std::map<void*, size_t> blocks;
 };
 inline FakeDevice fake_device;
@@ -42,9 +42,6 @@ inline hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
   p->totalGlobalMem = fake_device.capacity;
   return hipSuccess;
 }
-inline hipError_t hipDeviceSynchronize() {
-  return fake_device.sync_fails ? hipErrorStreamCaptureUnsupported : hipSuccess;
-}
 inline hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
 enum hipMemcpyKind { hipMemcpyHostToDevice, hipMemcpyDeviceToHost };
 inline hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
@@ -71,6 +68,7 @@ inline hipError_t hipFree(void* p) {
   if (it == d.blocks.end()) std::abort();
   d.used -= it->second;
   ++d.frees;
+  ++d.waits;
   d.blocks.erase(it);
   std::free(p);
   return hipSuccess;
