@@ -48,10 +48,9 @@ inline hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
   std::memset(p, v, n < 64 ? n : 64);
   return hipSuccess;
 }
-inline hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) {
+inline hipError_t hipMemcpyWithStream(void*, const void*, size_t, hipMemcpyKind, hipStream_t) {
   return hipSuccess;
 }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) {
   FakeDevice& d = fake_device;
   if (d.used + n > d.capacity) return hipErrorOutOfMemory;
