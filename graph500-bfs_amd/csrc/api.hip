@@ -345,7 +345,9 @@ int g500_graph_free(g500_graph* g) {
       g500::fail(G500_ERR_STATE, "graph still has %d engine(s): destroy them first",
                  g->live_engines);
     (void)hipSetDevice(g->device);
-    (void)hipStreamSynchronize(g->stream);
+    const bool idle = hipStreamSynchronize(g->stream) == hipSuccess;
+    g500::IdleReleases released;  // engines waited for their streams when they went
+    if (idle) released.now();
     delete g;
   });
 }
@@ -457,9 +459,12 @@ int g500_bfs_destroy(g500_bfs* b) {
     // a run that failed inside a level can leave kernels queued on either
     // stream (the pred gather runs on gstream): drain both before the
     // buffers and the pinned report they write are released
-    (void)hipStreamSynchronize(b->stream);
-    if (b->gstream) (void)hipStreamSynchronize(b->gstream);
+    const bool idle =
+        hipStreamSynchronize(b->stream) == hipSuccess &&
+        (!b->gstream || hipStreamSynchronize(b->gstream) == hipSuccess);
     --b->g->live_engines;
+    g500::IdleReleases released;
+    if (idle) released.now();
     delete b;
   });
 }
@@ -642,7 +647,7 @@ int g500_msbfs_destroy(g500_msbfs* b) {
     (void)hipSetDevice(b->g->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     --b->g->live_engines;
-    delete b;
+    delete b;  // (a caller's stream may still read the level arrays)
   });
 }
 

@@ -2864,7 +2864,11 @@ void bfs_levels(g500_bfs* b, uint16_t* out) {
   G500_CHECK_HIP(hipMemcpyAsync(out, lv.get(), g->n * sizeof(uint16_t),
                                 hipMemcpyDeviceToHost, b->stream));
   G500_CHECK_HIP(hipStreamSynchronize(b->stream));
-  if (g->n > kSmallVerts * 4) lv.release();
+  if (g->n > kSmallVerts * 4) {
+    IdleReleases released;
+    released.now();
+    lv.release();
+  }
 }
 
 }  // namespace g500

@@ -52,8 +52,21 @@ __device__ inline uint64_t lanemask_lt() {
 // *got and *device go back with device_release.  Null where there is no room.
 // scratch: freed again soon, so its size may be rounded up.
 void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* device);
-// Waits for the device's queued work, as hipFree does.
+// The block may still be in use by work queued so far, and who gets it next waits
+// for the device, unless the releasing thread has said otherwise (IdleReleases).
 void device_release(void* p, size_t bytes, int device);
+// Until it ends, what the thread releases after now() is idle: every stream that
+// used it has been waited for.  Declared before the buffers it is for, whose
+// destructors then run inside it; left by an exception it says nothing.
+struct IdleReleases {
+  void now() { (void)set(true); }
+  void over() { (void)set(false); }
+  ~IdleReleases() { (void)set(before); }
+
+ private:
+  static bool set(bool idle);
+  const bool before = set(false);
+};
 // Gives all kept blocks back to the device.
 void device_trim();
 // Gives back the kept blocks that no one took for ten seconds; a few

@@ -223,6 +223,7 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
   const int lg = g->log_n;
   const int64_t n = g->n;
   const int64_t nk = symmetric ? ne : 2 * ne;
+  IdleReleases released;
   DevBuf<uint64_t> ek, ek_alt;
   ek.alloc_raw((size_t)nk);
   ek_alt.alloc_raw((size_t)nk);
@@ -261,6 +262,7 @@ void sort_rows(g500_graph* g, const uint2* edges, int64_t ne, bool symmetric) {
                      g->m);
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
+  released.now();
 }
 
 }  // namespace
@@ -304,6 +306,7 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, DegreeMode mode,
   g->new2orig.alloc_raw((size_t)n);
   g->orig2new.alloc_raw((size_t)n);
   g->deg_new.alloc_raw((size_t)n);
+  IdleReleases released;
   {
     DevBuf<uint64_t> vk, vk_alt;
     vk.alloc_raw((size_t)n);
@@ -322,8 +325,10 @@ void build_csr(g500_graph* g, const uint2* edges, int64_t ne, DegreeMode mode,
                        g->orig2new.get(), g->deg_new.get());
     G500_CHECK_LAUNCH();
     G500_CHECK_HIP(hipStreamSynchronize(s));
+    released.now();
   }
   deg.release();
+  released.over();
 
   if (!build_rows(g, edges, ne, symmetric)) sort_rows(g, edges, ne, symmetric);
   {

@@ -386,6 +386,8 @@ void corebfs_prune(g500_graph* g) {
     G500_CHECK_LAUNCH();
   }
   G500_CHECK_HIP(hipStreamSynchronize(s));
+  IdleReleases released;
+  released.now();
   alive.release();
   tile_row.release();
   tile_cnt.release();
@@ -395,8 +397,11 @@ void corebfs_prune(g500_graph* g) {
   g->first.release();
   g->multi.release();
   g->row_off.release();
+  released.over();
   build_csr(g, core_edges.get(), (int64_t)m_core, DegreeMode::kSourceRuns, log_n);
+  released.now();  // build_csr waited for its stream
   core_edges.release();
+  released.over();
   g->core_vertices = g->n_c;
 
   // find_max_used_vertex over has_edge = core vertex or forest vertex

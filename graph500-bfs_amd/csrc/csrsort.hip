@@ -375,6 +375,7 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
   // partitioning pays once the ranges hold endpoints enough to be counted in
   // LDS; a sparse list over a large ID space keeps the atomics, and so does
   // one whose endpoints find no room (asked for last)
+  IdleReleases released;
   DevBuf<unsigned long long> total;  // per range, then (off) its first slot and a cursor
   DevBuf<uint64_t> off;
   DevBuf<uint16_t> ep;
@@ -412,6 +413,7 @@ void count_mode(const uint2* edges, int64_t ne, int64_t nv, uint32_t* deg,
                      s, ep.get(), off.get(), (int)ranges, deg);
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
+  released.now();
 }
 
 // --------------------------------------------------------------------- rows
@@ -1032,6 +1034,7 @@ static bool rows_by_buckets(g500_graph* g, const uint2* edges, int64_t ne, bool 
   const bool two = step > 1;
   const int64_t group_keys = step * kBucketMean;
   const int64_t group_cap = group_keys + group_keys / 8 + kPartTile;
+  IdleReleases released;
   DevBuf<uint64_t> roff, spl, part, sorted, off, ubase;
   DevBuf<uint32_t> cnt, ucnt, big, flag, uniq;
   DevBuf<unsigned long long> rows, cursor, gcursor;
@@ -1111,6 +1114,7 @@ static bool rows_by_buckets(g500_graph* g, const uint2* edges, int64_t ne, bool 
                      rows.get(), ubase.get(), n_c, g->m, g->row_off.get());
   G500_CHECK_LAUNCH();
   G500_CHECK_HIP(hipStreamSynchronize(s));  // the scratch is freed on return
+  released.now();
   return true;
 }
 
@@ -1144,6 +1148,7 @@ std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t
   if (tiles > kMaxParts)
     while (((int64_t)1 << (2 * step_log)) < tiles) ++step_log;
   const int64_t step = (int64_t)1 << step_log, groups = ceil_div(tiles, step);
+  IdleReleases released;
   DevBuf<uint64_t> part, keys, off;
   DevBuf<uint32_t> cnt;
   DevBuf<unsigned long long> cursor;
@@ -1225,6 +1230,7 @@ std::shared_ptr<const OrderedEdges> order_edges(const g500_graph* g, hipStream_t
   order->keys.swap(keys);
   order->n_chunks = (int64_t)chunks.size();
   order->part_bits = part_bits;
+  released.now();  // the stream was waited for above
   return order;
 }
 

@@ -11,9 +11,11 @@
 // the next call that allocates, frees, searches or validates.  A process that
 // makes no more calls keeps them.
 //
-// A block is kept only after the device has finished all work queued so far
-// (as hipFree waits for it), so whichever thread or stream takes it next has
-// it alone.
+// A kept block is handed out only after the device has finished all work queued
+// before it was released (hipFree would wait for that at once), so whichever
+// thread or stream takes it next has it alone.  One wait does for all blocks
+// released before it, and none is needed for blocks whose only users have just
+// been waited for (IdleReleases).
 #include <atomic>
 #include <chrono>
 #include <mutex>
@@ -35,6 +37,7 @@ struct Block {
   void* p;
   size_t bytes;
   int device;
+  uint64_t number;  // of its release, 0 where it was idle then
   Clock::time_point since;
 };
 
@@ -43,10 +46,16 @@ struct Block {
 struct Kept {
   std::mutex mu;
   std::vector<Block> blocks;  // oldest first
+  uint64_t releases = 0;
+  std::vector<uint64_t> waited;  // per device: releases that a wait has followed
   // when the oldest was released, the far future where there is none: read
   // without the lock by calls that only look for idle blocks
   std::atomic<Clock::rep> oldest{Clock::time_point::max().time_since_epoch().count()};
 
+  uint64_t& waited_for(int device) {
+    if ((int)waited.size() <= device) waited.resize((size_t)device + 1, 0);
+    return waited[(size_t)device];
+  }
   void changed() {
     const Clock::time_point t = blocks.empty() ? Clock::time_point::max() : blocks.front().since;
     oldest.store(t.time_since_epoch().count(), std::memory_order_relaxed);
@@ -80,6 +89,8 @@ struct BesideCaptures {
   }
 };
 
+thread_local bool t_idle = false;
+
 void free_blocks(const std::vector<Block>& out) {
   if (out.empty()) return;
   BesideCaptures scope;
@@ -89,12 +100,13 @@ void free_blocks(const std::vector<Block>& out) {
 // Waits for all work queued on the device.  hipDeviceSynchronize does that too,
 // but beside a capture in any thread, an engine's of its batch for one, it fails
 // and ends that capture, whatever its mode; hipFree waits as well and does not.
-// About 2 us where nothing is queued.
+// 10 us after the last work, then 1.  Of the current device.
 bool device_wait() {
   BesideCaptures scope;
   void* p = nullptr;
-  if (hipMalloc(&p, 4096) != hipSuccess) return false;
-  return hipFree(p) == hipSuccess;
+  if (hipMalloc(&p, 4096) == hipSuccess && hipFree(p) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
 }
 
 }  // namespace
@@ -131,8 +143,10 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
     want = (want + step - 1) / step * step;
   }
   const size_t most = want + (scratch ? want / 8 : want / 64);
+  Kept& k = kept();
+  bool idle = true;  // nothing queued before its release is left
+  uint64_t releases = 0;
   {
-    Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
     size_t best = k.blocks.size();
     for (size_t i = 0; i < k.blocks.size(); ++i) {
@@ -145,9 +159,22 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
       p = k.blocks[best].p;
       *got = k.blocks[best].bytes;
       *used = true;
+      idle = k.blocks[best].number <= k.waited_for(*device);
+      releases = k.releases;
       k.blocks.erase(k.blocks.begin() + (ptrdiff_t)best);
     }
     k.changed();
+  }
+  if (!idle) {
+    if (device_wait()) {
+      std::lock_guard<std::mutex> lock(k.mu);
+      uint64_t& waited = k.waited_for(*device);
+      waited = std::max(waited, releases);
+    } else {  // no memory left, or a fault: hipFree waits
+      (void)hipFree(p);
+      p = nullptr;
+      *used = false;
+    }
   }
   device_release_idle();
   if (p) return p;
@@ -155,13 +182,13 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
   return p;
 }
 
+bool IdleReleases::set(bool idle) { return std::exchange(t_idle, idle); }
+
 void device_release(void* p, size_t bytes, int device) {
   int current = 0;
   (void)hipGetDevice(&current);
   const size_t limit = keep_limit(device);
-  // where the wait fails (no memory left, or a fault), the block goes back at once
-  if (bytes < kKeepMin || bytes > limit || current != device || !device_wait()) {
-    (void)hipGetLastError();
+  if (bytes < kKeepMin || bytes > limit || current != device) {
     (void)hipFree(p);
     device_release_idle();
     return;
@@ -170,7 +197,7 @@ void device_release(void* p, size_t bytes, int device) {
   {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
-    k.blocks.push_back({p, bytes, device, Clock::now()});
+    k.blocks.push_back({p, bytes, device, t_idle ? 0 : ++k.releases, Clock::now()});
     size_t total = 0;
     for (const Block& b : k.blocks) total += b.device == device ? b.bytes : 0;
     for (size_t i = 0; i < k.blocks.size() && total > limit;) {

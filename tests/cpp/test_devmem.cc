@@ -161,16 +161,65 @@ int main() {
     CHECK(fake_device.used == 300 * kMiB);
   }
   fresh_device();
-  {  // a block is kept only after the device was waited for, else it goes back
-    const Got a = take(100 * kMiB);
-    const int waits = fake_device.waits;
+  {  // a kept block is handed out only after the device was waited for, once for all
+     // that were released before, else it goes back
+    const Got a = take(100 * kMiB), b = take(200 * kMiB), c = take(300 * kMiB);
     give(a);
-    CHECK(fake_device.used == 100 * kMiB && fake_device.waits == waits + 1);
-    const Got b = take(100 * kMiB), full = take(kAll - fake_device.used);
-    CHECK(b.p == a.p && fake_device.used == kAll);
-    give(b);  // no room for the wait's own bytes
-    CHECK(fake_device.used == full.bytes);
-    give(full);
+    give(b);
+    const int waits = fake_device.waits;
+    CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 1);
+    CHECK(take(200 * kMiB).p == b.p && fake_device.waits == waits + 1);
+    give(c);
+    give(a);
+    CHECK(take(300 * kMiB).p == c.p && fake_device.waits == waits + 2);
+    CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 2);
+    give(a);
+    CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 3);
+    {  // idle ones need none, until the releasing thread takes it back
+      g500::IdleReleases released;
+      give(a);
+      CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 4);
+      released.now();
+      give(a);
+      CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 4);
+      {
+        g500::IdleReleases inner;
+        give(a);
+        CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 5);
+        inner.now();
+      }
+      give(a);
+      CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 5);
+      released.over();
+      give(a);
+      CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 6);
+      released.now();
+    }
+    give(a);
+    CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 7);
+    give(a);
+    const Got full = take(kAll - fake_device.used);
+    CHECK(fake_device.used == kAll);
+    const Got d = take(100 * kMiB);  // no room for the wait's own bytes: hipFree waits
+    CHECK(d.p && fake_device.waits > waits + 7 && fake_device.used == kAll);
+    for (const Got& g : {b, c, d, full}) give(g);
+  }
+  fresh_device();
+  {  // every device has its own
+    const Got a = take(100 * kMiB);
+    fake_device.current = 1;
+    const Got b = take(100 * kMiB);
+    give(b);
+    fake_device.current = 0;
+    give(a);
+    const int waits = fake_device.waits;
+    CHECK(take(100 * kMiB).p == a.p && fake_device.waits == waits + 1);
+    fake_device.current = 1;
+    CHECK(take(100 * kMiB).p == b.p && fake_device.waits == waits + 2);
+    fake_device.current = 0;
+    give(a);  // b is device 1's: released from device 0 it goes back at once
+    give(b);
+    CHECK(fake_device.used == 100 * kMiB);
   }
   std::puts("devmem ok");
 }
