@@ -186,33 +186,40 @@ void* device_alloc(size_t bytes, bool scratch, bool* used, size_t* got, int* dev
 
 bool IdleReleases::set(bool idle) { return std::exchange(t_idle, idle); }
 
+// Buffers are released by destructors: a lack of host memory must not leave here.
 void device_release(void* p, size_t bytes, int device) {
   int current = 0;
   (void)hipGetDevice(&current);
-  const size_t limit = keep_limit(device);
-  if (bytes < kKeepMin || bytes > limit || current != device) {
-    (void)hipFree(p);
-    device_release_idle();
-    return;
-  }
   std::vector<Block> old;
-  {
-    Kept& k = kept();
-    std::lock_guard<std::mutex> lock(k.mu);
-    k.blocks.push_back({p, bytes, device, t_idle ? 0 : ++k.releases, Clock::now()});
-    size_t total = 0;
-    for (const Block& b : k.blocks) total += b.device == device ? b.bytes : 0;
-    for (size_t i = 0; i < k.blocks.size() && total > limit;) {
-      if (k.blocks[i].device != device) {
-        ++i;
-        continue;
+  bool keep = bytes >= kKeepMin && current == device;
+  if (keep) {
+    try {
+      const size_t limit = keep_limit(device);
+      Kept& k = kept();
+      std::lock_guard<std::mutex> lock(k.mu);
+      keep = false;
+      if (bytes <= limit) {
+        old.reserve(k.blocks.size() + 1);
+        k.blocks.push_back({p, bytes, device, t_idle ? 0 : ++k.releases, Clock::now()});
+        keep = true;
+        size_t total = 0;
+        for (const Block& b : k.blocks) total += b.device == device ? b.bytes : 0;
+        for (size_t i = 0; i < k.blocks.size() && total > limit;) {
+          if (k.blocks[i].device != device) {
+            ++i;
+            continue;
+          }
+          total -= k.blocks[i].bytes;
+          old.push_back(k.blocks[i]);
+          k.blocks.erase(k.blocks.begin() + (ptrdiff_t)i);
+        }
+        k.changed();
       }
-      total -= k.blocks[i].bytes;
-      old.push_back(k.blocks[i]);
-      k.blocks.erase(k.blocks.begin() + (ptrdiff_t)i);
+    } catch (const std::bad_alloc&) {
+      keep = false;
     }
-    k.changed();
   }
+  if (!keep) (void)hipFree(p);
   free_blocks(old);
   device_release_idle();
 }
@@ -235,6 +242,11 @@ void device_release_idle(Clock::time_point now) {
   std::vector<Block> old;
   {
     std::lock_guard<std::mutex> lock(k.mu);
+    try {
+      old.reserve(k.blocks.size());
+    } catch (const std::bad_alloc&) {
+      return;  // at another call
+    }
     while (!k.blocks.empty() && k.blocks.front().since < now - kIdle) {
       old.push_back(k.blocks.front());
       k.blocks.erase(k.blocks.begin());

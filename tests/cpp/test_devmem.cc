@@ -6,6 +6,16 @@
 #include "../../graph500-bfs_amd/csrc/devmem.hip"
 #include "../../graph500-bfs_amd/csrc/edgeorder.hip"
 
+// host memory that runs out on demand
+static bool no_host_memory = false;
+void* operator new(size_t n) {
+  void* p = no_host_memory ? nullptr : std::malloc(n);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 namespace {
 
 constexpr size_t kMiB = size_t(1) << 20, kGiB = size_t(1) << 30, kAll = 64 * kGiB;
@@ -220,6 +230,18 @@ int main() {
     give(a);  // b is device 1's: released from device 0 it goes back at once
     give(b);
     CHECK(fake_device.used == 100 * kMiB);
+  }
+  fresh_device();
+  {  // without host memory a released block goes back, and nothing is thrown
+    std::vector<Got> all;
+    for (int i = 0; i < 100; ++i) all.push_back(take(2 * kMiB));
+    no_host_memory = true;
+    for (const Got& g : all) give(g);
+    g500::device_release_idle(std::chrono::steady_clock::now() + std::chrono::seconds(11));
+    no_host_memory = false;
+    CHECK(fake_device.used < 200 * kMiB);
+    g500::device_trim();
+    CHECK(fake_device.used == 0);
   }
   std::puts("devmem ok");
 }
