@@ -22,7 +22,10 @@
 // edges, the first is direct: ordering takes 6 ms at SCALE 24, so a program that
 // validates one tree of a graph would lose by it.  The first, second and third
 // call take 8.0, 7.6 and 1.4 ms there (8.4 each when all are direct), 1.5, 2.0 and
-// 0.45 at SCALE 22 (1.6 each).
+// 0.45 at SCALE 22 (1.6 each).  From 2^28 edges on ordering at once would cost the
+// first call no more than the direct pass (33 against 38 ms at SCALE 26) while its 16
+// bytes an edge are at hand; where the driver has to clear them first it took 124
+// and 184 ms, which one tree does not earn back.
 // Graphs of fewer edges, or trees deeper than a byte's four bits hold, take
 // the direct form.
 #include "engine.hpp"
